@@ -435,11 +435,6 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
     for (int i = 0; i < 16; ++i) o_acc[cb][i] = 0.0f;
   float m_run = kRowFloor;
   float d_part = 0.0f;  // this lane's half of the row denominator
-  // The float whose bits the P·V accumulators start from, kept in a vector
-  // register: with a literal or scalar operand the subtraction that removes it
-  // issues at half the rate.
-  float seed_value;
-  asm volatile("v_mov_b32 %0, %1" : "=v"(seed_value) : "s"(kAccumulatorSeedBits));
 
   // capture bookkeeping
   [[maybe_unused]] uint32_t* stats = nullptr;
@@ -452,11 +447,8 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
     stat_row = static_cast<uint64_t>(bhq) * p.q_len + query;
   }
 
-  const int64_t mask_row =
-      (MASK_DT >= 0 && MASK_DT != kKeyBias)
-          ? static_cast<int64_t>(batch) * p.mask_stride_b + static_cast<int64_t>(head) * p.mask_stride_h +
-                static_cast<int64_t>(query) * p.mask_stride_q
-          : 0;
+  // First mask element of this lane's query; set behind the hand-scheduled loop.
+  [[maybe_unused]] int64_t mask_row = 0;
 
   // Lane words of one tile: 16 scalar register pairs per 32-key block, loaded through the
   // scalar cache from a wave-uniform address.  The words of a tile's first key block are
@@ -936,6 +928,10 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
     for (int j = 0; j < 2; ++j)
       frag[j] = *reinterpret_cast<const v4i*>(vl + swizzled<CTA_K>((cb + j) * 32 + l32, rb * 2 + half));
   };
+  // The float whose bits the P·V accumulators start from, kept in a vector
+  // register: with a literal or scalar operand the subtraction that removes it
+  // issues at half the rate.  (Set behind the hand-scheduled loop, which has its own.)
+  float seed_value = 0.0f;
   auto unseed = [&](int bits) { return __int_as_float(bits) - seed_value; };
   auto value_tile = [&](int stage, const v4i (&pk)[RB], v16i (&seed0)[2], v4i (&first0)[2], float t_scale) {
     // Three accumulator sets rotate when there are more than two pairs: one being
@@ -991,9 +987,31 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
   // the generator chose; the last listed tile (the one that may be partial) and the epilogue
   // stay below.
   constexpr bool ASM_LOOP = FAST && D == 128 && CTA_K == 128;
+  // Other launches have loops of the same kind, written by gen_tile_loops.py.  All are bound by
+  // vector issue; the loop the compiler schedules spends 706 (causal, 128-key tile), 330 (raw, 64)
+  // and 669 (float mask, 64) vector instructions on a wavefront's tile, these 620, 300 and 510.
+  // Whole calls, compiled loop -> this one, same machine: causal 32/8 heads x 8192 462 -> 410 us;
+  // 40 heads x 32760 queries x 512 keys 487 -> 469 us; float mask 2 x 24 heads x 4096 x 4608,
+  // 661 -> 556 us.
+  constexpr bool SCALED_LOOP = !FAST && D == 128 && CTA_K == 128 && MASK_DT == -1 && !INDEXED && !CAPTURE;
+  constexpr bool SHORT_LOOP = FAST && D == 128 && CTA_K == 64 && !INDEXED && !CAPTURE;
+  constexpr bool F32_MASK_LOOP = D == 128 && SHARED_MASK && !INDEXED && !CAPTURE;
   int first_tile = 0;
-  if constexpr (ASM_LOOP) {
+  // Listed tiles a hand-scheduled loop walks.  It copies whole tiles without looking at the key
+  // range, the one behind its last included, so a last tile of fewer keys leaves two to the loop
+  // below; under the causal rule only tiles below the diagonal are its own.
+  [[maybe_unused]] int walk = 0;
+  if constexpr (ASM_LOOP || SCALED_LOOP || SHORT_LOOP || F32_MASK_LOOP) {
     if (n_it > 1 && !p.compiled_loop) {
+      walk = n_it - 1;
+      if (p.k_len % CTA_K != 0 && (tile_at(n_it - 1) + 1) * CTA_K > p.k_len) --walk;
+      if (!FAST && p.causal) walk = min(walk, bx * (kQueryBlock / CTA_K));
+      // the loop's mask copies take every row of the query block
+      if (F32_MASK_LOOP && (bx + 1) * kQueryBlock > p.q_len) walk = 0;
+    }
+  }
+  if constexpr (ASM_LOOP) {
+    if (walk > 0) {
       typedef __attribute__((address_space(3))) unsigned char* LdsBytes;
       const uint32_t lds_address = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((LdsBytes)lds));
       issue_tile(tile_at(0), 0);
@@ -1013,7 +1031,7 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
       const uint64_t v_source = reinterpret_cast<uint64_t>(INDEXED ? v_base : v_base + CTA_K);
       const uint64_t sum_source = reinterpret_cast<uint64_t>(INDEXED ? sum_base : sum_base + D);
       const uint64_t ks_source = reinterpret_cast<uint64_t>(ks_base);
-      const int count = n_it - 1;
+      const int count = walk;
       if constexpr (INDEXED) {
         const uint64_t list = reinterpret_cast<uint64_t>(indices);
         asm volatile(
@@ -1074,8 +1092,68 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
         o_acc[2][i] = __int_as_float(out2[i]);
         o_acc[3][i] = __int_as_float(out3[i]);
       }
-      first_tile = n_it - 1;
+      first_tile = walk;
     }
+  } else if constexpr (SCALED_LOOP || SHORT_LOOP || F32_MASK_LOOP) {
+    if (walk > 0) {
+      typedef __attribute__((address_space(3))) unsigned char* LdsBytes;
+      const uint32_t lds_address = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((LdsBytes)lds));
+      issue_tile(tile_at(0), 0);
+      if constexpr (F32_MASK_LOOP) issue_mask_tile(tile_at(0), 0);
+      v16i out0 = {}, out1 = {}, out2 = {}, out3 = {};
+      // this lane's fragment addresses (row l32 of a 32-row block) and the lane shares of the copy
+      // source offsets, as above
+      constexpr int V_ROWS = 1024 / CTA_K;
+      uint32_t k_address[KK], v_address[RB], k_share[2], v_share[2];
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) k_address[kk] = lds_address + swizzled<D>(l32, kk * 2 + half);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) v_address[rb] = lds_address + swizzled<CTA_K>(l32, rb * 2 + half);
+      const uint32_t seed_address = lds_address + half * 16 + 2048;  // (the generator's SEED_BIAS)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        k_share[i] = k_source_offset(i, lane) - static_cast<uint32_t>(wave * NC + i) * 1024u;
+        v_share[i] = v_source_offset(i, lane) -
+                     static_cast<uint32_t>((wave * NC + i) * V_ROWS) * static_cast<uint32_t>(p.padded);
+      }
+      const uint64_t k_source = reinterpret_cast<uint64_t>(k_base + CTA_K * D);
+      const uint64_t v_source = reinterpret_cast<uint64_t>(v_base + CTA_K);
+      const uint64_t sum_source = reinterpret_cast<uint64_t>(sum_base + D);
+      const uint64_t ks_source = reinterpret_cast<uint64_t>(ks_base);
+      if constexpr (SCALED_LOOP) {
+#include "tile_loop_scaled_d128k128.inc"
+      } else if constexpr (SHORT_LOOP) {
+#include "tile_loop_raw_d128k64.inc"
+      } else if constexpr (F32_MASK_LOOP) {
+        // this wavefront's mask rows of tile 1; a copy takes four of them, 16 lanes each
+        const uint32_t row_bytes = static_cast<uint32_t>(p.mask_stride_q) * 4u, mask_step = row_bytes * 4u;
+        const uint64_t mask_source = reinterpret_cast<uint64_t>(mask_block + CTA_K * 4) +
+                                     static_cast<uint64_t>(wave * 32) * row_bytes;
+        const uint32_t mask_chunk = ((lane & 15) ^ (lane >> 4)) << 4, mask_row_share = (lane >> 4) * row_bytes;
+        const int row = wave * 32 + l32;
+        const uint32_t mask_address =
+            lds_address + Shape::kSharedMaskOffset + row * (CTA_K * 4) + ((half ^ (row & 15)) << 4);
+#include "tile_loop_f32mask_d128k64.inc"
+      }
+      lane = fresh_lane();
+      l32 = lane & 31;
+      half = lane >> 5;
+      query = bx * kQueryBlock + wave * 32 + l32;
+      query_ok = query < p.q_len;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        o_acc[0][i] = __int_as_float(out0[i]);
+        o_acc[1][i] = __int_as_float(out1[i]);
+        o_acc[2][i] = __int_as_float(out2[i]);
+        o_acc[3][i] = __int_as_float(out3[i]);
+      }
+      first_tile = walk;
+    }
+  }
+  asm volatile("v_mov_b32 %0, %1" : "=v"(seed_value) : "s"(kAccumulatorSeedBits));
+  if constexpr (MASK_DT >= 0 && MASK_DT != kKeyBias) {
+    mask_row = static_cast<int64_t>(batch) * p.mask_stride_b + static_cast<int64_t>(head) * p.mask_stride_h +
+               static_cast<int64_t>(query) * p.mask_stride_q;
   }
   if (n_it > 0) {
     v16i s[RB];
@@ -1086,14 +1164,14 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
     int tile = tile_at(first_tile);
     if (first_tile == 0) issue_tile(tile, 0);
     // The last listed tile reads its mask elements directly (it may be partial).
-    if (n_it > 1) issue_mask_tile(tile, 0);
+    if (first_tile < n_it - 1) issue_mask_tile(tile, first_tile & 1);
     load_lane_words(tile, 0);
     float ks0 = ks_base[tile * 4 + 2 * half];
     float ks1 = ks_base[tile * 4 + 2 * half + 1];
     // Listed tiles: the entry after the next one is requested a whole tile before it is
     // needed, ahead of the copies (read where it is needed, its round trip would be
     // waited for in every tile).
-    [[maybe_unused]] int listed_next = INDEXED && n_it > 1 ? tile_at(1) : 0;
+    [[maybe_unused]] int listed_next = INDEXED && first_tile < n_it - 1 ? tile_at(first_tile + 1) : 0;
     for (int it = first_tile; it < n_it - 1; ++it) {
       const int stage = it & 1;
       const int next_tile = INDEXED ? listed_next : it + 1;

@@ -1,0 +1,89 @@
+"""The tile loops of gen_tile_loops.py against the loop the compiler schedules
+(RISA_COMPILED_LOOP=1), bit for bit, on launches of more workgroups than compute units: causal
+launches, scales of both signs, short key ranges and masks, at the edges of tiles and query blocks."""
+
+import math
+
+import pytest
+import torch
+
+from tests.helpers import oracle_prequantize, relative_l2, seeded, to_numpy
+from tests.test_gpu_tile_loop import compiled_loop
+
+pytestmark = pytest.mark.gpu
+
+
+def both(risa, *tensors, **options):
+    mine = risa.int8_attention(*tensors, return_lse=True, **options)
+    with compiled_loop():
+        theirs = risa.int8_attention(*tensors, return_lse=True, **options)
+    for a, b in zip(mine, theirs):
+        # (rows that see nothing but infinite terms are no numbers on both sides)
+        assert torch.equal(torch.nan_to_num(a.float(), nan=123.0), torch.nan_to_num(b.float(), nan=123.0))
+    return mine
+
+
+def inputs(batch, heads, kv_heads, q_len, k_len, dim, dtype=torch.bfloat16, scale=1.5):
+    return (seeded((batch, heads, q_len, dim), dtype, q_len, scale=scale),
+            seeded((batch, kv_heads, k_len, dim), dtype, k_len + 1, scale=scale),
+            seeded((batch, kv_heads, k_len, dim), dtype, k_len + 2, offset=0.25))
+
+
+@pytest.mark.parametrize("q_len,k_len", [(1152, 1152), (1153, 1153), (2000, 2000), (2304, 1300), (1200, 2304), (600, 600), (513, 513)])
+@pytest.mark.parametrize("dim", [128, 64])
+def test_causal(risa, dim, q_len, k_len):
+    q, k, v = inputs(1, 60, 4, q_len, k_len, dim)
+    out, lse = both(risa, q, k, v, is_causal=True)
+    from oracle import pipeline
+
+    prepared = oracle_prequantize(q[:, :1], k[:, :1], v[:, :1], return_lse=True, is_causal=True)
+    expected, _, _ = pipeline.attend(prepared, return_lse=True)
+    assert relative_l2(to_numpy(out[:, :1]), expected) < 1e-3
+
+
+@pytest.mark.parametrize("k_len", [65, 128, 129, 512, 511, 1024, 1025, 1216, 2048])
+@pytest.mark.parametrize("scale", [None, -0.1, 0.0])
+@pytest.mark.parametrize("dim", [128, 64])
+def test_key_range_and_scale(risa, dim, scale, k_len):
+    q, k, v = inputs(2, 20, 4, 1030, k_len, dim, torch.float16)
+    both(risa, q, k, v, scale=scale)
+
+
+@pytest.mark.parametrize("q_len,k_len", [(1024, 1024), (1030, 512), (1152, 1100), (1153, 64), (896, 200), (1024, 128)])
+@pytest.mark.parametrize("kind", ["f32", "bf16", "bool", "bool_head"])
+@pytest.mark.parametrize("dim", [128, 64])
+def test_query_masks(risa, dim, kind, q_len, k_len):
+    """Float masks with hidden keys, numbers at the ends of the range, infinities and NaN, rows that
+    see nothing; boolean masks shared by the heads and per head; with and without the causal rule."""
+    q, k, v = inputs(2, 20, 4, q_len, k_len, dim)
+    pick = torch.Generator(device="cuda").manual_seed(q_len + k_len)
+    if kind.startswith("bool"):
+        mask = torch.rand(2, 20 if kind == "bool_head" else 1, q_len, k_len, generator=pick, device="cuda") < 0.7
+        mask[:, :, 5:9] = False
+        mask[:, :, :, : k_len // 2] |= torch.arange(q_len, device="cuda")[:, None] % 3 == 0
+    else:
+        mask = torch.randn(2, 1, q_len, k_len, generator=pick, device="cuda")
+        chance = torch.rand(mask.shape, generator=pick, device="cuda")
+        for low, term in ((0.90, -math.inf), (0.98, torch.finfo(torch.float32).min), (0.99, math.inf), (0.995, math.nan)):
+            mask[(chance > low) & (torch.arange(q_len, device="cuda")[:, None] % 2 == 0)] = term
+        mask[:, :, 5:9] = -math.inf
+        mask = mask.to(torch.float32 if kind == "f32" else torch.bfloat16)
+    both(risa, q, k, v, attn_mask=mask)
+    if q_len >= k_len:
+        both(risa, q, k, v, attn_mask=mask, is_causal=True)
+
+
+@pytest.mark.parametrize("k_len", [100, 1024, 1025, 1290, 2304])
+@pytest.mark.parametrize("kind", ["padding", "bias", "sparse_bias"])
+@pytest.mark.parametrize("dim", [128, 64])
+def test_key_masks(risa, dim, kind, k_len):
+    q, k, v = inputs(2, 20, 4, 1100, k_len, dim)
+    if kind == "padding":
+        mask = (torch.arange(k_len, device="cuda") < torch.tensor([[k_len], [k_len * 2 // 3]], device="cuda"))[:, None, None]
+    else:
+        mask = seeded((2, 1, 1, k_len), torch.float32, k_len)
+        if kind == "sparse_bias":  # tiles of zeros, of both signs, among others, and hidden keys
+            mask = torch.where(torch.arange(k_len, device="cuda") // 64 % 3 == 1, mask, mask * -0.0)
+            mask[..., ::97] = -math.inf
+    both(risa, q, k, v, attn_mask=mask)
+    both(risa, q, k, v, attn_mask=mask.expand(2, 20, 1, k_len).contiguous(), is_causal=k_len <= 1100)
