@@ -182,16 +182,34 @@ template <int D, int CTA_K, int MASK_DT, int MASK_MODE>
 using AttentionTileShape = TileShape<D, CTA_K, staged_mask_bytes(MASK_DT, MASK_MODE, CTA_K, false),
                                      staged_mask_bytes(MASK_DT, MASK_MODE, CTA_K, true)>;
 
+// Launches with a tile loop of gen_tile_loops.py.  The whole-list walk of a boolean mask takes the
+// listed loop too: its lists name every tile they walk.
+constexpr bool has_tile_loop(int d, int cta_k, bool fast, bool indexed, bool capture, int mask_dt, int mask_mode) {
+  if (capture || d > 128) return false;
+  if (mask_dt == kKeyBias) return d == 64 || cta_k == 128;
+  if (mask_dt == kBool) return mask_mode == kMaskLanes && indexed;
+  if (mask_dt == kF32) return mask_mode == kMaskStaged && d == 128 && cta_k == 64 && !indexed;
+  if (mask_dt != -1 || indexed) return false;
+  return d == 64 || (fast ? cta_k == 64 : cta_k == 128);
+}
+
+// Workgroups per compute unit the registers have to leave room for.  Head dim 64: the tile loops
+// take up to 168 registers, three wavefronts per SIMD; lane words through the compiled loop keep
+// four at 128.
+constexpr int attention_workgroups(int d, int cta_k, bool fast, bool indexed, bool capture, int mask_dt, int mask_mode) {
+  if (d == 256) return 1;
+  if (d == 64 && has_tile_loop(d, cta_k, fast, indexed, capture, mask_dt, mask_mode)) return 3;
+  return d == 64 && mask_mode == kMaskLanes ? 4 : 2;
+}
+
 // MASK_DT: element type of the mask tensor (risa::kBool, kF32, kF16, kBF16), kKeyBias
 // for a key-only mask prepared as an FP32 row, or -1 for none; FAST (raw-score path)
 // implies -1.  MASK_MODE: kMaskScalar / kMaskVector / kMaskStaged; a template parameter
 // and not a run-time branch so that the tile loop holds one unrolled mask path and
 // stays inside the instruction cache.
 template <int D, int CTA_K, bool FAST, bool INDEXED, bool CAPTURE, int MASK_DT, int MASK_MODE>
-__global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskLanes ? 4 : 2)) void attention_kernel(
+__global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, CAPTURE, MASK_DT, MASK_MODE)) void attention_kernel(
     const KernelParams p) {
-  // (lane words, head dim 64: 128 registers keep four workgroups per compute unit; the variant
-  // that walks tile lists would otherwise take 130 and lose one)
   static_assert(!FAST || MASK_DT < 0, "the raw-score path takes no mask");
   static_assert(MASK_MODE == kMaskScalar || (MASK_DT >= 0 && MASK_DT != kKeyBias), "vector loads need a mask tensor");
   static_assert(MASK_MODE != kMaskStaged || CTA_K == 64, "staged masks: 64-key tiles");
@@ -993,19 +1011,18 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
   // Whole calls, compiled loop -> this one, same machine: causal 32/8 heads x 8192 462 -> 410 us;
   // 40 heads x 32760 queries x 512 keys 487 -> 469 us; float mask 2 x 24 heads x 4096 x 4608,
   // 661 -> 556 us.
-  constexpr bool SCALED_LOOP = !FAST && D == 128 && CTA_K == 128 && MASK_DT == -1 && !INDEXED && !CAPTURE;
-  constexpr bool SHORT_LOOP = FAST && D == 128 && CTA_K == 64 && !INDEXED && !CAPTURE;
   constexpr bool F32_MASK_LOOP = D == 128 && SHARED_MASK && !INDEXED && !CAPTURE;
+  constexpr bool TILE_LOOP = has_tile_loop(D, CTA_K, FAST, INDEXED, CAPTURE, MASK_DT, MASK_MODE);
   int first_tile = 0;
   // Listed tiles a hand-scheduled loop walks.  It copies whole tiles without looking at the key
   // range, the one behind its last included, so a last tile of fewer keys leaves two to the loop
   // below; under the causal rule only tiles below the diagonal are its own.
   [[maybe_unused]] int walk = 0;
-  if constexpr (ASM_LOOP || SCALED_LOOP || SHORT_LOOP || F32_MASK_LOOP) {
+  if constexpr (ASM_LOOP || TILE_LOOP) {
     if (n_it > 1 && !p.compiled_loop) {
       walk = n_it - 1;
       if (p.k_len % CTA_K != 0 && (tile_at(n_it - 1) + 1) * CTA_K > p.k_len) --walk;
-      if (!FAST && p.causal) walk = min(walk, bx * (kQueryBlock / CTA_K));
+      if (!FAST && p.causal) walk = INDEXED ? 0 : min(walk, bx * (kQueryBlock / CTA_K));
       // the loop's mask copies take every row of the query block
       if (F32_MASK_LOOP && (bx + 1) * kQueryBlock > p.q_len) walk = 0;
     }
@@ -1094,13 +1111,13 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
       }
       first_tile = walk;
     }
-  } else if constexpr (SCALED_LOOP || SHORT_LOOP || F32_MASK_LOOP) {
+  } else if constexpr (TILE_LOOP) {
     if (walk > 0) {
       typedef __attribute__((address_space(3))) unsigned char* LdsBytes;
       const uint32_t lds_address = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((LdsBytes)lds));
       issue_tile(tile_at(0), 0);
       if constexpr (F32_MASK_LOOP) issue_mask_tile(tile_at(0), 0);
-      v16i out0 = {}, out1 = {}, out2 = {}, out3 = {};
+      [[maybe_unused]] v16i out0 = {}, out1 = {}, out2 = {}, out3 = {};
       // this lane's fragment addresses (row l32 of a 32-row block) and the lane shares of the copy
       // source offsets, as above
       constexpr int V_ROWS = 1024 / CTA_K;
@@ -1116,14 +1133,34 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
         v_share[i] = v_source_offset(i, lane) -
                      static_cast<uint32_t>((wave * NC + i) * V_ROWS) * static_cast<uint32_t>(p.padded);
       }
-      const uint64_t k_source = reinterpret_cast<uint64_t>(k_base + CTA_K * D);
-      const uint64_t v_source = reinterpret_cast<uint64_t>(v_base + CTA_K);
-      const uint64_t sum_source = reinterpret_cast<uint64_t>(sum_base + D);
+      // dense: sources of tile 1 (the loop advances them); listed: bases of the head and the list
+      constexpr int AHEAD = INDEXED ? 0 : 1;
+      const uint64_t k_source = reinterpret_cast<uint64_t>(k_base + AHEAD * CTA_K * D);
+      const uint64_t v_source = reinterpret_cast<uint64_t>(v_base + AHEAD * CTA_K);
+      const uint64_t sum_source = reinterpret_cast<uint64_t>(sum_base + AHEAD * D);
       const uint64_t ks_source = reinterpret_cast<uint64_t>(ks_base);
-      if constexpr (SCALED_LOOP) {
-#include "tile_loop_scaled_d128k128.inc"
-      } else if constexpr (SHORT_LOOP) {
-#include "tile_loop_raw_d128k64.inc"
+      [[maybe_unused]] const uint64_t list = reinterpret_cast<uint64_t>(indices);
+      if constexpr (MASK_DT == kKeyBias) {
+        const uint64_t mask_source = reinterpret_cast<uint64_t>(bias_base + AHEAD * CTA_K);
+        if constexpr (D == 64 && INDEXED) {
+#include "tile_loop_bias_listed_d64k64.inc"
+        } else if constexpr (D == 64) {
+#include "tile_loop_bias_d64k64.inc"
+        } else if constexpr (INDEXED) {
+#include "tile_loop_bias_listed_d128k128.inc"
+        } else {
+#include "tile_loop_bias_d128k128.inc"
+        }
+      } else if constexpr (LANES) {
+        // this wavefront's lane words of tile 0
+        const uint64_t mask_source = reinterpret_cast<uint64_t>(
+            p.mask_lanes + batch * p.mask_lanes_stride_b + head * p.mask_lanes_stride_h +
+            lane_word_offset(bx * 4 + wave, p.n_kb, 0));
+        if constexpr (D == 64) {
+#include "tile_loop_lanes_listed_d64k64.inc"
+        } else {
+#include "tile_loop_lanes_listed_d128k64.inc"
+        }
       } else if constexpr (F32_MASK_LOOP) {
         // this wavefront's mask rows of tile 1; a copy takes four of them, 16 lanes each
         const uint32_t row_bytes = static_cast<uint32_t>(p.mask_stride_q) * 4u, mask_step = row_bytes * 4u;
@@ -1134,6 +1171,14 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
         const uint32_t mask_address =
             lds_address + Shape::kSharedMaskOffset + row * (CTA_K * 4) + ((half ^ (row & 15)) << 4);
 #include "tile_loop_f32mask_d128k64.inc"
+      } else if constexpr (D == 64 && FAST) {
+#include "tile_loop_raw_d64k64.inc"
+      } else if constexpr (D == 64) {
+#include "tile_loop_scaled_d64k64.inc"
+      } else if constexpr (FAST) {
+#include "tile_loop_raw_d128k64.inc"
+      } else {
+#include "tile_loop_scaled_d128k128.inc"
       }
       lane = fresh_lane();
       l32 = lane & 31;
@@ -1144,8 +1189,10 @@ __global__ __launch_bounds__(256, (D == 256 ? 1 : D == 64 && MASK_MODE == kMaskL
       for (int i = 0; i < 16; ++i) {
         o_acc[0][i] = __int_as_float(out0[i]);
         o_acc[1][i] = __int_as_float(out1[i]);
-        o_acc[2][i] = __int_as_float(out2[i]);
-        o_acc[3][i] = __int_as_float(out3[i]);
+        if constexpr (D == 128) {
+          o_acc[2][i] = __int_as_float(out2[i]);
+          o_acc[3][i] = __int_as_float(out3[i]);
+        }
       }
       first_tile = walk;
     }

@@ -152,8 +152,9 @@ def tile_body(e, p, stage, prio, label):
         # the row of additive terms, 16 bytes per lane: is any of them not zero?
         e.valu(f"v_mbcnt_lo_u32_b32 v{p.T[0]}, -1, 0", [p.T[0]])
         e.valu(f"v_and_b32_e32 v{p.T[0]}, {p.keys // 4 - 1}, v{p.T[0]}", [p.T[0]])
-        e.valu(f"v_lshl_add_u32 v{p.T[0]}, v{p.T[0]}, 4, s{p.lds}", [p.T[0]])
-        e.ds_read(p.PK[0], p.T[0], base + p.bias_region)
+        e.ins(f"s_add_u32 s{p.tmp_s}, s{p.lds}, {SEED_BIAS}")
+        e.valu(f"v_lshl_add_u32 v{p.T[0]}, v{p.T[0]}, 4, s{p.tmp_s}", [p.T[0]])
+        e.ds_read(p.PK[0], p.T[0], base + p.bias_region - SEED_BIAS)
     if p.mask == "f32":
         for kk in range(p.kk):
             source = p.ka
@@ -549,6 +550,14 @@ PROGRAMS = (
     Program("scaled_d128k128", 128, 128, scaled=True),
     Program("raw_d128k64", 128, 64, scaled=False),
     Program("f32mask_d128k64", 128, 64, scaled=True, mask="f32"),
+    Program("bias_d128k128", 128, 128, scaled=True, mask="bias"),
+    Program("bias_listed_d128k128", 128, 128, scaled=True, mask="bias", listed=True),
+    Program("lanes_listed_d128k64", 128, 64, scaled=True, mask="lanes", listed=True),
+    Program("raw_d64k64", 64, 64, scaled=False),
+    Program("scaled_d64k64", 64, 64, scaled=True),
+    Program("bias_d64k64", 64, 64, scaled=True, mask="bias"),
+    Program("bias_listed_d64k64", 64, 64, scaled=True, mask="bias", listed=True),
+    Program("lanes_listed_d64k64", 64, 64, scaled=True, mask="lanes", listed=True),
 )
 
 
