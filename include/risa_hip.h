@@ -115,6 +115,17 @@ int risa_sdpa_quantize(const void* q, void* q_int8, float* q_scale, const void* 
                        int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b, int64_t v_stride_h,
                        int64_t v_stride_n, int input_dtype, int midpoint_affine,
                        int32_t* anchor_indices, const int32_t* kv_permutation, void* stream);
+/* The same for rows that hold `channels` of the head_dim channels (a multiple of eight, rows of q,
+ * k and v 16-byte aligned): the others count as zeros, as if the rows had been padded beforehand. */
+int risa_sdpa_quantize_channels(const void* q, void* q_int8, float* q_scale, const void* k, void* k_int8,
+                       float* k_scale, const void* v, void* v_int8, float* v_scale, float* v_center,
+                       int32_t* v_tile_sum, void* v_workspace, size_t v_workspace_bytes, int batch,
+                       int q_heads, int q_len, int kv_heads, int k_len, int head_dim, int cta_k,
+                       int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_b,
+                       int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b, int64_t v_stride_h,
+                       int64_t v_stride_n, int input_dtype, int midpoint_affine,
+                       int32_t* anchor_indices, const int32_t* kv_permutation, int channels,
+                       void* stream);
 
 /*
  * Zero-point terms (128 x tile sums) of an already packed V matrix (for callers that build packed V
@@ -212,6 +223,18 @@ int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* work
               int64_t mask_stride_q, int64_t mask_stride_k, int mask_dtype, int mask_batch,
               int mask_heads, int is_causal, const int32_t* sparse_row_offsets,
               const int32_t* sparse_block_indices, void* stream);
+/* The same for rows of q, k and v that hold `channels` of the head_dim channels (see
+ * risa_sdpa_quantize_channels); the output rows are head_dim wide. */
+int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, void* workspace,
+              size_t workspace_bytes, int batch, int q_heads, int q_len, int kv_heads, int k_len,
+              int head_dim, int cta_k, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
+              int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b,
+              int64_t v_stride_h, int64_t v_stride_n, int64_t out_stride_b, int64_t out_stride_n,
+              int64_t out_stride_h, float sm_scale, int input_dtype, int output_dtype,
+              int midpoint_affine, const void* mask, int64_t mask_stride_b, int64_t mask_stride_h,
+              int64_t mask_stride_q, int64_t mask_stride_k, int mask_dtype, int mask_batch,
+              int mask_heads, int is_causal, const int32_t* sparse_row_offsets,
+              const int32_t* sparse_block_indices, int channels, void* stream);
 
 /*
  * Retained-mass selection over masses already sorted in descending order.

@@ -20,11 +20,12 @@ from .policy import (
     QUERY_BLOCK_SIZE,
     UNAVAILABLE,
     is_available,
+    kernel_head_dim,
     mask_signature,
     select_key_block_size,
     validate_inputs,
 )
-from .prepare import pad_head_dim, resolve_scale
+from .prepare import pad_head_dim, resolve_scale, rows_hold_whole_runs
 from .types import PrequantizedInt8Attention, RetainedMassPattern
 
 
@@ -196,7 +197,9 @@ def execute_dense_attention(
         raise ValueError(f"output_layout must be one of {OUTPUT_LAYOUTS}, got {output_layout!r}")
     attn_mask = validate_inputs(q, k, v, attn_mask)
     original_dim, input_dtype = q.shape[-1], q.dtype
-    q, k, v, dim = pad_head_dim(q, k, v)
+    dim = kernel_head_dim(original_dim)
+    if dim != original_dim and not rows_hold_whole_runs(q, k, v):
+        q, k, v, dim = pad_head_dim(q, k, v)
     attention_scale = resolve_scale(scale, original_dim)
     batch, q_heads, q_len, _ = q.shape
     kv_heads, k_len = k.shape[1], k.shape[2]
@@ -226,13 +229,13 @@ def execute_dense_attention(
                              mask_args[5], mask_args[3], mask_args[4], mask_args[6], mask_args[7]),
         dtype=torch.uint8, device=q.device)
     native.check(
-        lib.risa_sdpa(
+        lib.risa_sdpa_channels(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), output.data_ptr(), workspace.data_ptr(),
             workspace.numel(), batch, q_heads, q_len, kv_heads, k_len, dim, cta_k,
             q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
             v.stride(0), v.stride(1), v.stride(2), output.stride(0), output.stride(2), output.stride(1),
             attention_scale, DTYPE_CODES[input_dtype], DTYPE_CODES[output.dtype],
-            int(use_midpoint_affine), *mask_args, int(bool(is_causal)), *csr,
+            int(use_midpoint_affine), *mask_args, int(bool(is_causal)), *csr, q.shape[-1],
             native.current_stream(q.device),
         )
     )

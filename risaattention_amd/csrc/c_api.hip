@@ -95,12 +95,33 @@ int checked_qk_args(risa::QkArgs& a, const void* q, void* q_int8, float* q_scale
   a.head_dim = head_dim;
   a.cta_k = cta_k;
   a.dtype = input_dtype;
+  a.channels = head_dim;
   a.q_stride_b = q_stride_b;
   a.q_stride_h = q_stride_h;
   a.q_stride_n = q_stride_n;
   a.k_stride_b = k_stride_b;
   a.k_stride_h = k_stride_h;
   a.k_stride_n = k_stride_n;
+  return 0;
+}
+
+// Rows of `channels` elements stand for rows of head_dim with zeros behind them.  The fused
+// preparation reads them in runs of eight channels, 16 bytes at least, so the count is a multiple of
+// eight and Q and K keep the alignment V is always asked for.
+int checked_channels(risa::QkArgs& a, int channels) {
+  using risa::fail;
+  if (channels == a.head_dim) return 0;
+  if (channels <= 0 || channels > a.head_dim || channels % 8 != 0)
+    return fail("risa: channels must be a multiple of 8 of at most head_dim");
+  const int64_t per_16_bytes = a.dtype == 0 ? 4 : 8;
+  auto rows_ok = [&](const void* base, int heads, int length, int64_t stride_b, int64_t stride_h, int64_t stride_n) {
+    return aligned(base, 16) && stride_multiple(stride_b, a.batch, per_16_bytes) &&
+           stride_multiple(stride_h, heads, per_16_bytes) && stride_multiple(stride_n, length, per_16_bytes);
+  };
+  if (!rows_ok(a.q, a.q_heads, a.q_len, a.q_stride_b, a.q_stride_h, a.q_stride_n) ||
+      !rows_ok(a.k, a.kv_heads, a.k_len, a.k_stride_b, a.k_stride_h, a.k_stride_n))
+    return fail("risa: rows of fewer channels than head_dim must be 16-byte aligned");
+  a.channels = channels;
   return 0;
 }
 
@@ -213,20 +234,22 @@ int risa_quantize_v_noalloc(const void* v, void* out, float* scale, float* cente
   return risa::launch_quantize_v(a, static_cast<hipStream_t>(stream));
 }
 
-int risa_sdpa_quantize(const void* q, void* q_int8, float* q_scale, const void* k, void* k_int8,
+int risa_sdpa_quantize_channels(const void* q, void* q_int8, float* q_scale, const void* k, void* k_int8,
                        float* k_scale, const void* v, void* v_int8, float* v_scale, float* v_center,
                        int32_t* v_tile_sum, void* v_workspace, size_t v_workspace_bytes, int batch,
                        int q_heads, int q_len, int kv_heads, int k_len, int head_dim, int cta_k,
                        int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_b,
                        int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b, int64_t v_stride_h,
                        int64_t v_stride_n, int input_dtype, int midpoint_affine,
-                       int32_t* anchor_indices, const int32_t* kv_permutation, void* stream) {
+                       int32_t* anchor_indices, const int32_t* kv_permutation, int channels,
+                       void* stream) {
   if (cta_k != 64 && cta_k != 128) return risa::fail("risa_sdpa_quantize: cta_k must be 64 or 128");
   const int padded = (k_len + cta_k - 1) / cta_k * cta_k;
   risa::QkArgs qk{};
   int status = checked_qk_args(qk, q, q_int8, q_scale, k, k_int8, k_scale, batch, q_heads, q_len, kv_heads,
                                k_len, head_dim, cta_k, q_stride_b, q_stride_h, q_stride_n, k_stride_b,
                                k_stride_h, k_stride_n, input_dtype, anchor_indices, kv_permutation);
+  if (status == 0) status = checked_channels(qk, channels);
   if (status != 0) return status;
   risa::ValueArgs value{};
   status = checked_v_args(value, v, v_int8, v_scale, v_center, v_tile_sum, v_workspace, v_workspace_bytes,
@@ -235,9 +258,22 @@ int risa_sdpa_quantize(const void* q, void* q_int8, float* q_scale, const void* 
   if (status != 0) return status;
   hipStream_t hip_stream = static_cast<hipStream_t>(stream);
   if (risa::can_prepare_fused(qk, value)) return risa::launch_prepare_fused(qk, value, hip_stream);
+  if (channels != head_dim)
+    return risa::fail("risa_sdpa_quantize: rows of fewer channels than head_dim need the fused preparation");
   status = risa::launch_quantize_qk(qk, hip_stream);
   if (status != 0) return status;
   return risa::launch_quantize_v(value, hip_stream);
+}
+
+int risa_sdpa_quantize(const void* q, void* q_int8, float* q_scale, const void* k, void* k_int8,
+                       float* k_scale, const void* v, void* v_int8, float* v_scale, float* v_center,
+                       int32_t* v_tile_sum, void* v_workspace, size_t v_workspace_bytes, int batch,
+                       int q_heads, int q_len, int kv_heads, int k_len, int head_dim, int cta_k,
+                       int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_b,
+                       int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b, int64_t v_stride_h,
+                       int64_t v_stride_n, int input_dtype, int midpoint_affine,
+                       int32_t* anchor_indices, const int32_t* kv_permutation, void* stream) {
+  return risa_sdpa_quantize_channels(q, q_int8, q_scale, k, k_int8, k_scale, v, v_int8, v_scale, v_center, v_tile_sum, v_workspace, v_workspace_bytes, batch, q_heads, q_len, kv_heads, k_len, head_dim, cta_k, q_stride_b, q_stride_h, q_stride_n, k_stride_b, k_stride_h, k_stride_n, v_stride_b, v_stride_h, v_stride_n, input_dtype, midpoint_affine, anchor_indices, kv_permutation, head_dim, stream);
 }
 
 int risa_value_tile_sums(const void* v_int8, int32_t* tile_sum, int batch_heads, int head_dim,
@@ -480,7 +516,7 @@ size_t risa_sdpa_workspace_bytes(int batch, int q_heads, int q_len, int kv_heads
       .bytes;
 }
 
-int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* workspace,
+int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, void* workspace,
               size_t workspace_bytes, int batch, int q_heads, int q_len, int kv_heads, int k_len,
               int head_dim, int cta_k, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
               int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b,
@@ -489,7 +525,7 @@ int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* work
               int midpoint_affine, const void* mask, int64_t mask_stride_b, int64_t mask_stride_h,
               int64_t mask_stride_q, int64_t mask_stride_k, int mask_dtype, int mask_batch,
               int mask_heads, int is_causal, const int32_t* sparse_row_offsets,
-              const int32_t* sparse_block_indices, void* stream) {
+              const int32_t* sparse_block_indices, int channels, void* stream) {
   using risa::fail;
   if (batch <= 0 || q_heads <= 0 || q_len <= 0 || kv_heads <= 0 || k_len <= 0 ||
       (cta_k != 64 && cta_k != 128))
@@ -520,6 +556,7 @@ int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* work
                                q_heads, q_len, kv_heads, k_len, head_dim, cta_k, q_stride_b,
                                q_stride_h, q_stride_n, k_stride_b, k_stride_h, k_stride_n,
                                input_dtype, reinterpret_cast<int32_t*>(base + l.anchors), nullptr);
+  if (status == 0) status = checked_channels(qk, channels);
   if (status != 0) return status;
   risa::ValueArgs value{};
   status = checked_v_args(value, v, base + l.v_codes, v_scale, v_center, tile_sum,
@@ -530,6 +567,8 @@ int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* work
   hipStream_t hip_stream = static_cast<hipStream_t>(stream);
   if (risa::can_prepare_fused(qk, value)) {
     status = risa::launch_prepare_fused(qk, value, hip_stream);
+  } else if (channels != head_dim) {
+    return fail("risa_sdpa: rows of fewer channels than head_dim need the fused preparation");
   } else {
     status = risa::launch_quantize_qk(qk, hip_stream);
     if (status == 0) status = risa::launch_quantize_v(value, hip_stream);
@@ -576,6 +615,19 @@ int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* work
                         sm_scale, output_dtype, sparse_row_offsets, sparse_block_indices, nullptr,
                         is_causal, nullptr, key_tiles, key_bias, bias_stride_b, bias_stride_h,
                         mask_lanes, lanes_stride_b, lanes_stride_h, stream);
+}
+
+int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* workspace,
+              size_t workspace_bytes, int batch, int q_heads, int q_len, int kv_heads, int k_len,
+              int head_dim, int cta_k, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
+              int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b,
+              int64_t v_stride_h, int64_t v_stride_n, int64_t out_stride_b, int64_t out_stride_n,
+              int64_t out_stride_h, float sm_scale, int input_dtype, int output_dtype,
+              int midpoint_affine, const void* mask, int64_t mask_stride_b, int64_t mask_stride_h,
+              int64_t mask_stride_q, int64_t mask_stride_k, int mask_dtype, int mask_batch,
+              int mask_heads, int is_causal, const int32_t* sparse_row_offsets,
+              const int32_t* sparse_block_indices, void* stream) {
+  return risa_sdpa_channels(q, k, v, out, workspace, workspace_bytes, batch, q_heads, q_len, kv_heads, k_len, head_dim, cta_k, q_stride_b, q_stride_h, q_stride_n, k_stride_b, k_stride_h, k_stride_n, v_stride_b, v_stride_h, v_stride_n, out_stride_b, out_stride_n, out_stride_h, sm_scale, input_dtype, output_dtype, midpoint_affine, mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, mask_batch, mask_heads, is_causal, sparse_row_offsets, sparse_block_indices, head_dim, stream);
 }
 
 }  // extern "C"

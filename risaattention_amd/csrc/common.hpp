@@ -128,6 +128,25 @@ __device__ __forceinline__ float load1(const void* base, int64_t offset) {
   }
 }
 
+// Elements channel .. channel + COUNT - 1 (4 or 8) of the row at element offset `row`.  PAD: the
+// row holds `channels` elements (a multiple of COUNT); runs past them read the first run of the
+// row instead and count as zeros.
+template <int DT, int COUNT, bool PAD>
+__device__ __forceinline__ void load_channels(const void* base, int64_t row, int channel, int channels, float (&out)[COUNT]) {
+  static_assert(COUNT == 4 || COUNT == 8, "runs of four or eight channels");
+  const bool held = !PAD || channel < channels;
+  const int64_t offset = row + (held ? channel : 0);
+  if constexpr (COUNT == 8) {
+    load8<DT>(base, offset, out);
+  } else {
+    load4<DT>(base, offset, out);
+  }
+  if constexpr (PAD) {
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) out[i] = held ? out[i] : 0.0f;
+  }
+}
+
 // Round to nearest even, saturate to the signed 8-bit range, NaN -> 0.
 // Round-to-nearest-even conversion of a code in [-127.5, 127.5] by adding 1.5 * 2^23: the sum's
 // integer part is rint(value) (the sum has an ulp of 1 and 1.5 * 2^23 is even, so ties go to the

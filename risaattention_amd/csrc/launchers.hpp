@@ -21,6 +21,7 @@ struct QkArgs {
   int* anchors;
   const int32_t* permutation;  // [B,Hkv,Lk] source token of every key, or null
   int batch, q_heads, q_len, kv_heads, k_len, head_dim, cta_k, dtype;
+  int channels;  // of head_dim that the rows of q, k (and v) hold; the others count as zeros
   int64_t q_stride_b, q_stride_h, q_stride_n;
   int64_t k_stride_b, k_stride_h, k_stride_n;
 };

@@ -207,12 +207,13 @@ __device__ __forceinline__ float half_wave_max(float value) {
 // `own_max` / `partner_max` (optional): LDS slots through which two wavefronts that share one
 // scale group (each with NTOK of its tokens) exchange their maxima; `own_max` is written, a
 // workgroup barrier follows, `partner_max` is read.  The maximum is order independent.
-template <int DT, int DK, int ROT, int NTOK, int LANES = 32, typename TokenOf>
+// PAD: rows hold `channels` of the DK channels, the rest counts as zeros.
+template <int DT, int DK, int ROT, int NTOK, int LANES = 32, bool PAD = false, typename TokenOf>
 __device__ __forceinline__ void quantize_group(const void* in, int64_t in_base, int64_t stride_n,
                                                int8_t* out, float* scale_slot, int length, int sub,
                                                bool has_bias, int64_t bias_offset, bool wide, TokenOf token_of,
                                                const int32_t* source = nullptr, float* own_max = nullptr,
-                                               const float* partner_max = nullptr) {
+                                               const float* partner_max = nullptr, int channels = DK) {
   constexpr int BLOCKS = DK == 256 ? 2 : 1;   // 128-channel rotation blocks
   constexpr int GROUPS = DK == 64 ? 1 : 2;    // runs of four channels per lane and block
   constexpr int PER_STEP = LANES / 16;
@@ -251,12 +252,12 @@ __device__ __forceinline__ void quantize_group(const void* in, int64_t in_base, 
       for (int block = 0; block < BLOCKS; ++block) {
         if constexpr (EIGHT) {
           float eight[8];
-          load8<DT>(in, row_base + channel_of(block, 0), eight);
+          load_channels<DT, 8, PAD>(in, row_base, channel_of(block, 0), channels, eight);
 #pragma unroll
           for (int c = 0; c < 8; ++c) dst[block][c / 4][c % 4] = eight[c];
         } else {
 #pragma unroll
-          for (int g = 0; g < GROUPS; ++g) load4<DT>(in, row_base + channel_of(block, g), dst[block][g]);
+          for (int g = 0; g < GROUPS; ++g) load_channels<DT, 4, PAD>(in, row_base, channel_of(block, g), channels, dst[block][g]);
         }
       }
     };
@@ -338,12 +339,12 @@ __device__ __forceinline__ void quantize_group(const void* in, int64_t in_base, 
 
 // One W-row slice of one (batch, head): eight 32-lane halves = the eight scale
 // groups (token index mod 8), W = 32 (16 for head_dim 256).  256 threads.
-template <int DT, int DK, int ROT>
+template <int DT, int DK, int ROT, bool PAD = false>
 __device__ __forceinline__ void quantize_q_block(const void* __restrict__ q, int8_t* __restrict__ codes,
                                                  float* __restrict__ scales, int length, int heads,
                                                  int scales_per_head, int64_t stride_b,
                                                  int64_t stride_h, int64_t stride_n, int wide,
-                                                 int slice, int h, int b) {
+                                                 int slice, int h, int b, int channels = DK) {
   constexpr int W = DK == 256 ? 16 : 32;
   constexpr int NR = W / 8;
   const int sub = threadIdx.x & 31;
@@ -351,9 +352,9 @@ __device__ __forceinline__ void quantize_q_block(const void* __restrict__ q, int
   const int64_t in_base = static_cast<int64_t>(b) * stride_b + static_cast<int64_t>(h) * stride_h;
   const int64_t bh = static_cast<int64_t>(b) * heads + h;
   const int base = slice * W + group;
-  quantize_group<DT, DK, ROT, NR>(q, in_base, stride_n, codes + bh * length * DK,
+  quantize_group<DT, DK, ROT, NR, 32, PAD>(q, in_base, stride_n, codes + bh * length * DK,
                                   scales + bh * scales_per_head + slice * 8 + group, length, sub,
-                                  false, 0, wide != 0, [base](int i) { return base + i * 8; });
+                                  false, 0, wide != 0, [base](int i) { return base + i * 8; }, nullptr, nullptr, nullptr, channels);
 }
 
 // grid (slices, Hq, B), 256 threads.  One slice (8 KB of input) per workgroup: two or
@@ -375,13 +376,13 @@ __global__ __launch_bounds__(256) void quantize_q_kernel(const void* __restrict_
 // group, each with half of the group's tokens, four tokens per step; the two exchange their
 // maxima through LDS.  A wavefront then keeps CTA_K / 8 rotated tokens in registers instead of
 // CTA_K / 4, and twice as many wavefronts stand behind every tile.
-template <int DT, int DK, int CTA_K, int ROT>
+template <int DT, int DK, int CTA_K, int ROT, bool PAD = false>
 __device__ __forceinline__ void quantize_k_block(const void* __restrict__ k, int8_t* __restrict__ codes,
                                                  float* __restrict__ scales, int anchor, int length,
                                                  int heads, int scales_per_head, int64_t stride_b,
                                                  int64_t stride_h, int64_t stride_n, int wide,
                                                  const int32_t* __restrict__ permutation, int tile,
-                                                 int part, int h, int b) {
+                                                 int part, int h, int b, int channels = DK) {
   constexpr int NTOK = CTA_K / 8;  // tokens of the group held by one wavefront
   __shared__ float wave_max[4];
   const int sub = threadIdx.x & 63;
@@ -395,11 +396,11 @@ __device__ __forceinline__ void quantize_k_block(const void* __restrict__ k, int
   const int anchor_row = anchor >= 0 && source != nullptr ? source[anchor] : anchor;
   const int64_t anchor_offset = static_cast<int64_t>(anchor_row) * stride_n;
   const int first = tile * CTA_K + group * 2;
-  quantize_group<DT, DK, ROT, NTOK, 64>(
+  quantize_group<DT, DK, ROT, NTOK, 64, PAD>(
       k, in_base, stride_n, codes + bh * length * DK, scales + bh * scales_per_head + tile * 4 + group,
       length, sub, anchor >= 0, anchor_offset, wide != 0,
       [first, first_index](int i) { return first + ((i + first_index) >> 1) * 8 + ((i + first_index) & 1); },
-      source, wave_max + wave, wave_max + (wave ^ 1));
+      source, wave_max + wave, wave_max + (wave ^ 1), channels);
 }
 
 // grid (2 * key tiles, Hkv, B), 256 threads: half a key tile of CTA_K tokens per workgroup.
@@ -441,10 +442,12 @@ __device__ __forceinline__ float segment_down_sum(float value) {
 __device__ __forceinline__ float segment_down_max(float value) { return half_wave_max(value); }
 
 // Returns the anchor row of (b, h), or -1, to every thread of the workgroup.
-template <int DT>
+// PAD: rows hold `channels` of the `dim` channels, the rest counts as zeros.
+template <int DT, bool PAD = false>
 __device__ __forceinline__ int detect_anchor_value(const void* __restrict__ k, int length, int dim, int heads,
                                                    int64_t stride_b, int64_t stride_h, int64_t stride_n,
-                                                   const int32_t* __restrict__ permutation, int h, int b) {
+                                                   const int32_t* __restrict__ permutation, int h, int b,
+                                                   int channels = 0) {
   __shared__ float samples[kSamples * 256];
   __shared__ float seg_energy[4], seg_max[4], seg_dist[kSamples][4], seg_best_energy[4],
       seg_best_max[4];
@@ -467,7 +470,7 @@ __device__ __forceinline__ int detect_anchor_value(const void* __restrict__ k, i
 #pragma unroll
     for (int part = 0; part < 2; ++part) {
       // a channel past the head dim reads channel 0 (never stored)
-      const int channel = tid + part * 128 < dim && working ? tid + part * 128 : 0;
+      const int channel = tid + part * 128 < (PAD ? channels : dim) && working ? tid + part * 128 : 0;
 #pragma unroll
       for (int s = 0; s < kSamples; ++s) fetched[part][s] = load1<DT>(k, base + rows[s] * stride_n + channel);
     }
@@ -476,7 +479,7 @@ __device__ __forceinline__ int detect_anchor_value(const void* __restrict__ k, i
       const int channel = tid + part * 128;
       if (working && channel < dim) {
 #pragma unroll
-        for (int s = 0; s < kSamples; ++s) samples[s * dim + channel] = fetched[part][s];
+        for (int s = 0; s < kSamples; ++s) samples[s * dim + channel] = !PAD || channel < channels ? fetched[part][s] : 0.0f;
       }
     }
   }
@@ -558,13 +561,13 @@ __device__ __forceinline__ int detect_anchor_value(const void* __restrict__ k, i
   return chosen;
 }
 
-template <int DT>
+template <int DT, bool PAD = false>
 __device__ __forceinline__ void detect_anchor_block(const void* __restrict__ k, int* __restrict__ anchors,
                                                     int length, int dim, int heads, int64_t stride_b,
                                                     int64_t stride_h, int64_t stride_n,
                                                     const int32_t* __restrict__ permutation, int h,
-                                                    int b) {
-  const int anchor = detect_anchor_value<DT>(k, length, dim, heads, stride_b, stride_h, stride_n, permutation, h, b);
+                                                    int b, int channels = 0) {
+  const int anchor = detect_anchor_value<DT, PAD>(k, length, dim, heads, stride_b, stride_h, stride_n, permutation, h, b, channels);
   if (threadIdx.x == 0) anchors[b * heads + h] = anchor;
 }
 

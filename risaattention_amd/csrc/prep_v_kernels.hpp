@@ -69,12 +69,13 @@ __device__ __forceinline__ int first_token_of_positions(int p0) {
 // 16 bytes of a 16-bit input per lane), so every load instruction of the wavefront
 // covers whole consecutive rows; the lanes holding the same channels are combined
 // with xor shuffles at the end.  min/max do not depend on the order.
-template <int DT, bool AFFINE>
+// PAD (here and below): rows hold `channels` of the channels, the rest counts as zeros.
+template <int DT, bool AFFINE, bool PAD = false>
 __device__ __forceinline__ void value_range_block(const void* __restrict__ v, float* __restrict__ part_max,
                                                   float* __restrict__ part_min, int length, int dim,
                                                   int heads, int chunks, int64_t stride_b,
                                                   int64_t stride_h, int64_t stride_n, int chunk_group,
-                                                  int bh) {
+                                                  int bh, int channels = 0) {
   const int b = bh / heads, h = bh - b * heads;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int chunk = chunk_group * 4 + wave;
@@ -99,7 +100,7 @@ __device__ __forceinline__ void value_range_block(const void* __restrict__ v, fl
     // loop keep eight of them in flight.
     const int n = min(first + t, length - 1);
     float x[8];
-    load8<DT>(v, base + static_cast<int64_t>(n) * stride_n + octet * 8, x);
+    load_channels<DT, 8, PAD>(v, base + static_cast<int64_t>(n) * stride_n, octet * 8, channels, x);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       if constexpr (AFFINE) {
@@ -231,7 +232,7 @@ struct FusedParams {
   int chunks;
 };
 
-template <int DT, int CTA_K, int PARAMS, int DK>
+template <int DT, int CTA_K, int PARAMS, int DK, bool PAD = false>
 __device__ __forceinline__ void value_codes_block(const void* __restrict__ v, int8_t* __restrict__ codes,
                                                   int32_t* __restrict__ tile_sum,
                                                   const float* __restrict__ inverse,
@@ -239,7 +240,8 @@ __device__ __forceinline__ void value_codes_block(const void* __restrict__ v, in
                                                   int padded, int heads, int64_t stride_b,
                                                   int64_t stride_h, int64_t stride_n,
                                                   const int32_t* __restrict__ permutation,
-                                                  const FusedParams& fused, int position_block, int bh) {
+                                                  const FusedParams& fused, int position_block, int bh,
+                                                  int channels = DK) {
   constexpr int OCTETS = DK / 8;        // lanes per token row
   constexpr int SLOTS = 256 / OCTETS;   // quads of positions in flight per load
   constexpr int QUADS = 32 / SLOTS;     // quads per thread
@@ -286,7 +288,7 @@ __device__ __forceinline__ void value_codes_block(const void* __restrict__ v, in
 #pragma unroll
       for (int j = 0; j < IN_FLIGHT; ++j) {
         const int n = min((first_pass + j) * SLOTS + slot, length - 1);
-        load8<DT>(v, base + static_cast<int64_t>(n) * stride_n + octet * 8, rows_in_flight[j]);
+        load_channels<DT, 8, PAD>(v, base + static_cast<int64_t>(n) * stride_n, octet * 8, channels, rows_in_flight[j]);
       }
 #pragma unroll
       for (int j = 0; j < IN_FLIGHT; ++j) {
@@ -406,7 +408,7 @@ __device__ __forceinline__ void value_codes_block(const void* __restrict__ v, in
     for (int j = 0; j < BATCH; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        load8<DT>(v, base + static_cast<int64_t>(from[j][r]) * stride_n + octet * 8, x[j][r]);
+        load_channels<DT, 8, PAD>(v, base + static_cast<int64_t>(from[j][r]) * stride_n, octet * 8, channels, x[j][r]);
 #pragma unroll
     for (int j = 0; j < BATCH; ++j) {
       const int quad = slot + SLOTS * (first + j);
@@ -469,14 +471,14 @@ __global__ __launch_bounds__(256) void value_codes_kernel(const void* __restrict
 
 // grid (T / (256/quads), B*H), 256 threads: thread = (summation thread t, four channels);
 // four rather than eight channels per thread so that a long sequence fills every SIMD.
-template <int DT>
+template <int DT, bool PAD = false>
 __device__ __forceinline__ void value_residual_block(const void* __restrict__ v, float* __restrict__ partial,
                                                      const float* __restrict__ inverse,
                                                      const float* __restrict__ midpoint, int length,
                                                      int dim, int heads, int threads, int64_t stride_b,
                                                      int64_t stride_h, int64_t stride_n,
                                                      const int32_t* __restrict__ permutation,
-                                                     int block, int bh) {
+                                                     int block, int bh, int channels = 0) {
   const int b = bh / heads, h = bh - b * heads;
   const int quads = dim / 4;
   const int quad = threadIdx.x % quads;
@@ -513,7 +515,7 @@ __device__ __forceinline__ void value_residual_block(const void* __restrict__ v,
       }
 #pragma unroll
       for (int j = 0; j < kInFlight; ++j)
-        load4<DT>(v, base + static_cast<int64_t>(from[j]) * stride_n + quad * 4, x[j]);
+        load_channels<DT, 4, PAD>(v, base + static_cast<int64_t>(from[j]) * stride_n, quad * 4, channels, x[j]);
 #pragma unroll
       for (int j = 0; j < kInFlight; ++j) {
         if (src0 - j * threads >= 0) {
@@ -579,12 +581,12 @@ __global__ __launch_bounds__(512) void value_center_from_partials_kernel(
 // threads t and t + 256 one after the other.  Warp totals land in the reference's order.
 // WALK: the ranges of the block's eight channels come from a walk over the whole sequence
 // instead of the partial ranges of an earlier launch.
-template <int DT, bool WALK = false>
+template <int DT, bool WALK = false, bool PAD = false>
 __device__ __forceinline__ void value_center_block(const void* __restrict__ v, const FusedParams& fused,
                                                    int length, int dim, int heads, int64_t stride_b,
                                                    int64_t stride_h, int64_t stride_n,
                                                    const int32_t* __restrict__ permutation, int octet,
-                                                   int bh) {
+                                                   int bh, int channels = 0) {
   __shared__ float warp_total[8][16];
   __shared__ float parameters[2][8];
   const int b = bh / heads, h = bh - b * heads;
@@ -604,7 +606,7 @@ __device__ __forceinline__ void value_center_block(const void* __restrict__ v, c
 #pragma unroll 4
     for (int pass = 0; pass < passes; ++pass) {
       float x[8];
-      load8<DT>(v, base + static_cast<int64_t>(min(pass * 256 + t, length - 1)) * stride_n + octet * 8, x);
+      load_channels<DT, 8, PAD>(v, base + static_cast<int64_t>(min(pass * 256 + t, length - 1)) * stride_n, octet * 8, channels, x);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         mx[i] = __builtin_fmaxf(mx[i], x[i]);
@@ -683,7 +685,7 @@ __device__ __forceinline__ void value_center_block(const void* __restrict__ v, c
         }
 #pragma unroll
         for (int j = 0; j < kInFlight; ++j)
-          load8<DT>(v, base + static_cast<int64_t>(from[j]) * stride_n + octet * 8, x[j]);
+          load_channels<DT, 8, PAD>(v, base + static_cast<int64_t>(from[j]) * stride_n, octet * 8, channels, x[j]);
 #pragma unroll
         for (int j = 0; j < kInFlight; ++j) {
           if (src0 - j * threads >= 0) {

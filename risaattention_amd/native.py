@@ -47,6 +47,10 @@ SIGNATURES = {
         _c_int,
         [_c_ptr] * 12 + [_c_size] + [_c_int] * 7 + [_c_i64] * 9 + [_c_int, _c_int, _c_ptr, _c_ptr, _c_ptr],
     ),
+    "risa_sdpa_quantize_channels": (
+        _c_int,
+        [_c_ptr] * 12 + [_c_size] + [_c_int] * 7 + [_c_i64] * 9 + [_c_int, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
+    ),
     "risa_value_tile_sums": (_c_int, [_c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr]),
     "risa_unpack_order": (None, [_c_ptr]),
     "risa_attention": (
@@ -72,6 +76,11 @@ SIGNATURES = {
         _c_int,
         [_c_ptr] * 5 + [_c_size] + [_c_int] * 7 + [_c_i64] * 12 + [_c_f32, _c_int, _c_int, _c_int]
         + [_c_ptr] + [_c_i64] * 4 + [_c_int] * 4 + [_c_ptr, _c_ptr, _c_ptr],
+    ),
+    "risa_sdpa_channels": (
+        _c_int,
+        [_c_ptr] * 5 + [_c_size] + [_c_int] * 7 + [_c_i64] * 12 + [_c_f32, _c_int, _c_int, _c_int]
+        + [_c_ptr] + [_c_i64] * 4 + [_c_int] * 4 + [_c_ptr, _c_ptr, _c_int, _c_ptr],
     ),
     "risa_selector_workspace_size": (_c_size, [_c_int]),
     "risa_select_retained_mass": (_c_int, [_c_ptr] * 8 + [_c_int, _c_int, _c_f64, _c_ptr]),

@@ -54,6 +54,21 @@ def pad_head_dim(q, k, v):
     return q, k, v, kernel_dim
 
 
+def rows_hold_whole_runs(*tensors) -> bool:
+    """Whether the preparation kernels can read rows shorter than the kernel's head dim where they
+    are: whole runs of eight channels, every row on a 16-byte boundary."""
+    if tensors[0].shape[-1] % 8 != 0:
+        return False
+    for tensor in tensors:
+        run = 16 // tensor.element_size()
+        if tensor.stride(-1) != 1 or tensor.data_ptr() % 16 != 0:
+            return False
+        for extent, stride in zip(tensor.shape[:-1], tensor.stride()[:-1]):
+            if extent > 1 and (stride <= 0 or stride % run != 0):
+                return False
+    return True
+
+
 def resolve_scale(scale: float | None, head_dim: int) -> float:
     value = head_dim**-0.5 if scale is None else float(scale)
     if not math.isfinite(value):
@@ -62,18 +77,21 @@ def resolve_scale(scale: float | None, head_dim: int) -> float:
 
 
 def quantize_inputs(q, k, v, attn_mask, scale, use_midpoint_affine: bool,
-                    kv_permutation: torch.Tensor | None = None) -> PreparedBuffers:
+                    kv_permutation: torch.Tensor | None = None, keep_rows: bool = False) -> PreparedBuffers:
     """Allocate the packed buffers and enqueue the Q/K and V preparation kernels.
 
     ``q``, ``k``, ``v`` are validated; ``attn_mask`` is already broadcast (its
     query stride decides the key tile size).  ``kv_permutation`` (int32
     ``[B,Hkv,Lk]``) makes the K and V kernels read key ``n`` from source token
-    ``kv_permutation[b,h,n]``: the gather fused into quantisation.
+    ``kv_permutation[b,h,n]``: the gather fused into quantisation.  ``keep_rows``: the
+    caller reads ``q_padded`` and ``k_padded`` (the LSE shift does).
     """
     lib = native.library()
     original_dim = q.shape[-1]
     input_dtype = q.dtype
-    q, k, v, dim = pad_head_dim(q, k, v)
+    dim = kernel_head_dim(original_dim)
+    if keep_rows or not rows_hold_whole_runs(q, k, v):
+        q, k, v, dim = pad_head_dim(q, k, v)
     attention_scale = resolve_scale(scale, original_dim)
     batch, q_heads, q_len, _ = q.shape
     _, kv_heads, k_len, _ = k.shape
@@ -86,8 +104,8 @@ def quantize_inputs(q, k, v, attn_mask, scale, use_midpoint_affine: bool,
     def empty(*shape, dtype):
         return torch.empty(shape, dtype=dtype, device=device)
 
-    q_codes = empty(*q.shape, dtype=torch.int8)
-    k_codes = empty(*k.shape, dtype=torch.int8)
+    q_codes = empty(batch, q_heads, q_len, dim, dtype=torch.int8)
+    k_codes = empty(batch, kv_heads, k_len, dim, dtype=torch.int8)
     q_scale = empty(batch, q_heads, -(-q_len // 128) * (64 if dim == 256 else 32), dtype=torch.float32)
     k_scale = empty(batch, kv_heads, -(-k_len // cta_k) * 4, dtype=torch.float32)
     v_codes = empty(rows, padded, dtype=torch.int8)
@@ -102,7 +120,7 @@ def quantize_inputs(q, k, v, attn_mask, scale, use_midpoint_affine: bool,
     stream = native.current_stream(device)
     code = DTYPE_CODES[input_dtype]
     native.check(
-        lib.risa_sdpa_quantize(
+        lib.risa_sdpa_quantize_channels(
             q.data_ptr(), q_codes.data_ptr(), q_scale.data_ptr(),
             k.data_ptr(), k_codes.data_ptr(), k_scale.data_ptr(),
             v.data_ptr(), v_codes.data_ptr(), v_scale.data_ptr(), v_center.data_ptr(),
@@ -110,7 +128,7 @@ def quantize_inputs(q, k, v, attn_mask, scale, use_midpoint_affine: bool,
             batch, q_heads, q_len, kv_heads, k_len, dim, cta_k,
             q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
             v.stride(0), v.stride(1), v.stride(2), code, int(use_midpoint_affine),
-            anchors.data_ptr(), native.pointer(kv_permutation), stream,
+            anchors.data_ptr(), native.pointer(kv_permutation), q.shape[-1], stream,
         )
     )
     return PreparedBuffers(q_codes, k_codes, v_codes, q_scale, k_scale, v_scale, v_center,
@@ -166,7 +184,8 @@ def prequantize_int8_attention(
             return_lse=return_lse, fuse=fuse_gather)
     use_midpoint_affine = uses_centered_values(v_quantization)
     original_dim, input_dtype = q.shape[-1], q.dtype
-    buffers = quantize_inputs(q, k, v, attn_mask, scale, use_midpoint_affine, fused_permutation)
+    buffers = quantize_inputs(q, k, v, attn_mask, scale, use_midpoint_affine, fused_permutation,
+                              keep_rows=return_lse)
     shift = lse_shift(buffers, input_dtype) if return_lse else None
     return PrequantizedInt8Attention(
         q=buffers.q_codes,
