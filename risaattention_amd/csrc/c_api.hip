@@ -591,22 +591,17 @@ int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, v
   }
   if (key_only) {
     auto* bias = reinterpret_cast<float*>(base + l.key_bias);
-    status = risa_prepare_key_bias(mask, bias, mask_batch, mask_heads, k_len, padded,
-                                   mask_batch > 1 ? mask_stride_b : 0,
-                                   mask_heads > 1 ? mask_stride_h : 0, mask_stride_k, mask_dtype,
-                                   stream);
-    if (status != 0) return status;
     key_bias = bias;
     bias_stride_h = mask_heads > 1 ? padded : 0;
     bias_stride_b = mask_batch > 1 ? static_cast<int64_t>(mask_heads) * padded : 0;
     // tile lists pay off under the conditions of reference _key_mask.py:9-28
-    if (k_len > 1024 && q_len >= 256 && sm_scale > 0.0f && is_causal == 0 && sparse_row_offsets == nullptr) {
-      auto* list = reinterpret_cast<int32_t*>(base + l.key_tiles);
-      status = risa_prepare_key_mask_tiles(mask, list, batch, q_heads, k_len, cta_k, mask_stride_b,
-                                           mask_stride_h, mask_stride_k, mask_dtype, stream);
-      if (status != 0) return status;
-      key_tiles = list;
-    }
+    const bool lists = k_len > 1024 && q_len >= 256 && sm_scale > 0.0f && is_causal == 0 && sparse_row_offsets == nullptr;
+    if (mask_dtype < 0 || mask_dtype > 3) return fail("risa_sdpa: attention mask must be bool, float16, bfloat16, or float32");
+    auto* list = lists ? reinterpret_cast<int32_t*>(base + l.key_tiles) : nullptr;
+    status = risa::launch_key_mask(mask, list, bias, batch, q_heads, mask_batch, mask_heads, k_len, padded, cta_k,
+                                   mask_stride_b, mask_stride_h, mask_stride_k, mask_dtype, hip_stream);
+    if (status != 0) return status;
+    key_tiles = list;
   }
   return risa_attention(base + l.q_codes, base + l.k_codes, base + l.v_codes, out, q_scale, k_scale,
                         v_scale, v_center, tile_sum, mask, mask_stride_b, mask_stride_h,

@@ -128,6 +128,11 @@ size_t mask_tile_list_offset(int batch, int heads, int q_len, int k_len);  // of
 int launch_mask_lanes(const void* mask, uint64_t* lanes, int batch, int heads, int q_len, int k_len,
                       int64_t stride_b, int64_t stride_h, int64_t stride_q, hipStream_t stream);
 
+// Both of one key-only mask in one launch; `tiles` may be null.
+int launch_key_mask(const void* mask, int32_t* tiles, float* bias, int batch, int heads, int mask_batch,
+                    int mask_heads, int length, int padded, int tile_size, int64_t stride_b,
+                    int64_t stride_h, int64_t stride_k, int dtype, hipStream_t stream);
+
 int launch_key_bias(const void* mask, float* bias, int batch, int heads, int length, int padded,
                     int64_t stride_b, int64_t stride_h, int64_t stride_k, int dtype,
                     hipStream_t stream);

@@ -192,78 +192,102 @@ __global__ __launch_bounds__(256) void compact_rows_kernel(const uint8_t* __rest
   }
 }
 
-__device__ __forceinline__ bool key_visible(const void* mask, int64_t index, int dtype) {
-  if (dtype == kBool) return static_cast<const uint8_t*>(mask)[index] != 0;
-  const float bias = dtype == kF32   ? load1<kF32>(mask, index)
-                     : dtype == kF16 ? load1<kF16>(mask, index)
-                                     : load1<kBF16>(mask, index);
-  return __builtin_isfinite(bias);
+// Both derived forms of a key-only mask in one launch: the list of tiles with a visible key per
+// (batch, head), and the additive row in the exp2 domain per mask plane (bias * log2(e), the FP32
+// product the attention kernel would form per score; -inf for hidden and out-of-range keys).
+// Either output may be null.
+struct KeyMaskArgs {
+  const void* mask;
+  int32_t* tiles;  // [batch, heads, tiles + 1]
+  float* bias;     // [bias_planes, padded]
+  int batch, heads, bias_heads, bias_planes, length, tile_size, padded;
+  int64_t stride_b, stride_h, stride_k;            // of the mask as the lists see it (0: shared)
+  int64_t bias_stride_b, bias_stride_h;
+};
+
+template <int DT> __device__ __forceinline__ float key_term(const void* mask, int64_t index) {
+  if constexpr (DT == kBool) {
+    return static_cast<const uint8_t*>(mask)[index] != 0 ? 0.0f : -__builtin_inff();
+  } else {
+    return load1<DT>(mask, index);
+  }
 }
 
-// One workgroup per (batch, head): flag tiles with any visible key, then one
-// wavefront compacts the active tile ids in ascending order and appends the count.
-__global__ __launch_bounds__(256) void key_mask_tiles_kernel(const void* __restrict__ mask,
-                                                             int32_t* __restrict__ output, int heads,
-                                                             int length, int tile_size,
-                                                             int64_t stride_b, int64_t stride_h,
-                                                             int64_t stride_k, int dtype) {
-  const int tiles = (length + tile_size - 1) / tile_size;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * heads + blockIdx.y;
-  const int64_t mask_row = blockIdx.x * stride_b + blockIdx.y * stride_h;
-  int32_t* out = output + row * (tiles + 1);
-  extern __shared__ int active_flags[];
-  for (int tile = wave; tile < tiles; tile += 4) {
-    bool visible = false;
-    for (int offset = lane; offset < tile_size; offset += 64) {
-      const int key = tile * tile_size + offset;
-      if (key < length) visible |= key_visible(mask, mask_row + key * stride_k, dtype);
+// The first batch * heads workgroups (when lists are asked for): flags of 64-key runs, eight loads
+// in flight per thread (one load per tile and wavefront, each waited for, took 10 us for 72
+// tiles), then one wavefront compacts the active tile ids in ascending order and appends the
+// count.  The others: 256 keys of a bias plane each.
+template <int DT> __global__ __launch_bounds__(256) void key_mask_kernel(const KeyMaskArgs a) {
+  extern __shared__ unsigned char run_flags[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int rows = a.tiles != nullptr ? a.batch * a.heads : 0;
+  if (static_cast<int>(blockIdx.x) >= rows) {
+    const int per_plane = (a.padded + 255) / 256;
+    const int block = blockIdx.x - rows;
+    const int plane = block / per_plane, key = block % per_plane * 256 + tid;
+    if (key >= a.padded) return;
+    float value = -__builtin_inff();
+    if (key < a.length) {
+      const float term = key_term<DT>(a.mask, plane / a.bias_heads * a.bias_stride_b + plane % a.bias_heads * a.bias_stride_h +
+                                                  key * a.stride_k);
+      if (__builtin_isfinite(term)) value = term * 1.44269504088896340736f;
     }
-    const bool any = __ballot(visible) != 0;
-    if (lane == 0) active_flags[tile] = any ? 1 : 0;
+    a.bias[static_cast<int64_t>(plane) * a.padded + key] = value;
+    return;
+  }
+  const int64_t row = blockIdx.x;
+  const int64_t mask_row = row / a.heads * a.stride_b + row % a.heads * a.stride_h;
+  constexpr int IN_FLIGHT = 8;
+  for (int first = 0; first < a.length; first += 256 * IN_FLIGHT) {
+    float term[IN_FLIGHT];
+#pragma unroll
+    for (int j = 0; j < IN_FLIGHT; ++j)
+      term[j] = key_term<DT>(a.mask, mask_row + min(first + j * 256 + tid, a.length - 1) * a.stride_k);
+#pragma unroll
+    for (int j = 0; j < IN_FLIGHT; ++j) {
+      const int run = first + j * 256 + wave * 64;  // first key of the wavefront's run
+      const bool any = __ballot(run + lane < a.length && __builtin_isfinite(term[j])) != 0;
+      if (lane == 0 && run < a.length) run_flags[run / 64] = any;
+    }
   }
   __syncthreads();
-  if (wave == 0) {
-    int count = 0;
-    for (int base = 0; base < tiles; base += 64) {
-      const int tile = base + lane;
-      const bool active = tile < tiles && active_flags[tile] != 0;
-      const uint64_t votes = __ballot(active);
-      if (active) {
-        const uint64_t lower = lane == 0 ? 0ull : (votes & ((1ull << lane) - 1ull));
-        out[count + __builtin_popcountll(lower)] = tile;
-      }
-      count += __builtin_popcountll(votes);
+  if (wave != 0) return;
+  const int tiles = (a.length + a.tile_size - 1) / a.tile_size;
+  const int runs = (a.length + 63) / 64, runs_per_tile = a.tile_size / 64;
+  int32_t* out = a.tiles + row * (tiles + 1);
+  int count = 0;
+  for (int base = 0; base < tiles; base += 64) {
+    const int tile = base + lane;
+    bool active = false;
+    for (int r = 0; r < runs_per_tile; ++r) {
+      const int run = tile * runs_per_tile + r;
+      active |= run < runs && run_flags[run] != 0;
     }
-    // Slots behind the active ids are never read by the attention kernel.
-    for (int slot = count + lane; slot < tiles; slot += 64) out[slot] = -1;
-    if (lane == 0) out[tiles] = count;
+    const uint64_t votes = __ballot(active);
+    if (active) {
+      const uint64_t lower = lane == 0 ? 0ull : (votes & ((1ull << lane) - 1ull));
+      out[count + __builtin_popcountll(lower)] = tile;
+    }
+    count += __builtin_popcountll(votes);
   }
+  // Slots behind the active ids are never read by the attention kernel.
+  for (int slot = count + lane; slot < tiles; slot += 64) out[slot] = -1;
+  if (lane == 0) out[tiles] = count;
 }
 
-// grid (ceil(padded/256), heads, batch), 256 threads: one key each.  The product
-// bias * log2(e) is the FP32 product the attention kernel would form per score.
-__global__ __launch_bounds__(256) void key_bias_kernel(const void* __restrict__ mask,
-                                                       float* __restrict__ bias, int length,
-                                                       int padded, int64_t stride_b, int64_t stride_h,
-                                                       int64_t stride_k, int dtype) {
-  const int key = blockIdx.x * 256 + threadIdx.x;
-  if (key >= padded) return;
-  float value = -__builtin_inff();
-  if (key < length) {
-    const int64_t index = blockIdx.z * stride_b + blockIdx.y * stride_h + key * stride_k;
-    if (dtype == kBool) {
-      if (static_cast<const uint8_t*>(mask)[index] != 0) value = 0.0f;
-    } else {
-      const float raw = dtype == kF32   ? load1<kF32>(mask, index)
-                        : dtype == kF16 ? load1<kF16>(mask, index)
-                                        : load1<kBF16>(mask, index);
-      if (__builtin_isfinite(raw)) value = raw * 1.44269504088896340736f;
-    }
-  }
-  bias[(static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y) * padded + key] = value;
+void launch_key_mask_kernel(const KeyMaskArgs& a, int dtype, hipStream_t stream) {
+  const int rows = a.tiles != nullptr ? a.batch * a.heads : 0;
+  const int blocks = rows + (a.bias != nullptr ? a.bias_planes * ((a.padded + 255) / 256) : 0);
+  const size_t flags = rows != 0 ? (a.length + 63) / 64 : 0;
+  if (dtype == kBool)
+    key_mask_kernel<kBool><<<blocks, 256, flags, stream>>>(a);
+  else if (dtype == kF32)
+    key_mask_kernel<kF32><<<blocks, 256, flags, stream>>>(a);
+  else if (dtype == kF16)
+    key_mask_kernel<kF16><<<blocks, 256, flags, stream>>>(a);
+  else
+    key_mask_kernel<kBF16><<<blocks, 256, flags, stream>>>(a);
 }
-
 
 // Lane words of a boolean mask (the form kMaskLanes of the attention kernel reads): for
 // every block of 32 queries and 64-key tile, 32 words; bit l of word 16*rb + i is the mask
@@ -427,9 +451,17 @@ int launch_mask_lanes(const void* mask, uint64_t* lanes, int batch, int heads, i
 int launch_key_bias(const void* mask, float* bias, int batch, int heads, int length, int padded,
                     int64_t stride_b, int64_t stride_h, int64_t stride_k, int dtype,
                     hipStream_t stream) {
-  const dim3 grid((padded + 255) / 256, heads, batch);
-  key_bias_kernel<<<grid, 256, 0, stream>>>(mask, bias, length, padded, stride_b, stride_h, stride_k,
-                                            dtype);
+  KeyMaskArgs a{};
+  a.mask = mask;
+  a.bias = bias;
+  a.bias_heads = heads;
+  a.bias_planes = batch * heads;
+  a.length = length;
+  a.padded = padded;
+  a.stride_k = stride_k;
+  a.bias_stride_b = stride_b;
+  a.bias_stride_h = stride_h;
+  launch_key_mask_kernel(a, dtype, stream);
   return check_launch("risa_prepare_key_bias");
 }
 
@@ -460,11 +492,41 @@ int launch_select_retained_mass(const SelectArgs& a, hipStream_t stream) {
 int launch_key_mask_tiles(const void* mask, int32_t* tiles, int batch, int heads, int length,
                           int tile_size, int64_t stride_b, int64_t stride_h, int64_t stride_k,
                           int dtype, hipStream_t stream) {
-  const int count = (length + tile_size - 1) / tile_size;
-  const dim3 grid(batch, heads);
-  key_mask_tiles_kernel<<<grid, 256, count * sizeof(int), stream>>>(
-      mask, tiles, heads, length, tile_size, stride_b, stride_h, stride_k, dtype);
+  KeyMaskArgs a{};
+  a.mask = mask;
+  a.tiles = tiles;
+  a.batch = batch;
+  a.heads = heads;
+  a.length = length;
+  a.tile_size = tile_size;
+  a.stride_b = stride_b;
+  a.stride_h = stride_h;
+  a.stride_k = stride_k;
+  launch_key_mask_kernel(a, dtype, stream);
   return check_launch("risa_prepare_key_mask_tiles");
+}
+
+int launch_key_mask(const void* mask, int32_t* tiles, float* bias, int batch, int heads, int mask_batch,
+                    int mask_heads, int length, int padded, int tile_size, int64_t stride_b,
+                    int64_t stride_h, int64_t stride_k, int dtype, hipStream_t stream) {
+  KeyMaskArgs a{};
+  a.mask = mask;
+  a.tiles = tiles;
+  a.bias = bias;
+  a.batch = batch;
+  a.heads = heads;
+  a.bias_heads = mask_heads;
+  a.bias_planes = mask_batch * mask_heads;
+  a.length = length;
+  a.tile_size = tile_size;
+  a.padded = padded;
+  a.stride_b = stride_b;
+  a.stride_h = stride_h;
+  a.stride_k = stride_k;
+  a.bias_stride_b = mask_batch > 1 ? stride_b : 0;
+  a.bias_stride_h = mask_heads > 1 ? stride_h : 0;
+  launch_key_mask_kernel(a, dtype, stream);
+  return check_launch("risa_sdpa key mask");
 }
 
 }  // namespace risa
