@@ -37,6 +37,7 @@ LOG2E = "0x3fb8aa3b"
 ROW_FLOOR = "0xc7435000"      # -50000
 MINUS_U8_OFFSET = "0xc0ffd1be"  # -7.9943534
 NEG_INF = "0xff800000"
+POS_INF = "0x7f800000"
 
 
 class Program:
@@ -293,18 +294,7 @@ def tile_body(e, p, stage, prio, label):
     scores = [p.S[rb] + i for rb in range(p.rb) for i in range(16)]
     scale_of = lambda i: p.sc1 if i & 2 else p.sc0
     if p.mask == "f32":
-        # mask terms in the exp2 domain, hidden keys (and terms that are no number) as -inf: a scaled
-        # score plus -inf is the -inf the compiled loop selects.  Beside the score products.
         e.valu(f"v_mov_b32_e32 v{p.tscale}, {LOG2E}", [p.tscale])
-        e.valu(f"v_mov_b32_e32 v{p.rowsum}, {NEG_INF}", [p.rowsum])
-        for group in range(8):
-            terms = [p.M + group * 4 + r for r in range(4)]
-            for r, term in enumerate(terms):
-                e.ins(f"v_cmp_class_f32_e64 {pair(p.pairs[r])}, v{term}, s{p.klass}")
-            for r, term in enumerate(terms):
-                e.valu(f"v_cndmask_b32_e64 v{term}, v{p.rowsum}, v{term}, {pair(p.pairs[r])}", [term])
-            for term in terms:
-                e.valu(f"v_mul_f32_e32 v{term}, v{term}, v{p.tscale}", [term])
     if not p.scaled:
         # ---- maxima of the seeded integer scores ---------------------------------------------------
         for rb in range(p.rb):
@@ -343,8 +333,15 @@ def tile_body(e, p, stage, prio, label):
             for i, register in enumerate(block):
                 e.valu(f"v_mul_f32_e32 v{register}, v{register}, v{scale_of(i)}", [register])
             if p.mask == "f32":
-                for i, register in enumerate(block):
-                    e.valu(f"v_add_f32_e32 v{register}, v{register}, v{p.M + rb * 16 + i}", [register])
+                # A term of -inf leaves -inf, one that is no number a score the maximum does not see
+                # and whose probability is zero: both as if the key were hidden.  Terms of +inf hide
+                # their keys too; they show in the maximum below.
+                for first in range(0, 16, 4):
+                    for r in range(4):
+                        e.valu(f"v_mul_f32_e32 v{p.T[r]}, v{p.M + rb * 16 + first + r}, v{p.tscale}", [p.T[r]])
+                    for r in range(4):
+                        register = block[first + r]
+                        e.valu(f"v_add_f32_e32 v{register}, v{register}, v{p.T[r]}", [register])
             if p.mask == "lanes":
                 if rb == 1:
                     e.ins("s_waitcnt lgkmcnt(0)")
@@ -368,13 +365,29 @@ def tile_body(e, p, stage, prio, label):
                     register = p.S[rb] + i
                     e.valu(f"v_add_f32_e32 v{register}, v{register}, v{terms + i}", [register])
             e.raw(f"{label}_zerorow:")
-        e.valu(f"v_mov_b32_e32 v{p.mx0}, {ROW_FLOOR}", [p.mx0])
-        e.valu(f"v_max_f32_e32 v{p.mx1}, v{scores[0]}, v{scores[1]}", [p.mx1])
-        targets = [p.mx0, p.mx1]
-        for index, at in enumerate(range(2, len(scores), 2)):
-            target = targets[index & 1]
-            e.valu(f"v_max3_f32 v{target}, v{target}, v{scores[at]}, v{scores[at + 1]}", [target])
-        e.valu(f"v_max_f32_e32 v{p.mx0}, v{p.mx0}, v{p.mx1}", [p.mx0])
+        def row_maximum():
+            e.valu(f"v_mov_b32_e32 v{p.mx0}, {ROW_FLOOR}", [p.mx0])
+            e.valu(f"v_max_f32_e32 v{p.mx1}, v{scores[0]}, v{scores[1]}", [p.mx1])
+            for index, at in enumerate(range(2, len(scores), 2)):
+                target = p.mx1 if index & 1 else p.mx0
+                e.valu(f"v_max3_f32 v{target}, v{target}, v{scores[at]}, v{scores[at + 1]}", [target])
+            e.valu(f"v_max_f32_e32 v{p.mx0}, v{p.mx0}, v{p.mx1}", [p.mx0])
+
+        row_maximum()
+        if p.mask == "f32":
+            # some score is +inf: take the keys out whose term is no finite number
+            e.valu(f"v_cmp_eq_f32_e32 vcc, {POS_INF}, v{p.mx0}")
+            e.nop(4)
+            e.ins(f"s_cbranch_vccz {label}_finite")
+            e.valu(f"v_mov_b32_e32 v{p.rowsum}, {NEG_INF}", [p.rowsum])
+            for group in range(8):
+                for r in range(4):
+                    e.ins(f"v_cmp_class_f32_e64 {pair(p.pairs[r])}, v{p.M + group * 4 + r}, s{p.klass}")
+                for r in range(4):
+                    register = scores[group * 4 + r]
+                    e.valu(f"v_cndmask_b32_e64 v{register}, v{p.rowsum}, v{register}, {pair(p.pairs[r])}", [register])
+            row_maximum()
+            e.raw(f"{label}_finite:")
         e.valu(f"v_add_f32_e32 v{p.mx0}, {MINUS_U8_OFFSET}, v{p.mx0}", [p.mx0])
     e.valu(f"v_mov_b32_e32 v{p.mx1}, v{p.mx0}", [p.mx1])
     e.nop(2)
