@@ -82,6 +82,9 @@ int launch_quantize_qk(const QkArgs& a, hipStream_t stream) {
 // grid (ceil(Lq/8), Hq, B), 256 threads: one 32-lane half per query row.
 // ---------------------------------------------------------------------------
 namespace {
+// Eight rows per half wavefront, loads of all of them in flight (one row per half, each channel
+// waited for, took 17 us for 48 heads x 4096 x 64 in 16 bits: 2.9 TB/s).
+constexpr int kShiftRows = 8;
 template <int DT>
 __global__ __launch_bounds__(256) void lse_shift_kernel(const void* __restrict__ q,
                                                         const void* __restrict__ k,
@@ -92,27 +95,43 @@ __global__ __launch_bounds__(256) void lse_shift_kernel(const void* __restrict__
                                                         int64_t kb, int64_t kh, int64_t kn,
                                                         float scale) {
   const int sub = threadIdx.x & 31;
-  const int row = blockIdx.x * 8 + (threadIdx.x >> 5);
+  const int first_row = (blockIdx.x * 8 + (threadIdx.x >> 5)) * kShiftRows;
   const int head = blockIdx.y, batch = blockIdx.z;
-  if (row >= q_len) return;
+  if (first_row >= q_len) return;
   const int kv_head = head / (q_heads / kv_heads);
   const int anchor = anchors[batch * kv_heads + kv_head];
-  float sum = 0.0f;
+  float sum[kShiftRows];
+#pragma unroll
+  for (int i = 0; i < kShiftRows; ++i) sum[i] = 0.0f;
   if (anchor >= 0) {
-    const int64_t q_base = batch * qb + head * qh + static_cast<int64_t>(row) * qn;
+    const int64_t q_base = batch * qb + head * qh;
     const int64_t k_base = batch * kb + kv_head * kh + static_cast<int64_t>(anchor) * kn;
+#pragma unroll 2
     for (int d = sub; d < dim; d += 32) {
-      const float product = load1<DT>(q, q_base + d) * load1<DT>(k, k_base + d);
-      sum = sum + product;
+      const float key = load1<DT>(k, k_base + d);
+      float query[kShiftRows];
+#pragma unroll
+      for (int i = 0; i < kShiftRows; ++i)  // (rows past the end read the last one)
+        query[i] = load1<DT>(q, q_base + static_cast<int64_t>(min(first_row + i, q_len - 1)) * qn + d);
+#pragma unroll
+      for (int i = 0; i < kShiftRows; ++i) {
+        const float product = query[i] * key;
+        sum[i] = sum[i] + product;
+      }
     }
-    sum = segment_down_sum(sum);
+#pragma unroll
+    for (int i = 0; i < kShiftRows; ++i) sum[i] = segment_down_sum(sum[i]);
   }
-  if (sub == 0) out[(static_cast<int64_t>(batch) * q_heads + head) * q_len + row] = sum * scale;
+  float mine = sum[0];
+#pragma unroll
+  for (int i = 1; i < kShiftRows; ++i) mine = sub == i ? sum[i] : mine;
+  if (sub < kShiftRows && first_row + sub < q_len)
+    out[(static_cast<int64_t>(batch) * q_heads + head) * q_len + first_row + sub] = mine * scale;
 }
 }  // namespace
 
 int launch_lse_shift(const LseShiftArgs& a, hipStream_t stream) {
-  dim3 grid((a.q_len + 7) / 8, a.q_heads, a.batch);
+  dim3 grid((a.q_len + 8 * kShiftRows - 1) / (8 * kShiftRows), a.q_heads, a.batch);
 #define RISA_LSE(DTV)                                                                             \
   lse_shift_kernel<DTV><<<grid, 256, 0, stream>>>(a.q, a.k, a.anchors, a.out, a.q_heads,           \
                                                   a.kv_heads, a.q_len, a.head_dim, a.q_stride_b,   \
