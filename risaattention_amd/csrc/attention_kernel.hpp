@@ -178,9 +178,17 @@ constexpr int staged_mask_bytes(int mask_dtype, int mask_mode, int cta_k, bool s
              ? kQueryBlock * cta_k * mask_element_bytes(mask_dtype)
              : 0;
 }
+// Behind the tiles: V scale and centre of every channel, copied with the first tile.  The epilogue
+// is the end of a chain nothing overlaps when a compute unit's two workgroups are short (eight
+// 64-key tiles: 16 us), and a round trip to L2 for them stood in it.
 template <int D, int CTA_K, int MASK_DT, int MASK_MODE>
-using AttentionTileShape = TileShape<D, CTA_K, staged_mask_bytes(MASK_DT, MASK_MODE, CTA_K, false),
-                                     staged_mask_bytes(MASK_DT, MASK_MODE, CTA_K, true)>;
+struct AttentionTileShape : TileShape<D, CTA_K, staged_mask_bytes(MASK_DT, MASK_MODE, CTA_K, false),
+                                      staged_mask_bytes(MASK_DT, MASK_MODE, CTA_K, true)> {
+  using Tiles = TileShape<D, CTA_K, staged_mask_bytes(MASK_DT, MASK_MODE, CTA_K, false),
+                          staged_mask_bytes(MASK_DT, MASK_MODE, CTA_K, true)>;
+  static constexpr int kChannelOffset = Tiles::kLdsBytes > 256 * D ? Tiles::kLdsBytes : 256 * D;  // (the output rows)
+  static constexpr int kLdsBytes = kChannelOffset + 2 * D * 4;
+};
 
 // Launches with a tile loop of gen_tile_loops.py: the unmasked and causal ones, key-only masks, lane
 // words and staged float masks, each where the compiled loop was measured slower.  Whole calls,
@@ -450,6 +458,11 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
       }
     }
   };
+
+  if (wave >= 2 && lane < D / 4) {  // V scale by the third wavefront, centre by the fourth
+    copy16_to_lds_uniform(reinterpret_cast<const int8_t*>((wave == 2 ? p.v_scale : p.v_center) + bhk * D),
+                          static_cast<uint32_t>(lane) * 16, lds + Shape::kChannelOffset + (wave - 2) * (D * 4));
+  }
 
   float o_acc[CB][16];
 #pragma unroll
@@ -1309,6 +1322,7 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
   // listed tile per query block: 155 of 264 us).  The rows go through LDS instead (every
   // wavefront has left the tiles by then; 64 * D bytes per wavefront) and leave as whole
   // rows, 16 bytes per lane.
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // (without a listed tile nothing has waited for the channel parameters)
   __syncthreads();  // no wavefront reads a tile any more
   constexpr int ROW_BYTES = D * 2;
   constexpr int CHUNKS = ROW_BYTES / 16;  // 16-byte pieces of a row
@@ -1329,8 +1343,8 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
 #pragma unroll
     for (int b4 = 0; b4 < 4; ++b4) {
       const int c = cb * 32 + b4 * 8 + half * 4;
-      const v4f scale4 = *reinterpret_cast<const v4f*>(p.v_scale + bhk * D + c);
-      const v4f center4 = *reinterpret_cast<const v4f*>(p.v_center + bhk * D + c);
+      const v4f scale4 = *reinterpret_cast<const v4f*>(lds + Shape::kChannelOffset + c * 4);
+      const v4f center4 = *reinterpret_cast<const v4f*>(lds + Shape::kChannelOffset + D * 4 + c * 4);
       float value[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
