@@ -215,6 +215,15 @@ constexpr int attention_workgroups(int d, int cta_k, bool fast, bool indexed, bo
   return d == 64 && mask_mode == kMaskLanes ? 4 : 2;
 }
 
+// Where a hand-scheduled loop starts.  Most of its 8-byte vector instructions then sit on 8-byte
+// boundaries or between them, and the loops of 128-key raw scores feel it: 16 heads x 32768 at words
+// 0..7 of a 32-byte block 5228 5194 5233 5190 5222 5183 5222 5185 us (dense, odd words better),
+// reuse 2613 2641 2620 2632 2614 2628 2615 2641 and construction at 16384 1486 1492 1489 1500 1485
+// 1497 1484 1490 us (even words better); the others are within 0.3 %.  Left to the compiler's code
+// in front of it, the start moves with every change there.
+#define RISA_LOOP_AT_EVEN_WORD ".p2align 3\n\t"
+#define RISA_LOOP_AT_ODD_WORD ".p2align 3\n\ts_nop 0\n\t"
+
 // MASK_DT: element type of the mask tensor (risa::kBool, kF32, kF16, kBF16), kKeyBias
 // for a key-only mask prepared as an FP32 row, or -1 for none; FAST (raw-score path)
 // implies -1.  MASK_MODE: kMaskScalar / kMaskVector / kMaskStaged; a template parameter
@@ -1069,7 +1078,7 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
       const int count = walk;
       if constexpr (INDEXED) {
         const uint64_t list = reinterpret_cast<uint64_t>(indices);
-        asm volatile(
+        asm volatile(RISA_LOOP_AT_EVEN_WORD
 #include "sparse_loop_d128.inc"
             : "+{v[128:143]}"(out0), "+{v[144:159]}"(out1), "+{v[160:175]}"(out2), "+{v[176:191]}"(out3),
               "+{v241}"(m_run), "+{v242}"(d_part)
@@ -1087,7 +1096,7 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
             stats + (bhq * static_cast<uint64_t>(p.n_kb - 1) * p.q_len + (bx * kQueryBlock + wave * 32)) * 2);
         const uint32_t tile_bytes = static_cast<uint32_t>(p.q_len) * 8u;
         const uint64_t storing = __builtin_amdgcn_ballot_w64(half == 0 && query_ok);
-        asm volatile(
+        asm volatile(RISA_LOOP_AT_EVEN_WORD
 #include "capture_loop_d128.inc"
             : "+{v[128:143]}"(out0), "+{v[144:159]}"(out1), "+{v[160:175]}"(out2), "+{v[176:191]}"(out3),
               "+{v241}"(m_run), "+{v242}"(d_part)
@@ -1101,7 +1110,7 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
 #include "capture_loop_d128_clobbers.inc"
         );
       } else {
-        asm volatile(
+        asm volatile(RISA_LOOP_AT_ODD_WORD
 #include "dense_loop_d128.inc"
             : "+{v[128:143]}"(out0), "+{v[144:159]}"(out1), "+{v[160:175]}"(out2), "+{v[176:191]}"(out3),
               "+{v241}"(m_run), "+{v242}"(d_part)

@@ -606,7 +606,7 @@ def render(p, prio=(0, 1, 2, 0)):
     """The asm statement as the include file holds it."""
     e = generate(p, prio)
     outputs, inputs, named = operands(p)
-    text = "asm volatile(\n" + "".join('"{}\\n\\t"\n'.format(line.replace('"', '\\"')) for line in e.lines)
+    text = "asm volatile(RISA_LOOP_AT_EVEN_WORD\n" + "".join('"{}\\n\\t"\n'.format(line.replace('"', '\\"')) for line in e.lines)
     text += "    : " + ", ".join(f'"+{c}"({x})' for c, x in outputs) + "\n"
     text += "    : " + ", ".join(f'"{c}"({x})' for c, x in inputs) + ",\n"
     text += "      " + ", ".join(f'[{n}] "s"({x})' for n, x in named) + "\n"
