@@ -192,6 +192,21 @@ int risa_attention(const void* q_int8, const void* k_int8, const void* v_int8, v
                    const float* key_bias, int64_t key_bias_stride_b, int64_t key_bias_stride_h,
                    const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
                    int64_t mask_lanes_stride_h, void* stream);
+/* The same, told that k_bytes bytes can be read from k_int8 on.  With cta_k * head_dim of them behind
+ * the last key the kernels copy a last key tile of fewer keys whole (what lies there has no influence
+ * on the result); risa_attention assumes that nothing behind the keys can be read. */
+int risa_attention_readable_keys(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
+                   const float* q_scale, const float* k_scale, const float* v_scale,
+                   const float* v_center, const int32_t* v_tile_sum, const void* mask,
+                   int64_t mask_stride_b, int64_t mask_stride_h, int64_t mask_stride_q,
+                   int64_t mask_stride_k, int mask_dtype, int cta_k, int batch, int q_len,
+                   int k_len, int q_heads, int kv_heads, int head_dim, int64_t out_stride_b,
+                   int64_t out_stride_n, int64_t out_stride_h, float sm_scale, int out_dtype,
+                   const int32_t* sparse_row_offsets, const int32_t* sparse_block_indices,
+                   float* block_mass, int is_causal, float* lse, const int32_t* key_mask_tiles,
+                   const float* key_bias, int64_t key_bias_stride_b, int64_t key_bias_stride_h,
+                   const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
+                   int64_t mask_lanes_stride_h, int64_t k_bytes, void* stream);
 
 /*
  * Quantise and attend in one call.  Replaces risa_sdpa (reference

@@ -25,7 +25,7 @@ from .policy import (
     select_key_block_size,
     validate_inputs,
 )
-from .prepare import pad_head_dim, resolve_scale, rows_hold_whole_runs
+from .prepare import KEYS_WITH_ROOM, pad_head_dim, resolve_scale, rows_hold_whole_runs
 from .types import PrequantizedInt8Attention, RetainedMassPattern
 
 
@@ -149,18 +149,21 @@ def launch_attention(*, q_codes, k_codes, v_codes, output, q_scale, k_scale, v_s
     bias_args = (None, 0, 0) if key_bias is None else (key_bias[0].data_ptr(), key_bias[1], key_bias[2])
     mask_lanes = prepare_mask_lanes(attn_mask, cta_k, dim)
     lane_args = (None, 0, 0) if mask_lanes is None else (mask_lanes[0].data_ptr(), mask_lanes[1], mask_lanes[2])
+    # (a last tile of fewer keys is copied whole where the storage goes on behind the keys)
+    whole = padded == k_len or k_len < KEYS_WITH_ROOM
+    readable_keys = 0 if whole else k_codes.untyped_storage().nbytes() - k_codes.storage_offset()
     out_b = output.stride(0) if batch > 1 else q_heads * q_len * dim
     out_n = output.stride(2) if q_len > 1 else dim
     out_h = output.stride(1) if q_heads > 1 else q_len * dim
     native.check(
-        native.library().risa_attention(
+        native.library().risa_attention_readable_keys(
             q_codes.data_ptr(), k_codes.data_ptr(), v_codes.data_ptr(), output.data_ptr(),
             q_scale.data_ptr(), k_scale.data_ptr(), v_scale.data_ptr(), v_center.data_ptr(),
             sums.data_ptr(), *mask_args, cta_k, batch, q_len, k_len, q_heads, kv_heads, dim,
             out_b, out_n, out_h, float(sm_scale), DTYPE_CODES[output.dtype],
             native.pointer(row_offsets), native.pointer(block_indices), native.pointer(block_mass),
             int(bool(is_causal)), native.pointer(lse), native.pointer(key_mask_tiles),
-            *bias_args, *lane_args, native.current_stream(q_codes.device),
+            *bias_args, *lane_args, readable_keys, native.current_stream(q_codes.device),
         )
     )
 

@@ -181,6 +181,7 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
   p.workspace = a.block_mass;
   p.lse = a.lse;
   p.causal = a.is_causal ? 1 : 0;
+  p.whole_key_tiles = a.whole_key_tiles ? 1 : 0;
   // Diagnostic switch, read at every launch: RISA_COMPILED_LOOP=1 sends the raw-score kernels of
   // head dim 128 through the tile loop the compiler schedules instead of the hand-scheduled one
   // (same results bit for bit; the tests compare the two).

@@ -81,6 +81,7 @@ struct KernelParams {
   float* workspace;  // capture
   float* lse;
   int causal;
+  int whole_key_tiles;  // the last key tile can be copied whole although fewer keys are left
   int compiled_loop;  // non-zero: every tile through the loop the compiler schedules (see RISA_COMPILED_LOOP)
 };
 
@@ -1043,12 +1044,13 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
   int first_tile = 0;
   // Listed tiles a hand-scheduled loop walks.  It copies whole tiles without looking at the key
   // range, the one behind its last included, so a last tile of fewer keys leaves two to the loop
-  // below; under the causal rule only tiles below the diagonal are its own.
+  // below where nothing is known about the memory behind the keys (1045 tokens, 32 heads: 48
+  // against 45 us); under the causal rule only tiles below the diagonal are its own.
   [[maybe_unused]] int walk = 0;
   if constexpr (ASM_LOOP || TILE_LOOP) {
     if (n_it > 1 && !p.compiled_loop) {
       walk = n_it - 1;
-      if (p.k_len % CTA_K != 0 && (tile_at(n_it - 1) + 1) * CTA_K > p.k_len) --walk;
+      if (!p.whole_key_tiles && p.k_len % CTA_K != 0 && (tile_at(n_it - 1) + 1) * CTA_K > p.k_len) --walk;
       if (!FAST && p.causal) walk = INDEXED ? 0 : min(walk, bx * (kQueryBlock / CTA_K));
       // the loop's mask copies take every row of the query block
       if (F32_MASK_LOOP && (bx + 1) * kQueryBlock > p.q_len) walk = 0;

@@ -78,6 +78,7 @@ struct AttentionArgs {
   const int32_t* sparse_block_indices;
   float* block_mass;
   bool is_causal;
+  bool whole_key_tiles;  // cta_k rows behind the last key can be read (their contents do not matter)
   float* lse;
   const int32_t* key_mask_tiles;
   const float* key_bias;  // [Bm,Hm,padded] from launch_key_bias, or null

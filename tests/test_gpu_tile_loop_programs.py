@@ -89,3 +89,19 @@ def test_key_masks(risa, dim, kind, k_len):
             mask[..., ::97] = -math.inf
     both(risa, q, k, v, attn_mask=mask)
     both(risa, q, k, v, attn_mask=mask.expand(2, 20, 1, k_len).contiguous(), is_causal=k_len <= 1100)
+
+
+@pytest.mark.parametrize("k_len", [2049, 2300, 4223])
+def test_key_codes_without_room_behind_them(risa, k_len):
+    """Packed keys in storage of their own size (a saved or copied container): the last tile of fewer
+    keys is then copied key by key; the results are those of the container with room behind."""
+    import dataclasses
+
+    q, k, v = inputs(1, 40, 4, 1045, k_len, 128)
+    packed = risa.prequantize_int8_attention(q, k, v, return_lse=True)
+    assert packed.k.is_contiguous() and packed.k.untyped_storage().nbytes() >= packed.k.numel() + packed.cta_k * 128
+    exact = dataclasses.replace(packed, k=packed.k.clone())
+    assert exact.k.untyped_storage().nbytes() < packed.k.untyped_storage().nbytes()
+    for a, b in zip(risa.int8_attention_from_prequantized(packed, return_lse=True),
+                    risa.int8_attention_from_prequantized(exact, return_lse=True)):
+        assert torch.equal(a, b)
