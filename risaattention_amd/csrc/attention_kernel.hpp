@@ -193,8 +193,8 @@ struct AttentionTileShape : TileShape<D, CTA_K, staged_mask_bytes(MASK_DT, MASK_
 
 // Launches with a tile loop of gen_tile_loops.py: the unmasked and causal ones, key-only masks, lane
 // words and staged float masks, each where the compiled loop was measured slower.  Whole calls,
-// 2 x 24 heads x 4096 x 4608, head dim 64: key padding (335 -> 290 vector instructions on a
-// wavefront's tile) 305 -> 266 us, boolean mask with log-normalisers (380 -> 320) 388 -> 319 us.
+// 2 x 24 heads x 4096 x 4608, head dim 64: key padding (335 -> 304 vector instructions on a
+// wavefront's tile) 305 -> 266 us, boolean mask with log-normalisers (380 -> 333) 388 -> 319 us.
 // The whole-list walk of a boolean mask takes the listed loop too: its lists name every tile they
 // walk.  Masks read per score or staged in 8 or 16 bits, sparse walks of short key ranges and
 // pattern construction behind a mask keep the compiled loop.
@@ -1034,11 +1034,11 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
   // stay below.
   constexpr bool ASM_LOOP = FAST && D == 128 && CTA_K == 128;
   // Other launches have loops of the same kind, written by gen_tile_loops.py.  All are bound by
-  // vector issue; the loop the compiler schedules spends 706 (causal, 128-key tile), 330 (raw, 64)
-  // and 669 (float mask, 64) vector instructions on a wavefront's tile, these 620, 300 and 510.
-  // Whole calls, compiled loop -> this one, same machine: causal 32/8 heads x 8192 462 -> 410 us;
-  // 40 heads x 32760 queries x 512 keys 487 -> 469 us; float mask 2 x 24 heads x 4096 x 4608,
-  // 661 -> 556 us.
+  // vector issue; per wavefront and tile, prologue and epilogue included, the loop the compiler
+  // schedules issues 706 (causal, 128-key tile), 430 (raw, 64) and 669 (float mask, 64) vector
+  // instructions, these 613, 409 and 482 (SQ_INSTS_VALU).  Whole calls, compiled loop -> this one,
+  // same machine: causal 32/8 heads x 8192 462 -> 410 us; 40 heads x 32760 queries x 512 keys
+  // 487 -> 469 us; float mask 2 x 24 heads x 4096 x 4608, 661 -> 536 us.
   constexpr bool F32_MASK_LOOP = D == 128 && SHARED_MASK && !INDEXED && !CAPTURE;
   constexpr bool TILE_LOOP = has_tile_loop(D, CTA_K, FAST, INDEXED, CAPTURE, MASK_DT, MASK_MODE);
   int first_tile = 0;
