@@ -208,12 +208,18 @@ constexpr bool has_tile_loop(int d, int cta_k, bool fast, bool indexed, bool cap
 }
 
 // Workgroups per compute unit the registers have to leave room for.  Head dim 64: the tile loops
-// take up to 168 registers, three wavefronts per SIMD; lane words through the compiled loop keep
-// four at 128.
+// take up to 168 registers, three wavefronts per SIMD; with lane words four, at 128.  Their tile
+// lists can be short, and a launch of up to 1024 workgroups then runs in one round: attention kernel,
+// 32 heads x 4096 x 4096, in 155 registers and three per unit -> 128 and four (-> the loop the compiler
+// schedules, four): documents of 128 tokens 16.4 -> 14.5 (14.4) us, of 256 21.6 -> 18.5 (19.6), a window
+// of 256 26.7 -> 22.3 (24.8), no key hidden 173 -> 152 (176), but a lower triangle 83.7 -> 90.7 (116).
+// Where three already give one round: 24 heads, no key hidden, 111.5 -> 113.5 (143.9), documents of 128
+// tokens 11.9 -> 11.6 (11.7); where both give two: 48 x 4096, a window of 1024 63.0 -> 66.8 (78.5).
 constexpr int attention_workgroups(int d, int cta_k, bool fast, bool indexed, bool capture, int mask_dt, int mask_mode) {
   if (d == 256) return 1;
+  if (d == 64 && mask_mode == kMaskLanes) return 4;
   if (d == 64 && has_tile_loop(d, cta_k, fast, indexed, capture, mask_dt, mask_mode)) return 3;
-  return d == 64 && mask_mode == kMaskLanes ? 4 : 2;
+  return 2;
 }
 
 // Where a hand-scheduled loop starts.  Most of its 8-byte vector instructions then sit on 8-byte
@@ -1333,6 +1339,13 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
   // listed tile per query block: 155 of 264 us).  The rows go through LDS instead (every
   // wavefront has left the tiles by then; 64 * D bytes per wavefront) and leave as whole
   // rows, 16 bytes per lane.
+  if constexpr (TILE_LOOP && LANES && D == 64) {  // (128 registers: not kept over the loop above)
+    lane = fresh_lane();
+    l32 = lane & 31;
+    half = lane >> 5;
+    query = bx * kQueryBlock + wave * 32 + l32;
+    query_ok = query < p.q_len;
+  }
   __builtin_amdgcn_s_waitcnt(0x0f70);  // (without a listed tile nothing has waited for the channel parameters)
   __syncthreads();  // no wavefront reads a tile any more
   constexpr int ROW_BYTES = D * 2;

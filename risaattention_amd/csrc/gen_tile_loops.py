@@ -43,9 +43,15 @@ POS_INF = "0x7f800000"
 class Program:
     """Shape, registers and operands of one program."""
 
-    def __init__(self, name, dim, keys, scaled, mask=None, listed=False):
+    def __init__(self, name, dim, keys, scaled, mask=None, listed=False, tight=False):
+        """tight: within 128 registers, for four workgroups per compute unit.  Probabilities are formed
+        and packed over the scores, the score seeds stand in accumulator and V fragment registers (16
+        moves per tile; read from LDS instead, lists of two to four tiles are 2-4 % slower and long ones
+        1 % faster), and values whose uses do not overlap share registers."""
         self.name, self.dim, self.keys, self.scaled, self.mask, self.listed = name, dim, keys, scaled, mask, listed
+        self.tight = tight
         assert scaled or mask is None
+        assert not tight or (dim == 64 and mask == "lanes")
         self.kk, self.cb, self.rb = dim // 32, dim // 32, keys // 32
         self.tile_bytes = dim * keys
         self.seed_region = 2 * self.tile_bytes
@@ -61,22 +67,33 @@ class Program:
         self.S = [take(16) for _ in range(self.rb)]
         self.M = take(32) if mask == "f32" else None
         self.ACC = [take(16) for _ in range(self.cb)]
+        if tight:  # (right behind the accumulators, see SEEDS)
+            self.VF = [take(4) for _ in range(self.cb)]
         self.O = [take(16) for _ in range(self.cb)]
         self.Q = [take(4) for _ in range(self.kk)]
-        self.VF = [take(4) for _ in range(self.cb)]
-        self.PK = [take(4), take(4)]
+        if not tight:
+            self.VF = [take(4) for _ in range(self.cb)]
+        self.PK = list(self.S) if tight else [take(4), take(4)]
         # seed block of the score products: registers of its own where they are free (no moves), else
         # the V fragment registers, free in that phase
-        roomy = keys == 64 and mask != "f32"
-        self.SEEDS = take(16) if roomy else self.VF[0]
+        # (tight: K fragments fill the lower half of an accumulator; the upper half of the last one
+        # and the V fragments are sixteen free registers in a row)
+        roomy = keys == 64 and mask != "f32" and not tight
+        self.SEEDS = take(16) if roomy else self.ACC[-1] + 8 if tight else self.VF[0]
         self.seeds_kept = roomy
-        self.T = [take(1) for _ in range(4)]
-        self.sc0, self.sc1, self.mx0 = take(1), take(1), take(1)
+        self.T = None if tight else [take(1) for _ in range(4)]
+        self.sc0, self.sc1 = take(1), take(1)
+        self.mx0 = self.sc0 if tight else take(1)  # (the maxima follow the last use of the scales)
         self.negm = None if scaled else take(1)
         # free in the phases that use them
-        self.mx1, self.tmp, self.tmp2 = self.PK[1], self.PK[1] + 1, self.PK[1] + 2
+        if tight:
+            self.mx1 = self.tmp = self.sc1
+        else:
+            self.mx1, self.tmp = self.PK[1], self.PK[1] + 1
         self.tscale, self.mrun, self.dpart = take(1), take(1), take(1)
         self.rowsum, self.qscale, self.seedval = take(1), take(1), take(1)
+        self.upper0, self.upper1 = (self.rowsum, self.tscale) if tight else (self.tmp, self.PK[1] + 2)
+        self.lane16 = self.rowsum if tight else self.T[0]  # lane * 16, row copies
         self.ka = take(1) if mask == "f32" else None     # K fragment address of k-step 0; the others by xor
         self.KA = None if mask == "f32" else [take(1) for _ in range(self.kk)]
         if keys == dim and self.KA:
@@ -91,7 +108,8 @@ class Program:
         if mask == "f32":
             self.maddr, self.mch, self.mrow = take(1), take(1), take(1)
         assert self.next_vgpr <= 255, (name, self.next_vgpr)  # v255 is left to the compiler
-        assert dim == 128 or self.next_vgpr <= 167, (name, self.next_vgpr)  # three wavefronts per SIMD
+        # head dim 64: three wavefronts per SIMD, four of a tight program (and three registers for the compiler)
+        assert dim == 128 or self.next_vgpr <= (125 if tight else 167), (name, self.next_vgpr)
         self.next_sgpr = FIRST_SGPR
         stake = self.stake
         if mask == "lanes":
@@ -223,9 +241,9 @@ def tile_body(e, p, stage, prio, label):
             e.ins(f"s_mov_b64 exec, {hex((1 << lanes) - 1)}")
             e.ins(f"s_add_u32 m0, s{p.lds}, {other * p.stage + region}")
             e.ins("s_nop 0")
-            e.ins(f"v_mbcnt_lo_u32_b32 v{p.T[0]}, -1, 0")
-            e.ins(f"v_lshlrev_b32_e32 v{p.T[0]}, 4, v{p.T[0]}")
-            e.ins(f"global_load_lds_dwordx4 v{p.T[0]}, {pair(p.tmp_s)}")
+            e.ins(f"v_mbcnt_lo_u32_b32 v{p.lane16}, -1, 0")
+            e.ins(f"v_lshlrev_b32_e32 v{p.lane16}, 4, v{p.lane16}")
+            e.ins(f"global_load_lds_dwordx4 v{p.lane16}, {pair(p.tmp_s)}")
             e.ins("s_mov_b64 exec, -1")  # (every wavefront of the kernel runs with all its lanes)
             e.raw(f"{label}_{name}:")
         return emit
@@ -282,9 +300,9 @@ def tile_body(e, p, stage, prio, label):
 
     # ---- K scales of this tile (scalar registers) -> score scales of this lane's two key groups ----
     e.ins(f"s_setprio {prio[1]}")
-    for register, slot in ((p.tmp, 2), (p.tmp2, 3), (p.sc0, 0), (p.sc1, 1)):
+    for register, slot in ((p.upper0, 2), (p.upper1, 3), (p.sc0, 0), (p.sc1, 1)):
         e.valu(f"v_mov_b32_e32 v{register}, s{p.ks + slot}", [register])
-    for register, upper in ((p.sc0, p.tmp), (p.sc1, p.tmp2)):
+    for register, upper in ((p.sc0, p.upper0), (p.sc1, p.upper1)):
         e.valu(f"v_cndmask_b32_e64 v{register}, v{register}, v{upper}, {pair(p.halfmask)}", [register])
     for register in (p.sc0, p.sc1):
         e.valu(f"v_mul_f32_e32 v{register}, v{p.qscale}, v{register}", [register])
@@ -433,12 +451,14 @@ def tile_body(e, p, stage, prio, label):
     def pack_group(rb, b4, pk):
         """Four scores -> one register of signed probability bytes, and their sum."""
         registers = [p.S[rb] + b4 * 4 + r for r in range(4)]
+        # (tight: over scores of this group or of one already packed)
+        targets = registers if p.tight else p.T
         for r in range(4):
-            e.valu(f"v_exp_f32_e32 v{p.T[r]}, v{registers[r]}", [p.T[r]], trans=True)
+            e.valu(f"v_exp_f32_e32 v{targets[r]}, v{registers[r]}", [targets[r]], trans=True)
         for r in range(4):
-            e.need_trans(p.T[r])
+            e.need_trans(targets[r])
             previous = "0" if r == 0 else f"v{pk + b4}"
-            e.valu(f"v_cvt_pk_u8_f32 v{pk + b4}, v{p.T[r]}, {r}, {previous}", [pk + b4])
+            e.valu(f"v_cvt_pk_u8_f32 v{pk + b4}, v{targets[r]}, {r}, {previous}", [pk + b4])
         e.valu(f"v_sad_u8 v{p.rowsum}, v{pk + b4}, 0, v{p.rowsum}", [p.rowsum])
         e.valu(f"v_xor_b32_e32 v{pk + b4}, 0x80808080, v{pk + b4}", [pk + b4])
 
@@ -461,8 +481,9 @@ def tile_body(e, p, stage, prio, label):
             pack_group(rb, b4, current)
     for cb in range(p.cb):
         value_products(cb, p.PK[(p.rb - 1) & 1])
-    e.valu(f"v_cvt_f32_u32_e32 v{p.T[0]}, v{p.rowsum}", [p.T[0]])
-    e.valu(f"v_fmac_f32_e32 v{p.dpart}, v{p.T[0]}, v{p.tscale}", [p.dpart])
+    total = p.rowsum if p.tight else p.T[0]
+    e.valu(f"v_cvt_f32_u32_e32 v{total}, v{p.rowsum}", [total])
+    e.valu(f"v_fmac_f32_e32 v{p.dpart}, v{total}, v{p.tscale}", [p.dpart])
     # ---- scalar loads of the next tile: waited for at the next barrier ------------------------------
     if p.listed:
         e.ins(f"s_lshl_b32 s{p.tmp_s}, s{p.tnext}, 4")
@@ -485,10 +506,11 @@ def tile_body(e, p, stage, prio, label):
     for cb in range(p.cb):
         e.need_mfma_result(p.ACC[cb])
         for i in range(0, 16, 4):
+            targets = [p.ACC[cb] + i + j for j in range(4)] if p.tight else p.T
             for j in range(4):
-                e.valu(f"v_sub_f32_e32 v{p.T[j]}, v{p.ACC[cb] + i + j}, v{p.seedval}", [p.T[j]])
+                e.valu(f"v_sub_f32_e32 v{targets[j]}, v{p.ACC[cb] + i + j}, v{p.seedval}", [targets[j]])
             for j in range(4):
-                e.valu(f"v_fmac_f32_e32 v{p.O[cb] + i + j}, v{p.T[j]}, v{p.tscale}", [p.O[cb] + i + j])
+                e.valu(f"v_fmac_f32_e32 v{p.O[cb] + i + j}, v{targets[j]}, v{p.tscale}", [p.O[cb] + i + j])
 
 
 def generate(p, prio):
@@ -570,7 +592,7 @@ PROGRAMS = (
     Program("scaled_d64k64", 64, 64, scaled=True),
     Program("bias_d64k64", 64, 64, scaled=True, mask="bias"),
     Program("bias_listed_d64k64", 64, 64, scaled=True, mask="bias", listed=True),
-    Program("lanes_listed_d64k64", 64, 64, scaled=True, mask="lanes", listed=True),
+    Program("lanes_listed_d64k64", 64, 64, scaled=True, mask="lanes", listed=True, tight=True),
 )
 
 
