@@ -207,6 +207,10 @@ constexpr bool has_tile_loop(int d, int cta_k, bool fast, bool indexed, bool cap
   return d == 64 || (fast ? cta_k == 64 : cta_k == 128);
 }
 
+constexpr bool reads_float_mask_per_score(int d, bool indexed, bool capture, int mask_dt, int mask_mode) {
+  return d == 64 && !indexed && !capture && mask_mode == kMaskScalar && (mask_dt == kF32 || mask_dt == kF16 || mask_dt == kBF16);
+}
+
 // Workgroups per compute unit the registers have to leave room for.  Head dim 64: the tile loops
 // take up to 168 registers, three wavefronts per SIMD; with lane words four, at 128.  Their tile
 // lists can be short, and a launch of up to 1024 workgroups then runs in one round: attention kernel,
@@ -215,9 +219,12 @@ constexpr bool has_tile_loop(int d, int cta_k, bool fast, bool indexed, bool cap
 // of 256 26.7 -> 22.3 (24.8), no key hidden 173 -> 152 (176), but a lower triangle 83.7 -> 90.7 (116).
 // Where three already give one round: 24 heads, no key hidden, 111.5 -> 113.5 (143.9), documents of 128
 // tokens 11.9 -> 11.6 (11.7); where both give two: 48 x 4096, a window of 1024 63.0 -> 66.8 (78.5).
+// Float masks read per score stand at the edge of three: one register more, 169, cost 48 heads x 2048 x
+// 1001 149 -> 216 us (bfloat16) and 138 -> 176 us (fp32).  (The launcher takes two where three gain nothing.)
 constexpr int attention_workgroups(int d, int cta_k, bool fast, bool indexed, bool capture, int mask_dt, int mask_mode) {
   if (d == 256) return 1;
   if (d == 64 && mask_mode == kMaskLanes) return 4;
+  if (reads_float_mask_per_score(d, indexed, capture, mask_dt, mask_mode)) return 3;
   if (d == 64 && has_tile_loop(d, cta_k, fast, indexed, capture, mask_dt, mask_mode)) return 3;
   return 2;
 }

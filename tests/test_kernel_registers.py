@@ -63,3 +63,9 @@ def test_hand_scheduled_loops_of_head_dim_64_leave_room_for_three_workgroups(att
     for fast, indexed, mask in ((1, 0, -1), (0, 0, -1), (0, 0, KEY_BIAS), (0, 1, KEY_BIAS)):
         kernel = attention_kernels[64, 64, fast, indexed, 0, mask, SCALAR]
         assert workgroups(kernel) == 3 and kernel[".private_segment_fixed_size"] == 0, (fast, indexed, mask)
+
+
+def test_float_masks_read_per_score_leave_room_for_three_workgroups(attention_kernels):
+    for mask in FLOATS:
+        kernel = attention_kernels[64, 64, 0, 0, 0, mask, SCALAR]
+        assert workgroups(kernel) == 3 and kernel[".private_segment_fixed_size"] == 0, mask
