@@ -82,10 +82,11 @@ int launch_quantize_qk(const QkArgs& a, hipStream_t stream) {
 // grid (ceil(Lq/8), Hq, B), 256 threads: one 32-lane half per query row.
 // ---------------------------------------------------------------------------
 namespace {
-// Eight rows per half wavefront, loads of all of them in flight (one row per half, each channel
-// waited for, took 17 us for 48 heads x 4096 x 64 in 16 bits: 2.9 TB/s).
-constexpr int kShiftRows = 8;
-template <int DT>
+// kShiftRows rows per half wavefront, loads of all of them in flight: eight (one took 17 us for 48
+// heads x 4096 x 64 in 16 bits, 2.9 TB/s; eight take 5.3), but one for launches of up to four
+// workgroups per compute unit, where eight rows are a longer chain than one and leave wavefronts out
+// (16 heads x 64 x 128 3.3 us with eight, 2.5 with one; x 512 3.3 and 3.2; x 768 3.3 and 3.7).
+template <int DT, int kShiftRows>
 __global__ __launch_bounds__(256) void lse_shift_kernel(const void* __restrict__ q,
                                                         const void* __restrict__ k,
                                                         const int* __restrict__ anchors,
@@ -131,12 +132,13 @@ __global__ __launch_bounds__(256) void lse_shift_kernel(const void* __restrict__
 }  // namespace
 
 int launch_lse_shift(const LseShiftArgs& a, hipStream_t stream) {
-  dim3 grid((a.q_len + 8 * kShiftRows - 1) / (8 * kShiftRows), a.q_heads, a.batch);
+  const int64_t small = static_cast<int64_t>((a.q_len + 7) / 8) * a.q_heads * a.batch;
+  const int rows = small <= 4 * static_cast<int64_t>(narrow_attention_limit()) ? 1 : 8;
+  dim3 grid((a.q_len + 8 * rows - 1) / (8 * rows), a.q_heads, a.batch);
 #define RISA_LSE(DTV)                                                                             \
-  lse_shift_kernel<DTV><<<grid, 256, 0, stream>>>(a.q, a.k, a.anchors, a.out, a.q_heads,           \
-                                                  a.kv_heads, a.q_len, a.head_dim, a.q_stride_b,   \
-                                                  a.q_stride_h, a.q_stride_n, a.k_stride_b,        \
-                                                  a.k_stride_h, a.k_stride_n, a.scale)
+  (rows == 1 ? lse_shift_kernel<DTV, 1> : lse_shift_kernel<DTV, 8>)<<<grid, 256, 0, stream>>>(     \
+      a.q, a.k, a.anchors, a.out, a.q_heads, a.kv_heads, a.q_len, a.head_dim, a.q_stride_b,        \
+      a.q_stride_h, a.q_stride_n, a.k_stride_b, a.k_stride_h, a.k_stride_n, a.scale)
   if (a.dtype == kF32)
     RISA_LSE(kF32);
   else if (a.dtype == kF16)

@@ -149,6 +149,31 @@ def test_lse_shift_closed_form(risa, dtype, dim):
     assert torch.count_nonzero(out[0, :2]) == 0
 
 
+@pytest.mark.parametrize("dim", [64, 128, 256])
+def test_lse_shift_does_not_depend_on_the_rows_of_a_launch(risa, dim):
+    """Launches of more than four workgroups per compute unit take eight rows per half wavefront,
+    shorter ones (a head alone) one: the sums have one order, so the bits are the same."""
+    from risaattention_amd import native
+
+    q_len = 643  # ten times 64 rows and three
+    heads = 4 * torch.cuda.get_device_properties(0).multi_processor_count // -(-q_len // 8) + 1
+    q, k = seeded((1, heads, q_len, dim), torch.bfloat16, 1), seeded((1, heads, 5, dim), torch.bfloat16, 2)
+    anchors = torch.full((1, heads), 3, device="cuda", dtype=torch.int32)
+
+    def shift(q, k, anchors):
+        out = torch.empty(q.shape[:3], device="cuda")
+        native.check(
+            native.library().risa_lse_shift(
+                q.data_ptr(), k.data_ptr(), anchors.data_ptr(), out.data_ptr(), 1, q.shape[1], q.shape[1], q_len, dim,
+                *q.stride()[:3], *k.stride()[:3], 0.125, 2, torch.cuda.current_stream().cuda_stream,
+            )
+        )
+        return out
+
+    alone = [shift(q[:, h:h + 1], k[:, h:h + 1], anchors[:, h:h + 1]) for h in range(heads)]
+    assert torch.equal(shift(q, k, anchors), torch.cat(alone, 1))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("layout", ["hnd", "nhd", "interleaved"])
 @pytest.mark.parametrize("mode", ["absmax", "midpoint_affine"])
