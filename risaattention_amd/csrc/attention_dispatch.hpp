@@ -15,8 +15,8 @@ template <int D> int launch_attention_variant(const KernelParams& p, int cta_k, 
 // of them, else two, which LDS that nobody uses sees to (three times 64 KB exceed a unit's 160).  In
 // as many rounds, three at once only spread the reads of the mask: 64 heads x 2048 x 1001, fp32 190
 // us with two and 212 with three, bfloat16 222 and 276; 48 heads 176 and 139, 218 and 151.
-template <int D, bool INDEXED, bool CAPTURE, int MASK_DT, int MASK_MODE> size_t lds_that_keeps_a_third_out(const KernelParams& p) {
-  if constexpr (reads_float_mask_per_score(D, INDEXED, CAPTURE, MASK_DT, MASK_MODE)) {
+template <int D, bool CAPTURE, int MASK_DT, int MASK_MODE> size_t lds_that_keeps_a_third_out(const KernelParams& p) {
+  if constexpr (reads_float_mask_per_score(D, CAPTURE, MASK_DT, MASK_MODE)) {
     const int64_t units = narrow_attention_limit(), workgroups = static_cast<int64_t>(p.n_qb) * p.q_heads * p.batch;
     if ((workgroups + 3 * units - 1) / (3 * units) == (workgroups + 2 * units - 1) / (2 * units)) return 64 * 1024;
   }
@@ -43,7 +43,7 @@ int launch_one(const KernelParams& p, hipStream_t stream) {
   }
   const dim3 grid(static_cast<unsigned>(p.n_qb) * p.q_heads * p.batch);
   const size_t lds_bytes = std::max<size_t>(
-      Shape::kLdsBytes, lds_that_keeps_a_third_out<D, INDEXED, CAPTURE, MASK_DT, MASK_MODE>(p));
+      Shape::kLdsBytes, lds_that_keeps_a_third_out<D, CAPTURE, MASK_DT, MASK_MODE>(p));
   kernel<<<grid, 256, lds_bytes, stream>>>(p);
   return 0;
 }

@@ -67,5 +67,13 @@ def test_hand_scheduled_loops_of_head_dim_64_leave_room_for_three_workgroups(att
 
 def test_float_masks_read_per_score_leave_room_for_three_workgroups(attention_kernels):
     for mask in FLOATS:
-        kernel = attention_kernels[64, 64, 0, 0, 0, mask, SCALAR]
-        assert workgroups(kernel) == 3 and kernel[".private_segment_fixed_size"] == 0, mask
+        for indexed in (0, 1):
+            kernel = attention_kernels[64, 64, 0, indexed, 0, mask, SCALAR]
+            assert workgroups(kernel) == 3 and kernel[".private_segment_fixed_size"] == 0, (mask, indexed)
+
+
+def test_key_only_masks_spill_no_scalar_register(attention_kernels):
+    """Spilled around the hand-scheduled loop, sixteen of them cost launches of one or two key tiles 2-6 %."""
+    for shape in ((64, 64), (128, 128)):
+        for indexed in (0, 1):
+            assert attention_kernels[(*shape, 0, indexed, 0, KEY_BIAS, SCALAR)][".sgpr_spill_count"] == 0, (shape, indexed)
