@@ -116,8 +116,14 @@ def library_path() -> Path:
 
 def load_library(path: Path | str) -> ctypes.CDLL:
     """Another build of the C-ABI library (same entry points), with its signatures bound.
-    Raises OSError / AttributeError when the file cannot be loaded or lacks an entry point."""
+    Raises OSError / AttributeError when the file cannot be loaded or lacks an entry point (entry
+    points are added without a new ABI version, which counts changed signatures and layouts)."""
     loaded = ctypes.CDLL(str(path))
+    missing = [name for name in SIGNATURES if not hasattr(loaded, name)]
+    if missing:
+        version = loaded.risa_abi_version() if hasattr(loaded, "risa_abi_version") else "unknown"
+        raise AttributeError(f"{path} (ABI version {version}) lacks {', '.join(missing)}: "
+                             "it was built from other sources than this package, build it again")
     for name, (restype, argtypes) in SIGNATURES.items():
         function = getattr(loaded, name)
         function.restype = restype

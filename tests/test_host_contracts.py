@@ -3,6 +3,7 @@ operator registration (in the spirit of reference tests/contracts/test_risa_atte
 
 import ctypes
 import re
+import subprocess
 from pathlib import Path
 from unittest.mock import patch
 
@@ -483,6 +484,18 @@ def test_bench_profile_range_names():
     bench = _bench_module()
     assert bench.profile_range_names("dense", ("absmax", "midpoint_affine")) == ["risa/dense/absmax", "risa/dense/midpoint_affine"]
     assert bench.profile_range_names("attend", ("absmax",)) == ["risa/attend/absmax"]
+
+
+def test_library_of_older_sources_is_named_with_what_it_lacks(tmp_path):
+    """A library of this ABI version without the entry points added since: the error says which file,
+    which version and what is missing."""
+    source = tmp_path / "older.c"
+    entries = [name for name in native.SIGNATURES if not name.endswith("_channels")]
+    source.write_text("".join(f"int {name}(void) {{ return {3 * (name == 'risa_abi_version')}; }}\n" for name in entries))
+    library = tmp_path / "older.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", str(source), "-o", str(library)], check=True)
+    with pytest.raises(AttributeError, match=r"older\.so \(ABI version 3\) lacks .*risa_sdpa_channels"):
+        native.load_library(library)
 
 
 def test_library_swap_routes_calls_and_restores():
