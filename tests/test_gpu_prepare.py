@@ -28,6 +28,10 @@ CASES = [
     # long absmax self-attention shapes take at most 64 partial V ranges and no parameter launch
     (torch.bfloat16, 128, 5000, 5000, 2, 1, "absmax", 0.0),
     (torch.float16, 64, 9100, 9100, 1, 1, "absmax", 0.0),
+    # from half as much Q as V on; one with less keeps the parameter launch
+    (torch.bfloat16, 128, 3000, 5000, 1, 1, "absmax", 0.0),
+    (torch.bfloat16, 128, 2500, 5000, 1, 1, "absmax", 0.0),
+    (torch.bfloat16, 128, 2499, 5000, 1, 1, "absmax", 0.0),
 ]
 
 

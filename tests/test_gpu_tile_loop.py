@@ -151,7 +151,8 @@ def test_random_shapes_equal_the_compiled_loop(risa, seed):
     k = seeded((batch, kv_heads, k_len, 128), dtype, 3 * seed + 1, scale=1.0 + seed % 2)
     v = seeded((batch, kv_heads, k_len, 128), dtype, 3 * seed + 2, offset=0.1 * seed)
     packed = risa.prequantize_int8_attention(q, k, v, v_quantization=mode, return_lse=True)
-    # (the tile policy gives short key ranges 64-key tiles: those launches keep the compiled loop)
+    # (the tile policy gives short key ranges 64-key tiles: of those launches the dense one has a loop of
+    # gen_tile_loops.py, the others keep the compiled loop)
     tiles, query_blocks = -(-k_len // packed.cta_k), -(-q_len // 128)
     lists = [np.sort(rng.choice(tiles, size=int(rng.integers(1, tiles + 1)), replace=False))
              for _ in range(batch * q_heads * query_blocks)]
