@@ -32,7 +32,7 @@ extern "C" {
 /* Message of the last failed call on this host thread ("" if none). */
 const char* risa_last_error(void);
 
-/* Library/ABI version, bumped when a signature or a packed layout changes. */
+/* Library/ABI version, bumped when a signature or a packed layout changes (not when entry points are added). */
 int risa_abi_version(void);
 
 /*

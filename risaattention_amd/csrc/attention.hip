@@ -182,9 +182,9 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
   p.lse = a.lse;
   p.causal = a.is_causal ? 1 : 0;
   p.whole_key_tiles = a.whole_key_tiles ? 1 : 0;
-  // Diagnostic switch, read at every launch: RISA_COMPILED_LOOP=1 sends the raw-score kernels of
-  // head dim 128 through the tile loop the compiler schedules instead of the hand-scheduled one
-  // (same results bit for bit; the tests compare the two).
+  // Diagnostic switch, read at every launch: RISA_COMPILED_LOOP=1 sends every kernel that has a
+  // hand-scheduled tile loop through the loop the compiler schedules instead (same results bit for
+  // bit; the tests compare the two).
   const char* compiled_loop = std::getenv("RISA_COMPILED_LOOP");
   p.compiled_loop = compiled_loop != nullptr && compiled_loop[0] != '\0' && compiled_loop[0] != '0';
 

@@ -197,9 +197,18 @@ struct AttentionTileShape : TileShape<D, CTA_K, staged_mask_bytes(MASK_DT, MASK_
 };
 
 // Launches with a tile loop of gen_tile_loops.py: the unmasked and causal ones, key-only masks, lane
-// words and staged float masks, each where the compiled loop was measured slower.  Whole calls,
-// 2 x 24 heads x 4096 x 4608, head dim 64: key padding (335 -> 304 vector instructions on a
-// wavefront's tile) 305 -> 266 us, boolean mask with log-normalisers (380 -> 333) 388 -> 319 us.
+// words and staged float masks.  Attention kernel through the compiled loop -> the program, 24 to 64
+// heads x 2048 to 8192 queries, at few key tiles and at the most measured (two tiles are 0.99 to 1.04
+// times as fast, so the rule needs no length):
+//   head dim 128, raw 64-key tiles: 29.6 -> 28.2 us at 256 keys, 70.8 -> 64.8 at 1024;
+//     negative scale: 41.9 -> 37.6 at 1200, 130 -> 109 at 4608; causal 49.7 -> 42.3 at 2048, 432 -> 382
+//     at 8192; fp32 mask: 19.7 -> 17.8 at 256, 204 -> 136 at 4608; additive row, causal: 34.8 -> 29.0 at
+//     1200, 141 -> 119 at 4096, over lists: 39.7 -> 33.3 at 1100, 131 -> 102 at 4608; lane words: eight
+//     documents 55.8 -> 47.6 at 4096, no key hidden 1090 -> 890 at 8192.
+//   head dim 64, raw: 19.1 -> 18.6 at 256, 47.8 -> 45.2 at 1024; negative scale: 17.2 -> 15.4 at 512,
+//     106 -> 86 at 4608; causal 54.3 -> 50.0 at 2048, 613 -> 557 at 8192; additive row: 11.9 -> 11.2 at
+//     256, 30.3 -> 25.8 at 1024, over lists: 35.2 -> 28.3 at 1100, 121 -> 91 at 4608; lane words: eight
+//     documents 34.7 -> 30.3 at 4096, no key hidden 703 -> 607 at 8192.
 // The whole-list walk of a boolean mask takes the listed loop too: its lists name every tile they
 // walk.  Masks read per score or staged in 8 or 16 bits, sparse walks of short key ranges and
 // pattern construction behind a mask keep the compiled loop.
@@ -220,10 +229,10 @@ constexpr bool reads_float_mask_per_score(int d, bool capture, int mask_dt, int 
 // take up to 168 registers, three wavefronts per SIMD; with lane words four, at 128.  Their tile
 // lists can be short, and a launch of up to 1024 workgroups then runs in one round: attention kernel,
 // 32 heads x 4096 x 4096, in 155 registers and three per unit -> 128 and four (-> the loop the compiler
-// schedules, four): documents of 128 tokens 16.4 -> 14.5 (14.4) us, of 256 21.6 -> 18.5 (19.6), a window
-// of 256 26.7 -> 22.3 (24.8), no key hidden 173 -> 152 (176), but a lower triangle 83.7 -> 90.7 (116).
-// Where three already give one round: 24 heads, no key hidden, 111.5 -> 113.5 (143.9), documents of 128
-// tokens 11.9 -> 11.6 (11.7); where both give two: 48 x 4096, a window of 1024 63.0 -> 66.8 (78.5).
+// schedules, four): documents of 128 tokens 16.6 -> 14.2 (14.3) us, of 256 21.9 -> 18.9 (20.0), a window
+// of 256 26.8 -> 23.0 (25.3), no key hidden 180 -> 160 (183), but a lower triangle 90.4 -> 94.2 (118).
+// Where three already give one round: 24 heads, no key hidden, 119 -> 121 (149), documents of 128
+// tokens 11.9 -> 11.6 (11.7); where both give two: 48 x 4096, a window of 1024 66.0 -> 69.8 (81.7).
 // Float masks read per score stand at the edge of three: one register more, 169, cost 48 heads x 2048 x
 // 1001 149 -> 216 us (bfloat16) and 138 -> 176 us (fp32).  (The launcher takes two where three gain nothing.)
 constexpr int attention_workgroups(int d, int cta_k, bool fast, bool indexed, bool capture, int mask_dt, int mask_mode) {
@@ -374,9 +383,11 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
   // masked kernels have none to spare (a spilled offset would be reloaded through
   // the same counter the LDS copies complete on, serialising them) and recompute
   // them per tile from a lane id the compiler cannot see through.
-  // (The hand-scheduled tile loop issues its own copies and owns every vector register: kernels
-  // that have it issue at most two tiles from here, and offsets kept for them would live in
-  // scratch memory across the loop.)
+  // (The hand-scheduled loops issue their own copies, and kernels that have one at most two tiles
+  // from here.  That of 128-key raw scores owns every vector register: offsets kept for them would
+  // live in scratch memory across it.  The 64-key raw loops leave room, 244 registers and 159 in
+  // all, and offsets formed anew there gain nothing: 40 heads x 32760 x 512 341 -> 345 us, shorter
+  // launches within 1 %.)
   constexpr bool KEEP_OFFSETS = FAST && !(D == 128 && CTA_K == 128);
   auto k_source_offset = [&](int i, int lane_id) -> uint32_t {
     constexpr int CH = D / 16;
@@ -1051,19 +1062,18 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
   // the generator chose; the last listed tile (the one that may be partial) and the epilogue
   // stay below.
   constexpr bool ASM_LOOP = FAST && D == 128 && CTA_K == 128;
-  // Other launches have loops of the same kind, written by gen_tile_loops.py.  All are bound by
-  // vector issue; per wavefront and tile, prologue and epilogue included, the loop the compiler
-  // schedules issues 706 (causal, 128-key tile), 430 (raw, 64) and 669 (float mask, 64) vector
-  // instructions, these 613, 409 and 482 (SQ_INSTS_VALU).  Whole calls, compiled loop -> this one,
-  // same machine: causal 32/8 heads x 8192 462 -> 410 us; 40 heads x 32760 queries x 512 keys
-  // 487 -> 469 us; float mask 2 x 24 heads x 4096 x 4608, 661 -> 536 us.
+  // Other launches have loops of the same kind, written by gen_tile_loops.py (has_tile_loop holds
+  // what they measured).  Long walks are bound by vector issue (98 to 115 % of the cycles; 80 % in
+  // the raw loop over eight 64-key tiles, where prologue and epilogue weigh): per wavefront and
+  // tile, those included, the loop the compiler schedules issues 706 (causal, 128-key tile), 430
+  // (raw, 64) and 669 (float mask, 64) vector instructions, these 613, 409 and 482 (SQ_INSTS_VALU).
   constexpr bool F32_MASK_LOOP = D == 128 && SHARED_MASK && !INDEXED && !CAPTURE;
   constexpr bool TILE_LOOP = has_tile_loop(D, CTA_K, FAST, INDEXED, CAPTURE, MASK_DT, MASK_MODE);
   int first_tile = 0;
   // Listed tiles a hand-scheduled loop walks.  It copies whole tiles without looking at the key
   // range, the one behind its last included, so a last tile of fewer keys leaves two to the loop
-  // below where nothing is known about the memory behind the keys (1045 tokens, 32 heads: 48
-  // against 45 us); under the causal rule only tiles below the diagonal are its own.
+  // below where nothing is known about the memory behind the keys (1045 tokens, 32 heads: 27.5
+  // against 26.7 us); under the causal rule only tiles below the diagonal are its own.
   [[maybe_unused]] int walk = 0;
   if constexpr (ASM_LOOP || TILE_LOOP) {
     if (n_it > 1 && !p.compiled_loop) {

@@ -1,4 +1,5 @@
-// Q/K/V preparation in two launches (three beyond 4096 tokens, one up to 1024 tokens).
+// Q/K/V preparation in two launches (one up to 1024 tokens; three beyond 4096 for midpoint_affine, and
+// for absmax where Q holds less than half as much as V).
 //
 // The separate preparation kernels (prep_qk.hip, prep_v.hip) are five to seven
 // launches whose order is fixed by data: anchor -> K codes, V range -> V parameters
@@ -8,8 +9,9 @@
 // The work has only two levels of dependence, so two launches are enough:
 //   stage 1  K anchor | Q codes | V partial ranges      (independent workgroups)
 //   stage 2  K codes (needs the anchor) | V codes (reduce the partial ranges themselves)
-// With more than 64 partial ranges per channel (beyond 4096 tokens) the small
-// parameter kernel runs between the stages instead of inside every code workgroup.
+// With more than 64 partial ranges per channel (beyond 4096 tokens, unless the launcher
+// caps them because enough Q work covers the longer walks) the small parameter kernel
+// runs between the stages instead of inside every code workgroup.
 // A workgroup finds its role from its index; every role runs the same device
 // function as the stand-alone kernel, so results are bit-identical.  Used when K and V
 // have the same extents (always, for callers of the attention API).
