@@ -15,6 +15,7 @@ namespace risa {
 template <> int launch_attention_variant<64>(const KernelParams&, int, bool, bool, bool, int, hipStream_t);
 template <> int launch_attention_variant<128>(const KernelParams&, int, bool, bool, bool, int, hipStream_t);
 int launch_attention_narrow(const KernelParams& p, int head_dim, int cta_k, hipStream_t stream);
+int launch_attention_d256(const KernelParams& p, bool fast, hipStream_t stream);
 int launch_attention_narrow_general(const KernelParams& p, int head_dim, int cta_k, bool fast, bool indexed,
                                     bool capture, int mask_mode, hipStream_t stream);
 
@@ -227,7 +228,21 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
   const bool narrow_general = !narrow && mask_mode != kMaskLanes &&
                               (a.head_dim > 128 || workgroups <= narrow_attention_limit());
   int status;
-  if (narrow)
+  // Head dim 256 over 128-key tiles: thirty-two queries per wavefront where there is more than one
+  // workgroup per compute unit (attention_d256.hip; it copies whole key tiles).  A workgroup takes
+  // longer there (two share a unit), so one round of them is no gain (16 heads x 2048 74.2 against 75.5
+  // us whole call), and under the causal rule, where the longest block is the time, neither are two
+  // rounds of one per unit: attention from packed operands at 384 / 480 / 512 / 544 / 1024 workgroups,
+  // full 97.5 -> 73.2, 100 -> 82.5, 107 -> 86.2, 150 -> 125, 213 -> 169 us (2048 tokens); causal 53.0 ->
+  // 58.0, 63.3 -> 62.6, 66.6 -> 63.9, 80.1 -> 66.0, 136 -> 100 there and 188 -> 191, 185 -> 203, 212 -> 215,
+  // 286 -> 238 (640), 398 -> 312 us at 8192.
+  const bool wide_heads = a.head_dim == 256 && a.cta_k == 128 && !capture && !sparse && !p.compiled_loop &&
+                          (a.mask == nullptr || a.key_bias != nullptr) &&
+                          (a.whole_key_tiles || a.k_len % 128 == 0) &&
+                          workgroups > (a.is_causal ? 2 : 1) * narrow_attention_limit();
+  if (wide_heads)
+    status = launch_attention_d256(p, fast, stream);
+  else if (narrow)
     status = launch_attention_narrow(p, a.head_dim, a.cta_k, stream);
   else if (narrow_general)
     status = launch_attention_narrow_general(p, a.head_dim, a.cta_k, fast, indexed, capture, mask_mode, stream);
