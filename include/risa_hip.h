@@ -207,6 +207,27 @@ int risa_attention_readable_keys(const void* q_int8, const void* k_int8, const v
                    const float* key_bias, int64_t key_bias_stride_b, int64_t key_bias_stride_h,
                    const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
                    int64_t mask_lanes_stride_h, int64_t k_bytes, void* stream);
+/* The same with a workspace (16-byte aligned, nullable) for launches of few query blocks: workgroups of
+ * their own then walk ranges of the key tiles, and a second kernel puts their results together (the
+ * order of FP32 additions differs from a walk over all tiles, nothing else).  Without it, or with fewer bytes
+ * than risa_attention_split_bytes says, a workgroup walks all key tiles of its queries.  The size is 0
+ * where nothing is split, for any scale and causal flag; capturing and sparse calls are not split.
+ * mask_dtype is -1 without a mask. */
+int risa_attention_split(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
+                   const float* q_scale, const float* k_scale, const float* v_scale,
+                   const float* v_center, const int32_t* v_tile_sum, const void* mask,
+                   int64_t mask_stride_b, int64_t mask_stride_h, int64_t mask_stride_q,
+                   int64_t mask_stride_k, int mask_dtype, int cta_k, int batch, int q_len,
+                   int k_len, int q_heads, int kv_heads, int head_dim, int64_t out_stride_b,
+                   int64_t out_stride_n, int64_t out_stride_h, float sm_scale, int out_dtype,
+                   const int32_t* sparse_row_offsets, const int32_t* sparse_block_indices,
+                   float* block_mass, int is_causal, float* lse, const int32_t* key_mask_tiles,
+                   const float* key_bias, int64_t key_bias_stride_b, int64_t key_bias_stride_h,
+                   const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
+                   int64_t mask_lanes_stride_h, int64_t k_bytes, void* split_workspace,
+                   size_t split_workspace_bytes, void* stream);
+size_t risa_attention_split_bytes(int batch, int q_heads, int q_len, int k_len, int head_dim, int cta_k,
+                                  int mask_dtype, int64_t mask_stride_q);
 
 /*
  * Quantise and attend in one call.  Replaces risa_sdpa (reference

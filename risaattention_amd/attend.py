@@ -152,20 +152,32 @@ def launch_attention(*, q_codes, k_codes, v_codes, output, q_scale, k_scale, v_s
     # (a last tile of fewer keys is copied whole where the storage goes on behind the keys)
     whole = padded == k_len or k_len < KEYS_WITH_ROOM
     readable_keys = 0 if whole else k_codes.untyped_storage().nbytes() - k_codes.storage_offset()
+    # (launches of few query blocks split the keys over workgroups and keep their results here)
+    split_bytes = 0
+    if block_mass is None and row_offsets is None:
+        split_bytes = attention_split_bytes(batch, q_heads, q_len, k_len, dim, cta_k, mask_args[5], mask_args[3])
+    split = torch.empty(split_bytes, dtype=torch.uint8, device=q_codes.device) if split_bytes else None
     out_b = output.stride(0) if batch > 1 else q_heads * q_len * dim
     out_n = output.stride(2) if q_len > 1 else dim
     out_h = output.stride(1) if q_heads > 1 else q_len * dim
     native.check(
-        native.library().risa_attention_readable_keys(
+        native.library().risa_attention_split(
             q_codes.data_ptr(), k_codes.data_ptr(), v_codes.data_ptr(), output.data_ptr(),
             q_scale.data_ptr(), k_scale.data_ptr(), v_scale.data_ptr(), v_center.data_ptr(),
             sums.data_ptr(), *mask_args, cta_k, batch, q_len, k_len, q_heads, kv_heads, dim,
             out_b, out_n, out_h, float(sm_scale), DTYPE_CODES[output.dtype],
             native.pointer(row_offsets), native.pointer(block_indices), native.pointer(block_mass),
             int(bool(is_causal)), native.pointer(lse), native.pointer(key_mask_tiles),
-            *bias_args, *lane_args, readable_keys, native.current_stream(q_codes.device),
+            *bias_args, *lane_args, readable_keys, native.pointer(split), split_bytes,
+            native.current_stream(q_codes.device),
         )
     )
+
+
+@functools.lru_cache(maxsize=256)
+def attention_split_bytes(*extents) -> int:
+    """``risa_attention_split_bytes`` of the library, remembered like ``sdpa_workspace_bytes``."""
+    return native.library().risa_attention_split_bytes(*extents)
 
 
 @functools.lru_cache(maxsize=256)
@@ -178,6 +190,7 @@ def sdpa_workspace_bytes(*extents) -> int:
 def forget_cached_sizes() -> None:
     """Drop the remembered workspace sizes (they belong to the library that computed them)."""
     sdpa_workspace_bytes.cache_clear()
+    attention_split_bytes.cache_clear()
 
 
 def execute_dense_attention(

@@ -227,6 +227,21 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
   // the 32-query kernel that reads them.
   const bool narrow_general = !narrow && mask_mode != kMaskLanes &&
                               (a.head_dim > 128 || workgroups <= narrow_attention_limit());
+  // Few query blocks: ranges of the key tiles go to workgroups of their own.  (A sparse pattern's lists
+  // can be much shorter than the key range, which nothing here knows.)
+  if ((narrow || narrow_general) && !capture && !sparse && a.split_workspace != nullptr) {
+    const AttentionExtents extents{a.batch, a.q_heads, a.q_len, a.k_len, a.head_dim, a.cta_k};
+    const SplitKind kind = fast ? SplitKind::kPlain
+                           : a.mask != nullptr && a.key_bias == nullptr ? SplitKind::kMaskTensor : SplitKind::kScaled;
+    const int parts = attention_key_parts(extents, kind, a.is_causal);
+    const size_t blocks = static_cast<size_t>(workgroups);
+    if (parts > 1 && a.split_workspace_bytes >= parts * blocks * key_part_bytes(a.head_dim)) {
+      if (reinterpret_cast<uintptr_t>(a.split_workspace) % 16 != 0)
+        return fail("risa_attention: the workspace of key ranges must be 16-byte aligned");
+      p.key_parts = parts;
+      p.partial = static_cast<float*>(a.split_workspace);
+    }
+  }
   int status;
   // Head dim 256 over 128-key tiles: thirty-two queries per wavefront where there is more than one
   // workgroup per compute unit (attention_d256.hip; it copies whole key tiles).  A workgroup takes

@@ -88,6 +88,8 @@ struct KernelParams {
   int causal;
   int whole_key_tiles;  // the last key tile can be copied whole although fewer keys are left
   int compiled_loop;  // non-zero: every tile through the loop the compiler schedules (see RISA_COMPILED_LOOP)
+  int key_parts;   // ranges of the key tiles that workgroups of their own walk (sixteen-query kernel; 0, 1: one)
+  float* partial;  // their results, before merge_key_parts_kernel
 };
 
 // Byte offset of 16-byte chunk `chunk` of row `row` in a swizzled LDS tile.

@@ -64,6 +64,56 @@ __device__ __forceinline__ uint32_t sum_across_row_pairs(uint32_t x) {
   return both[0] + both[1];
 }
 
+// Output of one query from the sixteen-query layout: channel blocks first_cb .. first_cb + BLOCKS - 1.
+// `guarded`: rows without any visible key (masks, causal) are zeros.
+// A lane owns one query and four channels per 16-channel block: stored from there, an
+// instruction would write 32 bytes into each of 16 rows.  Two blocks are exchanged between
+// neighbouring rows of lanes first (v_permlane16_swap: the odd rows of one register for the
+// even rows of the other), after which a lane holds eight consecutive channels and an
+// instruction writes 64 contiguous bytes of each row.  (The four lanes of a query are
+// active or inactive together, so the exchange works inside a branch on the query.)
+template <int D, int BLOCKS>
+__device__ __forceinline__ void store_narrow_rows(const KernelParams& p, int64_t bhk, int batch, int head,
+                                                  int query, int grp, int first_cb, const float (&o_acc)[BLOCKS][4],
+                                                  float d_total, bool guarded) {
+  const float inv_d = 1.0f / d_total;
+  const bool zero_row = guarded && !(d_total > 0.0f);
+  const float* vs = p.v_scale + bhk * D;
+  const float* vc = p.v_center + bhk * D;
+  unsigned char* out_row = static_cast<unsigned char*>(p.out) +
+                           2 * (batch * p.out_stride_b + head * p.out_stride_h +
+                                static_cast<int64_t>(query) * p.out_stride_n);
+#pragma unroll
+  for (int cb = 0; cb < BLOCKS; cb += 2) {
+    uint32_t word[2][2];  // [block of the pair][channel pair]
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int c = (first_cb + cb + j) * 16 + grp * 4;
+      const v4f scale4 = *reinterpret_cast<const v4f*>(vs + c);
+      const v4f center4 = *reinterpret_cast<const v4f*>(vc + c);
+      float value[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        value[r] = __builtin_fmaf(o_acc[cb + j][r] * inv_d, scale4[r], center4[r]);
+        value[r] = zero_row ? 0.0f : value[r];
+      }
+      word[j][0] = to_output_pair(value[0], value[1], p.out_dtype);
+      word[j][1] = to_output_pair(value[2], value[3], p.out_dtype);
+    }
+    // even rows of lanes end with channels 8*(grp/2) .. +7 of the first block, odd rows
+    // with the same channels of the second block
+    const auto low = __builtin_amdgcn_permlane16_swap(word[0][0], word[1][0], false, false);
+    const auto high = __builtin_amdgcn_permlane16_swap(word[0][1], word[1][1], false, false);
+    const v4i piece = {static_cast<int>(low[0]), static_cast<int>(high[0]), static_cast<int>(low[1]),
+                       static_cast<int>(high[1])};
+    *reinterpret_cast<v4i*>(out_row + (first_cb + cb + (grp & 1)) * 32 + (grp >> 1) * 16) = piece;
+  }
+}
+
+__device__ __forceinline__ void store_narrow_lse(const KernelParams& p, int64_t bhq, int query, float m, float d_total) {
+  p.lse[bhq * p.q_len + query] = d_total > 0.0f ? (__builtin_amdgcn_logf(d_total) + m) / kLog2e : -__builtin_inff();
+}
+
 template <int D, int CTA_K, int WAVES, int KSPLIT = 1, bool INDEXED = false, bool GENERAL = false,
           bool CAPTURE = false, int MASK_DT = -1, bool MASK_VEC = false>
 __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(const KernelParams p) {
@@ -93,17 +143,19 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
   unsigned char* lds = lds_all + part * Shape::kLdsBytes;
 
   const int query_blocks = (p.q_len + QUERIES - 1) / QUERIES;
+  constexpr bool RANGES = WAVES == 8 && KSPLIT == 1 && !CAPTURE;  // of the key tiles: blockIdx.y, p.key_parts of them
+  const int block = blockIdx.x, key_part = blockIdx.y;
   int bx, head, batch;
   if (GENERAL && p.causal) {
     // longest query blocks first, across all heads (as in the wide kernel)
     const int heads = p.q_heads * p.batch;
-    const int rest = blockIdx.x % heads;
-    bx = query_blocks - 1 - blockIdx.x / heads;
+    const int rest = block % heads;
+    bx = query_blocks - 1 - block / heads;
     head = rest % p.q_heads;
     batch = rest / p.q_heads;
   } else {
-    bx = blockIdx.x % query_blocks;
-    const int rest = blockIdx.x / query_blocks;
+    bx = block % query_blocks;
+    const int rest = block / query_blocks;
     head = rest % p.q_heads;
     batch = rest / p.q_heads;
   }
@@ -122,33 +174,47 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
 
   const int query = bx * QUERIES + wave * 16 + ql;
   const bool query_ok = query < p.q_len;
-  // KSPLIT == 2: the second part takes the last floor(n/2) tiles, the first part the rest.
-  const int second_half = p.n_kb / 2;
-  int n_it = KSPLIT == 1 ? p.n_kb : part == 0 ? p.n_kb - second_half : second_half;
-  const int first_tile = part == 0 ? 0 : p.n_kb - second_half;
+  int listed = p.n_kb;  // key tiles of the query block
   [[maybe_unused]] const int32_t* indices = nullptr;
   if constexpr (INDEXED) {
     if (p.index_mode == 1) {
       const int64_t row = bhq * p.n_qb + (bx * QUERIES) / kQueryBlock;
       const int start = p.row_offsets[row];
-      n_it = __builtin_amdgcn_readfirstlane(p.row_offsets[row + 1] - start);
+      listed = __builtin_amdgcn_readfirstlane(p.row_offsets[row + 1] - start);
       indices = p.tile_indices + start;
     } else {
       indices = p.tile_indices + bhq * (p.n_kb + 1);
-      n_it = __builtin_amdgcn_readfirstlane(indices[p.n_kb]);
+      listed = __builtin_amdgcn_readfirstlane(indices[p.n_kb]);
     }
   } else if constexpr (GENERAL && !CAPTURE) {
     if (p.causal) {
       const int limit = min(p.k_len, (bx + 1) * QUERIES);
-      n_it = (limit + CTA_K - 1) / CTA_K;
+      listed = (limit + CTA_K - 1) / CTA_K;
     }
   }
+  // This workgroup's range of them: all, or one of p.key_parts ranges whose results
+  // merge_key_parts_kernel puts together.  KSPLIT == 2: its second part takes the last floor(n/2) tiles
+  // of the range, the first part the rest.
+  int first_tile = 0, n_it = listed;
+  if (RANGES && p.key_parts > 1) {
+    first_tile = listed * key_part / p.key_parts;
+    n_it = listed * (key_part + 1) / p.key_parts - first_tile;
+  }
+  const int in_range = n_it;
+  if constexpr (KSPLIT == 2) {
+    n_it = part == 0 ? in_range - in_range / 2 : in_range / 2;
+    if (part == 1) first_tile += in_range - n_it;
+  }
+  // Only the last listed tile of the query block takes the last-tile formulas: its maxima start from
+  // this floor, and only it can hold keys past the end.
+  const bool holds_last = first_tile + n_it == listed;
+  const float last_floor = holds_last ? kRowFloor : -__builtin_inff();
   // listed tiles come through the scalar cache (uniform address; as vector loads their wait
   // would include every vector load requested before them)
   auto tile_at = [&](int step) -> int {
     if constexpr (INDEXED) {
       typedef const __attribute__((address_space(4))) int32_t* UniformEntries;
-      return ((UniformEntries)(reinterpret_cast<uintptr_t>(indices)))[step];
+      return ((UniformEntries)(reinterpret_cast<uintptr_t>(indices)))[first_tile + step];
     }
     return first_tile + step;
   };
@@ -511,8 +577,8 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
             mx0 = max(mx0, s[kb][i]);
           s[kb][i] = __float_as_int(score_value(s[kb][i]));
         }
-      tile_m = __builtin_fmaxf(__builtin_fmaf(__builtin_fmaxf(kRowFloor, score_value(mx0)), sc0, -kU8Offset),
-                               __builtin_fmaf(__builtin_fmaxf(kRowFloor, score_value(mx1)), sc1, -kU8Offset));
+      tile_m = __builtin_fmaxf(__builtin_fmaf(__builtin_fmaxf(last_floor, score_value(mx0)), sc0, -kU8Offset),
+                               __builtin_fmaf(__builtin_fmaxf(last_floor, score_value(mx1)), sc1, -kU8Offset));
     } else {
       // Last tile: out-of-range keys become -1e30 and every scale group's maximum
       // starts from -50000 before scaling.
@@ -654,7 +720,7 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       __syncthreads();
       [[maybe_unused]] int listed_after_next = 0;
-      if constexpr (INDEXED) listed_after_next = indices[min(step + 2, n_it - 1)];
+      if constexpr (INDEXED) listed_after_next = indices[first_tile + min(step + 2, n_it - 1)];
       load_k_fragments(lds + stage * Shape::kStageBytes, 0, k_first);
       tile_scales(stage, ks0, ks1);
       if constexpr (PRELOAD) {
@@ -684,13 +750,7 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
     load_k_fragments(lds + stage * Shape::kStageBytes, 0, k_first);
     tile_scales(stage, ks0, ks1);
     score_tile(stage, k_first, s);
-    // Only the last tile of the sequence takes the last-tile formulas.
-    float t_scale;
-    if (KSPLIT == 1 || part == KSPLIT - 1) {
-      t_scale = softmax_tile(std::true_type{}, n_it - 1, tile, ks0, ks1, s, pk);
-    } else {
-      t_scale = softmax_tile(std::false_type{}, n_it - 1, tile, ks0, ks1, s, pk);
-    }
+    const float t_scale = softmax_tile(std::true_type{}, n_it - 1, tile, ks0, ks1, s, pk);
     load_group(stage, 0, acc_first, v_first);
     value_tile(stage, pk, acc_first, v_first, t_scale);
   }
@@ -698,7 +758,7 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
   if constexpr (KSPLIT == 2) {
     // Both parts share the workgroup's barrier: with an odd tile count the second part has
     // walked one tile less and takes the barrier of the tile it does not have.
-    if (part == 1 && (p.n_kb & 1)) __syncthreads();
+    if (part == 1 && (in_range & 1)) __syncthreads();
   }
 
   // ---- merge of the two key halves ----------------------------------------------------------
@@ -732,6 +792,20 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
     m_run = merged_m;
   }
 
+  // ---- partial result of a range of the key tiles ---------------------------------------------
+  // Value-major, so that the lanes of a wavefront store neighbouring words.
+  if (RANGES && p.key_parts > 1) {
+    constexpr int VALUES = CB * 4 + 2;
+    float* at = p.partial + ((static_cast<int64_t>(key_part) * gridDim.x + block) * WAVES + wave) * (VALUES * 64) + lane;
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) at[(cb * 4 + i) * 64] = o_acc[cb][i];
+    at[(CB * 4) * 64] = m_run;
+    at[(CB * 4 + 1) * 64] = d_part;
+    return;
+  }
+
   // ---- epilogue ---------------------------------------------------------------------------
   float d_total = d_part + __shfl_xor(d_part, 16);
   d_total += __shfl_xor(d_total, 32);
@@ -743,50 +817,86 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
       state[stat_row * 2 + 1] = d_total;
     }
   }
-  const float inv_d = 1.0f / d_total;
-  // rows without any visible key (masks, causal): zeros
-  const bool zero_row = GENERAL && (MASK_DT >= 0 || p.causal) && !(d_total > 0.0f);
-  // A lane owns one query and four channels per 16-channel block: stored from there, an
-  // instruction would write 32 bytes into each of 16 rows.  Two blocks are exchanged between
-  // neighbouring rows of lanes first (v_permlane16_swap: the odd rows of one register for the
-  // even rows of the other), after which a lane holds eight consecutive channels and an
-  // instruction writes 64 contiguous bytes of each row.  (The four lanes of a query are
-  // active or inactive together, so the exchange stays inside the branch.)
   if (query_ok) {
-    const float* vs = p.v_scale + bhk * D;
-    const float* vc = p.v_center + bhk * D;
-    unsigned char* out_row = static_cast<unsigned char*>(p.out) +
-                             2 * (batch * p.out_stride_b + head * p.out_stride_h +
-                                  static_cast<int64_t>(query) * p.out_stride_n);
+    store_narrow_rows<D, CB>(p, bhk, batch, head, query, grp, 0, o_acc, d_total,
+                             GENERAL && (MASK_DT >= 0 || p.causal));
+    if (p.lse != nullptr && grp == 0) store_narrow_lse(p, bhq, query, m_run, d_total);
+  }
+}
+
+// Puts the ranges of the key tiles together (p.key_parts partial results per query): the online-softmax
+// update once more, so only the order of FP32 additions differs from a walk over all tiles.  A wavefront
+// takes sixteen queries of an attention_narrow_kernel<D, CTA_K, 8> workgroup and 64 channels, so that
+// few query blocks still fill the machine.
+template <int D> __global__ __launch_bounds__(256) void merge_key_parts_kernel(const KernelParams p) {
+  constexpr int CB = D / 16, VALUES = CB * 4 + 2, WAVES = 8, QUERIES = 16 * WAVES;
+  const int lane = threadIdx.x & 63, ql = lane & 15, grp = lane >> 4;
+  const int query_blocks = (p.q_len + QUERIES - 1) / QUERIES;
+  const int blocks = query_blocks * p.q_heads * p.batch;
+  const int index = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int first_cb = index % (D / 64) * 4, walked = index / (D / 64);  // wavefront of the walking launch
+  if (walked >= blocks * WAVES) return;
+  const int wave = walked % WAVES, block = walked / WAVES;
+  int bx, head, batch;
+  if (p.causal) {
+    const int heads = p.q_heads * p.batch;
+    const int rest = block % heads;
+    bx = query_blocks - 1 - block / heads;
+    head = rest % p.q_heads;
+    batch = rest / p.q_heads;
+  } else {
+    bx = block % query_blocks;
+    const int rest = block / query_blocks;
+    head = rest % p.q_heads;
+    batch = rest / p.q_heads;
+  }
+  const int64_t bhk = static_cast<int64_t>(batch) * p.kv_heads + head / (p.q_heads / p.kv_heads);
+  const int64_t bhq = static_cast<int64_t>(batch) * p.q_heads + head;
+  const int query = bx * QUERIES + wave * 16 + ql;
+  const int64_t part_stride = static_cast<int64_t>(blocks) * WAVES * (VALUES * 64);
+  const float* at = p.partial + static_cast<int64_t>(walked) * (VALUES * 64) + lane;
+  // Four ranges at a time, their loads in flight together (one by one, a range costs its round trip:
+  // 16 of them 23 us for 16 query blocks of 128 channels).  Past the last range the last one is read again
+  // and counts nothing.
+  constexpr int BATCH = 4;
+  float m = kRowFloor, d = 0.0f, o_acc[4][4] = {};
+  for (int first = 0; first < p.key_parts; first += BATCH) {
+    float value[BATCH][4][4], its_m[BATCH], its_d[BATCH];
 #pragma unroll
-    for (int cb = 0; cb < CB; cb += 2) {
-      uint32_t word[2][2];  // [block of the pair][channel pair]
+    for (int j = 0; j < BATCH; ++j) {
+      const float* source = at + min(first + j, p.key_parts - 1) * part_stride;
+      its_m[j] = source[CB * 4 * 64];
+      its_d[j] = source[(CB * 4 + 1) * 64];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int c = (cb + j) * 16 + grp * 4;
-        const v4f scale4 = *reinterpret_cast<const v4f*>(vs + c);
-        const v4f center4 = *reinterpret_cast<const v4f*>(vc + c);
-        float value[4];
+      for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          value[r] = __builtin_fmaf(o_acc[cb + j][r] * inv_d, scale4[r], center4[r]);
-          value[r] = zero_row ? 0.0f : value[r];
-        }
-        word[j][0] = to_output_pair(value[0], value[1], p.out_dtype);
-        word[j][1] = to_output_pair(value[2], value[3], p.out_dtype);
-      }
-      // even rows of lanes end with channels 8*(grp/2) .. +7 of the first block, odd rows
-      // with the same channels of the second block
-      const auto low = __builtin_amdgcn_permlane16_swap(word[0][0], word[1][0], false, false);
-      const auto high = __builtin_amdgcn_permlane16_swap(word[0][1], word[1][1], false, false);
-      const v4i piece = {static_cast<int>(low[0]), static_cast<int>(high[0]), static_cast<int>(low[1]),
-                         static_cast<int>(high[1])};
-      *reinterpret_cast<v4i*>(out_row + (cb + (grp & 1)) * 32 + (grp >> 1) * 16) = piece;
+        for (int i = 0; i < 4; ++i) value[j][cb][i] = source[((first_cb + cb) * 4 + i) * 64];
     }
-    if (p.lse != nullptr && grp == 0) {
-      p.lse[bhq * p.q_len + query] =
-          d_total > 0.0f ? (__builtin_amdgcn_logf(d_total) + m_run) / kLog2e : -__builtin_inff();
+    float top = m;
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) top = __builtin_fmaxf(top, its_m[j]);
+    const float scale = __builtin_amdgcn_exp2f(m - top);
+    m = top;
+    d *= scale;
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o_acc[cb][i] *= scale;
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) {
+      const float weight = first + j < p.key_parts ? __builtin_amdgcn_exp2f(its_m[j] - m) : 0.0f;
+      d = __builtin_fmaf(its_d[j], weight, d);
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o_acc[cb][i] = __builtin_fmaf(value[j][cb][i], weight, o_acc[cb][i]);
     }
+  }
+  float d_total = d + __shfl_xor(d, 16);
+  d_total += __shfl_xor(d_total, 32);
+  if (query < p.q_len) {
+    store_narrow_rows<D, 4>(p, bhk, batch, head, query, grp, first_cb, o_acc, d_total, p.mask_dtype >= 0 || p.causal);
+    if (p.lse != nullptr && grp == 0 && first_cb == 0) store_narrow_lse(p, bhq, query, m, d_total);
   }
 }
 
@@ -808,9 +918,14 @@ int launch_narrow_block(const KernelParams& p, hipStream_t stream) {
     configured_device = device;
   }
   constexpr int QUERIES = 16 * WAVES;
-  const unsigned query_blocks = static_cast<unsigned>((p.q_len + QUERIES - 1) / QUERIES);
-  const dim3 grid(query_blocks * p.q_heads * p.batch);
-  kernel<<<grid, 64 * WAVES * KSPLIT, kLdsBytes, stream>>>(p);
+  const unsigned blocks = static_cast<unsigned>((p.q_len + QUERIES - 1) / QUERIES) * p.q_heads * p.batch;
+  constexpr bool RANGES = WAVES == 8 && KSPLIT == 1 && !CAPTURE;
+  const unsigned parts = RANGES && p.key_parts > 1 ? p.key_parts : 1;
+  kernel<<<dim3(blocks, parts), 64 * WAVES * KSPLIT, kLdsBytes, stream>>>(p);
+  if constexpr (RANGES) {
+    const unsigned wavefronts = blocks * WAVES * (D / 64);
+    if (parts > 1) merge_key_parts_kernel<D><<<dim3((wavefronts + 3) / 4), 256, 0, stream>>>(p);
+  }
   return 0;
 }
 

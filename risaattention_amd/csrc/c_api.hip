@@ -289,7 +289,15 @@ void risa_unpack_order(int32_t* order) {
   for (int token = 0; token < 32; ++token) order[risa::packed_value_position(token)] = token;
 }
 
-int risa_attention_readable_keys(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
+size_t risa_attention_split_bytes(int batch, int q_heads, int q_len, int k_len, int head_dim, int cta_k,
+                                  int mask_dtype, int64_t mask_stride_q) {
+  if (batch <= 0 || q_heads <= 0 || q_len <= 0 || k_len <= 0 || (cta_k != 64 && cta_k != 128) ||
+      (head_dim != 64 && head_dim != 128 && head_dim != 256))
+    return 0;
+  return risa::attention_split_bytes({batch, q_heads, q_len, k_len, head_dim, cta_k}, mask_dtype, mask_stride_q);
+}
+
+int risa_attention_split(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
                    const float* q_scale, const float* k_scale, const float* v_scale,
                    const float* v_center, const int32_t* v_tile_sum, const void* mask,
                    int64_t mask_stride_b, int64_t mask_stride_h, int64_t mask_stride_q,
@@ -300,7 +308,8 @@ int risa_attention_readable_keys(const void* q_int8, const void* k_int8, const v
                    float* block_mass, int is_causal, float* lse, const int32_t* key_mask_tiles,
                    const float* key_bias, int64_t key_bias_stride_b, int64_t key_bias_stride_h,
                    const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
-                   int64_t mask_lanes_stride_h, int64_t k_bytes, void* stream) {
+                   int64_t mask_lanes_stride_h, int64_t k_bytes, void* split_workspace,
+                   size_t split_workspace_bytes, void* stream) {
   using risa::fail;
   if (out_dtype != 1 && out_dtype != 2)
     return fail("risa_attention: output dtype code must be 1 (fp16) or 2 (bf16)");
@@ -355,7 +364,24 @@ int risa_attention_readable_keys(const void* q_int8, const void* k_int8, const v
   a.mask_lanes_stride_h = mask_lanes_stride_h;
   // whole tiles of K may be copied where the bytes behind the last key can be read
   a.whole_key_tiles = k_bytes >= (static_cast<int64_t>(batch) * kv_heads * k_len + cta_k) * head_dim;
+  a.split_workspace = split_workspace;
+  a.split_workspace_bytes = split_workspace_bytes;
   return risa::launch_attention(a, static_cast<hipStream_t>(stream));
+}
+
+int risa_attention_readable_keys(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
+                   const float* q_scale, const float* k_scale, const float* v_scale,
+                   const float* v_center, const int32_t* v_tile_sum, const void* mask,
+                   int64_t mask_stride_b, int64_t mask_stride_h, int64_t mask_stride_q,
+                   int64_t mask_stride_k, int mask_dtype, int cta_k, int batch, int q_len,
+                   int k_len, int q_heads, int kv_heads, int head_dim, int64_t out_stride_b,
+                   int64_t out_stride_n, int64_t out_stride_h, float sm_scale, int out_dtype,
+                   const int32_t* sparse_row_offsets, const int32_t* sparse_block_indices,
+                   float* block_mass, int is_causal, float* lse, const int32_t* key_mask_tiles,
+                   const float* key_bias, int64_t key_bias_stride_b, int64_t key_bias_stride_h,
+                   const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
+                   int64_t mask_lanes_stride_h, int64_t k_bytes, void* stream) {
+  return risa_attention_split(q_int8, k_int8, v_int8, out, q_scale, k_scale, v_scale, v_center, v_tile_sum, mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, cta_k, batch, q_len, k_len, q_heads, kv_heads, head_dim, out_stride_b, out_stride_n, out_stride_h, sm_scale, out_dtype, sparse_row_offsets, sparse_block_indices, block_mass, is_causal, lse, key_mask_tiles, key_bias, key_bias_stride_b, key_bias_stride_h, mask_lanes, mask_lanes_stride_b, mask_lanes_stride_h, k_bytes, nullptr, 0, stream);
 }
 
 int risa_attention(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
@@ -530,7 +556,8 @@ size_t risa_sdpa_workspace_bytes(int batch, int q_heads, int q_len, int kv_heads
                                              batch, q_heads, mask_batch, mask_heads, q_len, k_len);
   return sdpa_layout(batch, q_heads, q_len, kv_heads, k_len, head_dim, cta_k, midpoint_affine != 0,
                      key_only, lanes)
-      .bytes;
+             .bytes +
+         risa_attention_split_bytes(batch, q_heads, q_len, k_len, head_dim, cta_k, mask_dtype, mask_stride_q);
 }
 
 int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, void* workspace,
@@ -620,14 +647,16 @@ int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, v
     if (status != 0) return status;
     key_tiles = list;
   }
-  // (behind the K codes lie those of V, a whole key tile at least)
-  return risa_attention_readable_keys(base + l.q_codes, base + l.k_codes, base + l.v_codes, out, q_scale, k_scale,
+  // (behind the K codes lie those of V, a whole key tile at least; behind the sections the partial results
+  // of key ranges, where the workspace is as large as risa_sdpa_workspace_bytes says)
+  return risa_attention_split(base + l.q_codes, base + l.k_codes, base + l.v_codes, out, q_scale, k_scale,
                         v_scale, v_center, tile_sum, mask, mask_stride_b, mask_stride_h,
                         mask_stride_q, mask_stride_k, mask_dtype, cta_k, batch, q_len, k_len,
                         q_heads, kv_heads, head_dim, out_stride_b, out_stride_n, out_stride_h,
                         sm_scale, output_dtype, sparse_row_offsets, sparse_block_indices, nullptr,
                         is_causal, nullptr, key_tiles, key_bias, bias_stride_b, bias_stride_h,
-                        mask_lanes, lanes_stride_b, lanes_stride_h, static_cast<int64_t>(l.bytes - l.k_codes), stream);
+                        mask_lanes, lanes_stride_b, lanes_stride_h, static_cast<int64_t>(l.bytes - l.k_codes),
+                        base + l.bytes, workspace_bytes - l.bytes, stream);
 }
 
 int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* workspace,

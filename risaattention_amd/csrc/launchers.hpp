@@ -85,11 +85,24 @@ struct AttentionArgs {
   int64_t key_bias_stride_b, key_bias_stride_h;
   const uint64_t* mask_lanes;  // lane words from launch_mask_lanes, or null
   int64_t mask_lanes_stride_b, mask_lanes_stride_h;  // in words
+  void* split_workspace;  // for partial results of key ranges, or null: a workgroup walks all key tiles
+  size_t split_workspace_bytes;
 };
 int launch_attention(const AttentionArgs& args, hipStream_t stream);
 // Number of 128-query workgroups up to which a launch takes the sixteen-query kernel: the
 // compute units of the current device (the MI355X's 256 when no device can be queried).
 int narrow_attention_limit();
+// Ranges that workgroups of their own walk where a launch has few query blocks (1: no split), and the
+// bytes their results take before they are put together (0 where nothing is split, whatever the scale
+// and the causal flag are).
+struct AttentionExtents {
+  int batch, q_heads, q_len, k_len, head_dim, cta_k;
+};
+enum class SplitKind { kPlain, kScaled, kMaskTensor };  // raw scores; pre-scaled ones, additive rows too; masks read per score
+int attention_key_parts(const AttentionExtents& e, SplitKind kind, bool causal);
+size_t attention_split_bytes(const AttentionExtents& e, int mask_dtype, int64_t mask_stride_q);
+// of one range of one query block: eight wavefronts, head_dim / 4 outputs, maximum and denominator a lane
+constexpr size_t key_part_bytes(int head_dim) { return size_t{512} * (head_dim / 4 + 2) * sizeof(float); }
 
 struct SelectArgs {
   const float* sorted_mass;

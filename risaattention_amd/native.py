@@ -71,6 +71,16 @@ SIGNATURES = {
         + [_c_f32, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr]
         + [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_ptr],
     ),
+    "risa_attention_split": (
+        _c_int,
+        [_c_ptr] * 10
+        + [_c_i64] * 4
+        + [_c_int] * 8
+        + [_c_i64] * 3
+        + [_c_f32, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr]
+        + [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_ptr, _c_size, _c_ptr],
+    ),
+    "risa_attention_split_bytes": (_c_size, [_c_int] * 7 + [_c_i64]),
     "risa_mask_lanes_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_i64, _c_i64] + [_c_int] * 6),
     "risa_prepare_mask_lanes": (
         _c_int,

@@ -526,3 +526,15 @@ def test_library_swap_routes_calls_and_restores():
     assert native.library() is own
     with pytest.raises(OSError):
         native.load_library(ROOT / "no_such_library.so")
+
+
+def test_partial_results_of_key_ranges_are_sized_by_the_extents():
+    """Only launches of few query blocks over many keys split; the size covers every scale and flag."""
+    size = native.library().risa_attention_split_bytes
+    assert size(1, 16, 32768, 32768, 128, 128, -1, 0) == 0
+    assert size(1, 16, 128, 64, 128, 64, -1, 0) == 0
+    plain = size(1, 16, 128, 8192, 128, 128, -1, 0)
+    part = 16 * 512 * (128 // 4 + 2) * 4
+    assert plain > 0 and plain % part == 0 and plain // part <= 16
+    assert size(1, 16, 128, 8192, 128, 64, 3, 8192) >= plain
+    assert size(1, 0, 128, 8192, 128, 128, -1, 0) == size(1, 16, 128, 8192, 96, 128, -1, 0) == 0
