@@ -271,6 +271,18 @@ int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, v
               int64_t mask_stride_q, int64_t mask_stride_k, int mask_dtype, int mask_batch,
               int mask_heads, int is_causal, const int32_t* sparse_row_offsets,
               const int32_t* sparse_block_indices, int channels, void* stream);
+/* The same with the natural-log normalisers of the rows, anchor correction included, in lse
+ * [batch][q_heads][q_len] (null: not stored). */
+int risa_sdpa_lse(const void* q, const void* k, const void* v, void* out, void* workspace,
+              size_t workspace_bytes, int batch, int q_heads, int q_len, int kv_heads, int k_len,
+              int head_dim, int cta_k, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
+              int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b,
+              int64_t v_stride_h, int64_t v_stride_n, int64_t out_stride_b, int64_t out_stride_n,
+              int64_t out_stride_h, float sm_scale, int input_dtype, int output_dtype,
+              int midpoint_affine, const void* mask, int64_t mask_stride_b, int64_t mask_stride_h,
+              int64_t mask_stride_q, int64_t mask_stride_k, int mask_dtype, int mask_batch,
+              int mask_heads, int is_causal, const int32_t* sparse_row_offsets,
+              const int32_t* sparse_block_indices, int channels, float* lse, void* stream);
 
 /*
  * Retained-mass selection over masses already sorted in descending order.

@@ -204,7 +204,8 @@ def execute_dense_attention(
     is_causal: bool = False,
     sparse_pattern: RetainedMassPattern | None = None,
     output_layout: str = "hnd",
-) -> torch.Tensor:
+    return_lse: bool = False,
+) -> torch.Tensor | tuple[torch.Tensor, torch.Tensor]:
     """Quantize and attend in one native call; the intermediate buffers are sections of
     one workspace that lives only for the call (reference _execution.py:28-134 over
     ``_C.risa_sdpa``).  With ``sparse_pattern`` the attention walks the pattern's key tiles
@@ -234,6 +235,7 @@ def execute_dense_attention(
         output = torch.empty(batch, q_len, q_heads, dim, dtype=out_dtype, device=q.device).permute(0, 2, 1, 3)
     else:
         output = torch.empty(batch, q_heads, q_len, dim, dtype=out_dtype, device=q.device)
+    lse = torch.empty((batch, q_heads, q_len), dtype=torch.float32, device=q.device) if return_lse else None
     if attn_mask is None:
         mask_args = (None, 0, 0, 0, 0, -1, 1, 1)
     else:
@@ -245,19 +247,21 @@ def execute_dense_attention(
                              mask_args[5], mask_args[3], mask_args[4], mask_args[6], mask_args[7]),
         dtype=torch.uint8, device=q.device)
     native.check(
-        lib.risa_sdpa_channels(
+        lib.risa_sdpa_lse(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), output.data_ptr(), workspace.data_ptr(),
             workspace.numel(), batch, q_heads, q_len, kv_heads, k_len, dim, cta_k,
             q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
             v.stride(0), v.stride(1), v.stride(2), output.stride(0), output.stride(2), output.stride(1),
             attention_scale, DTYPE_CODES[input_dtype], DTYPE_CODES[output.dtype],
-            int(use_midpoint_affine), *mask_args, int(bool(is_causal)), *csr, q.shape[-1],
+            int(use_midpoint_affine), *mask_args, int(bool(is_causal)), *csr, q.shape[-1], native.pointer(lse),
             native.current_stream(q.device),
         )
     )
     if original_dim != dim:
         output = output[..., :original_dim]
-    return output.float() if input_dtype == torch.float32 else output
+    if input_dtype == torch.float32:
+        output = output.float()
+    return (output, lse) if return_lse else output
 
 
 def check_pattern_for(pattern: RetainedMassPattern, *, batch, q_heads, q_len, k_len, cta_k,

@@ -181,6 +181,7 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
   p.out_dtype = a.out_dtype;
   p.workspace = a.block_mass;
   p.lse = a.lse;
+  p.lse_shift = a.lse_shift;
   p.causal = a.is_causal ? 1 : 0;
   p.whole_key_tiles = a.whole_key_tiles ? 1 : 0;
   // Diagnostic switch, read at every launch: RISA_COMPILED_LOOP=1 sends every kernel that has a

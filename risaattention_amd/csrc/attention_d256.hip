@@ -152,8 +152,8 @@ __global__ __launch_bounds__(256, 2) void attention_d256_kernel(const KernelPara
     }
   }
   if (p.lse != nullptr && half == 0 && query < p.q_len) {
-    p.lse[bhq * p.q_len + query] =
-        row_valid ? (__builtin_amdgcn_logf(d_total) + m_run) / kLog2e : -__builtin_inff();
+    store_lse(p, bhq * p.q_len + query,
+              row_valid ? (__builtin_amdgcn_logf(d_total) + m_run) / kLog2e : -__builtin_inff());
   }
 }
 

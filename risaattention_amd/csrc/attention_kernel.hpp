@@ -85,12 +85,18 @@ struct KernelParams {
   int64_t tile_list_stride_b, tile_list_stride_h;  // mode 3: elements between the lists of mask planes (0: shared)
   float* workspace;  // capture
   float* lse;
+  const float* lse_shift;  // added to the log-normalisers as they are stored (may be the same memory), or null
   int causal;
   int whole_key_tiles;  // the last key tile can be copied whole although fewer keys are left
   int compiled_loop;  // non-zero: every tile through the loop the compiler schedules (see RISA_COMPILED_LOOP)
   int key_parts;   // ranges of the key tiles that workgroups of their own walk (sixteen-query kernel; 0, 1: one)
   float* partial;  // their results, before merge_key_parts_kernel
 };
+
+// The log-normaliser of one row, with the logits that the K anchor took off where the caller has them.
+__device__ __forceinline__ void store_lse(const KernelParams& p, int64_t row, float value) {
+  p.lse[row] = p.lse_shift != nullptr ? value + p.lse_shift[row] : value;
+}
 
 // Byte offset of 16-byte chunk `chunk` of row `row` in a swizzled LDS tile.
 template <int ROWBYTES> __device__ __forceinline__ int swizzled(int row, int chunk) {
@@ -1415,8 +1421,8 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
     }
   }
   if (p.lse != nullptr && half == 0 && query_ok) {
-    p.lse[bhq * p.q_len + query] =
-        row_valid ? (__builtin_amdgcn_logf(d_total) + m_run) / kLog2e : -__builtin_inff();
+    store_lse(p, bhq * p.q_len + query,
+              row_valid ? (__builtin_amdgcn_logf(d_total) + m_run) / kLog2e : -__builtin_inff());
   }
 }
 

@@ -111,7 +111,7 @@ __device__ __forceinline__ void store_narrow_rows(const KernelParams& p, int64_t
 }
 
 __device__ __forceinline__ void store_narrow_lse(const KernelParams& p, int64_t bhq, int query, float m, float d_total) {
-  p.lse[bhq * p.q_len + query] = d_total > 0.0f ? (__builtin_amdgcn_logf(d_total) + m) / kLog2e : -__builtin_inff();
+  store_lse(p, bhq * p.q_len + query, d_total > 0.0f ? (__builtin_amdgcn_logf(d_total) + m) / kLog2e : -__builtin_inff());
 }
 
 template <int D, int CTA_K, int WAVES, int KSPLIT = 1, bool INDEXED = false, bool GENERAL = false,

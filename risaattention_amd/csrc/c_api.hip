@@ -171,6 +171,84 @@ int checked_v_args(risa::ValueArgs& a, const void* v, void* out, float* scale, f
 
 }  // namespace
 
+namespace {
+
+// One attention launch from the C arguments; `lse_shift`: the kernel adds it to `lse`.
+int attend(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
+                   const float* q_scale, const float* k_scale, const float* v_scale,
+                   const float* v_center, const int32_t* v_tile_sum, const void* mask,
+                   int64_t mask_stride_b, int64_t mask_stride_h, int64_t mask_stride_q,
+                   int64_t mask_stride_k, int mask_dtype, int cta_k, int batch, int q_len,
+                   int k_len, int q_heads, int kv_heads, int head_dim, int64_t out_stride_b,
+                   int64_t out_stride_n, int64_t out_stride_h, float sm_scale, int out_dtype,
+                   const int32_t* sparse_row_offsets, const int32_t* sparse_block_indices,
+                   float* block_mass, int is_causal, float* lse, const float* lse_shift, const int32_t* key_mask_tiles,
+                   const float* key_bias, int64_t key_bias_stride_b, int64_t key_bias_stride_h,
+                   const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
+                   int64_t mask_lanes_stride_h, int64_t k_bytes, void* split_workspace,
+                   size_t split_workspace_bytes, void* stream) {
+  using risa::fail;
+  if (out_dtype != 1 && out_dtype != 2)
+    return fail("risa_attention: output dtype code must be 1 (fp16) or 2 (bf16)");
+  if (mask != nullptr && (mask_dtype < 0 || mask_dtype > 3))
+    return fail("risa_attention: attention mask must be bool, float16, bfloat16, or float32");
+  if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_len <= 0 || k_len <= 0)
+    return fail("risa_attention: extents must be positive");
+  // (the output's alignment rule is checked once, by the launcher)
+  risa::AttentionArgs a{};
+  a.q = static_cast<const int8_t*>(q_int8);
+  a.k = static_cast<const int8_t*>(k_int8);
+  a.v = static_cast<const int8_t*>(v_int8);
+  a.out = out;
+  a.q_scale = q_scale;
+  a.k_scale = k_scale;
+  a.v_scale = v_scale;
+  a.v_center = v_center;
+  a.v_tile_sum = v_tile_sum;
+  a.mask = mask;
+  a.mask_stride_b = mask_stride_b;
+  a.mask_stride_h = mask_stride_h;
+  a.mask_stride_q = mask_stride_q;
+  a.mask_stride_k = mask_stride_k;
+  a.mask_dtype = mask_dtype;
+  a.cta_k = cta_k;
+  a.batch = batch;
+  a.q_len = q_len;
+  a.k_len = k_len;
+  a.q_heads = q_heads;
+  a.kv_heads = kv_heads;
+  a.head_dim = head_dim;
+  a.out_stride_b = out_stride_b;
+  a.out_stride_n = out_stride_n;
+  a.out_stride_h = out_stride_h;
+  a.sm_scale = sm_scale;
+  a.out_dtype = out_dtype;
+  a.sparse_row_offsets = sparse_row_offsets;
+  a.sparse_block_indices = sparse_block_indices;
+  a.block_mass = block_mass;
+  a.is_causal = is_causal != 0;
+  a.lse = lse;
+  a.lse_shift = lse_shift;
+  a.key_mask_tiles = key_mask_tiles;
+  if (key_bias != nullptr && (mask == nullptr || mask_stride_q != 0))
+    return fail("risa_attention: a key bias row goes with a key-only mask (query stride 0)");
+  a.key_bias = key_bias;
+  a.key_bias_stride_b = key_bias_stride_b;
+  a.key_bias_stride_h = key_bias_stride_h;
+  if (mask_lanes != nullptr && mask == nullptr)
+    return fail("risa_attention: lane words go with the boolean mask they were made from");
+  a.mask_lanes = mask_lanes;
+  a.mask_lanes_stride_b = mask_lanes_stride_b;
+  a.mask_lanes_stride_h = mask_lanes_stride_h;
+  // whole tiles of K may be copied where the bytes behind the last key can be read
+  a.whole_key_tiles = k_bytes >= (static_cast<int64_t>(batch) * kv_heads * k_len + cta_k) * head_dim;
+  a.split_workspace = split_workspace;
+  a.split_workspace_bytes = split_workspace_bytes;
+  return risa::launch_attention(a, static_cast<hipStream_t>(stream));
+}
+
+}  // namespace
+
 extern "C" {
 
 const char* risa_last_error(void) { return risa::last_error_storage().c_str(); }
@@ -310,63 +388,7 @@ int risa_attention_split(const void* q_int8, const void* k_int8, const void* v_i
                    const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
                    int64_t mask_lanes_stride_h, int64_t k_bytes, void* split_workspace,
                    size_t split_workspace_bytes, void* stream) {
-  using risa::fail;
-  if (out_dtype != 1 && out_dtype != 2)
-    return fail("risa_attention: output dtype code must be 1 (fp16) or 2 (bf16)");
-  if (mask != nullptr && (mask_dtype < 0 || mask_dtype > 3))
-    return fail("risa_attention: attention mask must be bool, float16, bfloat16, or float32");
-  if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_len <= 0 || k_len <= 0)
-    return fail("risa_attention: extents must be positive");
-  // (the output's alignment rule is checked once, by the launcher)
-  risa::AttentionArgs a{};
-  a.q = static_cast<const int8_t*>(q_int8);
-  a.k = static_cast<const int8_t*>(k_int8);
-  a.v = static_cast<const int8_t*>(v_int8);
-  a.out = out;
-  a.q_scale = q_scale;
-  a.k_scale = k_scale;
-  a.v_scale = v_scale;
-  a.v_center = v_center;
-  a.v_tile_sum = v_tile_sum;
-  a.mask = mask;
-  a.mask_stride_b = mask_stride_b;
-  a.mask_stride_h = mask_stride_h;
-  a.mask_stride_q = mask_stride_q;
-  a.mask_stride_k = mask_stride_k;
-  a.mask_dtype = mask_dtype;
-  a.cta_k = cta_k;
-  a.batch = batch;
-  a.q_len = q_len;
-  a.k_len = k_len;
-  a.q_heads = q_heads;
-  a.kv_heads = kv_heads;
-  a.head_dim = head_dim;
-  a.out_stride_b = out_stride_b;
-  a.out_stride_n = out_stride_n;
-  a.out_stride_h = out_stride_h;
-  a.sm_scale = sm_scale;
-  a.out_dtype = out_dtype;
-  a.sparse_row_offsets = sparse_row_offsets;
-  a.sparse_block_indices = sparse_block_indices;
-  a.block_mass = block_mass;
-  a.is_causal = is_causal != 0;
-  a.lse = lse;
-  a.key_mask_tiles = key_mask_tiles;
-  if (key_bias != nullptr && (mask == nullptr || mask_stride_q != 0))
-    return fail("risa_attention: a key bias row goes with a key-only mask (query stride 0)");
-  a.key_bias = key_bias;
-  a.key_bias_stride_b = key_bias_stride_b;
-  a.key_bias_stride_h = key_bias_stride_h;
-  if (mask_lanes != nullptr && mask == nullptr)
-    return fail("risa_attention: lane words go with the boolean mask they were made from");
-  a.mask_lanes = mask_lanes;
-  a.mask_lanes_stride_b = mask_lanes_stride_b;
-  a.mask_lanes_stride_h = mask_lanes_stride_h;
-  // whole tiles of K may be copied where the bytes behind the last key can be read
-  a.whole_key_tiles = k_bytes >= (static_cast<int64_t>(batch) * kv_heads * k_len + cta_k) * head_dim;
-  a.split_workspace = split_workspace;
-  a.split_workspace_bytes = split_workspace_bytes;
-  return risa::launch_attention(a, static_cast<hipStream_t>(stream));
+  return attend(q_int8, k_int8, v_int8, out, q_scale, k_scale, v_scale, v_center, v_tile_sum, mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, cta_k, batch, q_len, k_len, q_heads, kv_heads, head_dim, out_stride_b, out_stride_n, out_stride_h, sm_scale, out_dtype, sparse_row_offsets, sparse_block_indices, block_mass, is_causal, lse, nullptr, key_mask_tiles, key_bias, key_bias_stride_b, key_bias_stride_h, mask_lanes, mask_lanes_stride_b, mask_lanes_stride_h, k_bytes, split_workspace, split_workspace_bytes, stream);
 }
 
 int risa_attention_readable_keys(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
@@ -560,7 +582,7 @@ size_t risa_sdpa_workspace_bytes(int batch, int q_heads, int q_len, int kv_heads
          risa_attention_split_bytes(batch, q_heads, q_len, k_len, head_dim, cta_k, mask_dtype, mask_stride_q);
 }
 
-int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, void* workspace,
+int risa_sdpa_lse(const void* q, const void* k, const void* v, void* out, void* workspace,
               size_t workspace_bytes, int batch, int q_heads, int q_len, int kv_heads, int k_len,
               int head_dim, int cta_k, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
               int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b,
@@ -569,7 +591,7 @@ int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, v
               int midpoint_affine, const void* mask, int64_t mask_stride_b, int64_t mask_stride_h,
               int64_t mask_stride_q, int64_t mask_stride_k, int mask_dtype, int mask_batch,
               int mask_heads, int is_causal, const int32_t* sparse_row_offsets,
-              const int32_t* sparse_block_indices, int channels, void* stream) {
+              const int32_t* sparse_block_indices, int channels, float* lse, void* stream) {
   using risa::fail;
   if (batch <= 0 || q_heads <= 0 || q_len <= 0 || kv_heads <= 0 || k_len <= 0 ||
       (cta_k != 64 && cta_k != 128))
@@ -618,6 +640,14 @@ int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, v
     if (status == 0) status = risa::launch_quantize_v(value, hip_stream);
   }
   if (status != 0) return status;
+  if (lse != nullptr) {
+    // what the anchor took off the logits goes where the attention kernel adds its own term to it
+    const risa::LseShiftArgs shift{q, k, reinterpret_cast<const int32_t*>(base + l.anchors), lse, batch, q_heads, kv_heads,
+                                   q_len, channels, input_dtype, q_stride_b, q_stride_h, q_stride_n, k_stride_b,
+                                   k_stride_h, k_stride_n, sm_scale};
+    status = risa::launch_lse_shift(shift, hip_stream);
+    if (status != 0) return status;
+  }
   const float* key_bias = nullptr;
   const int32_t* key_tiles = nullptr;
   int64_t bias_stride_b = 0, bias_stride_h = 0;
@@ -649,14 +679,27 @@ int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, v
   }
   // (behind the K codes lie those of V, a whole key tile at least; behind the sections the partial results
   // of key ranges, where the workspace is as large as risa_sdpa_workspace_bytes says)
-  return risa_attention_split(base + l.q_codes, base + l.k_codes, base + l.v_codes, out, q_scale, k_scale,
+  return attend(base + l.q_codes, base + l.k_codes, base + l.v_codes, out, q_scale, k_scale,
                         v_scale, v_center, tile_sum, mask, mask_stride_b, mask_stride_h,
                         mask_stride_q, mask_stride_k, mask_dtype, cta_k, batch, q_len, k_len,
                         q_heads, kv_heads, head_dim, out_stride_b, out_stride_n, out_stride_h,
                         sm_scale, output_dtype, sparse_row_offsets, sparse_block_indices, nullptr,
-                        is_causal, nullptr, key_tiles, key_bias, bias_stride_b, bias_stride_h,
+                        is_causal, lse, lse, key_tiles, key_bias, bias_stride_b, bias_stride_h,
                         mask_lanes, lanes_stride_b, lanes_stride_h, static_cast<int64_t>(l.bytes - l.k_codes),
                         base + l.bytes, workspace_bytes - l.bytes, stream);
+}
+
+int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, void* workspace,
+              size_t workspace_bytes, int batch, int q_heads, int q_len, int kv_heads, int k_len,
+              int head_dim, int cta_k, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
+              int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b,
+              int64_t v_stride_h, int64_t v_stride_n, int64_t out_stride_b, int64_t out_stride_n,
+              int64_t out_stride_h, float sm_scale, int input_dtype, int output_dtype,
+              int midpoint_affine, const void* mask, int64_t mask_stride_b, int64_t mask_stride_h,
+              int64_t mask_stride_q, int64_t mask_stride_k, int mask_dtype, int mask_batch,
+              int mask_heads, int is_causal, const int32_t* sparse_row_offsets,
+              const int32_t* sparse_block_indices, int channels, void* stream) {
+  return risa_sdpa_lse(q, k, v, out, workspace, workspace_bytes, batch, q_heads, q_len, kv_heads, k_len, head_dim, cta_k, q_stride_b, q_stride_h, q_stride_n, k_stride_b, k_stride_h, k_stride_n, v_stride_b, v_stride_h, v_stride_n, out_stride_b, out_stride_n, out_stride_h, sm_scale, input_dtype, output_dtype, midpoint_affine, mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, mask_batch, mask_heads, is_causal, sparse_row_offsets, sparse_block_indices, channels, nullptr, stream);
 }
 
 int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* workspace,

@@ -17,9 +17,10 @@ from .prepare import prequantize_int8_attention
 OP_NAMESPACE = "risa_attention"
 
 
-def _run(q, k, v, attn_mask, scale, use_midpoint_affine, is_causal):
+def _run(q, k, v, attn_mask, scale, use_midpoint_affine, is_causal, return_lse=False):
     return execute_dense_attention(q, k, v, scale=scale, attn_mask=attn_mask,
-                                   use_midpoint_affine=use_midpoint_affine, is_causal=is_causal)
+                                   use_midpoint_affine=use_midpoint_affine, is_causal=is_causal,
+                                   return_lse=return_lse)
 
 
 def _same_shape_as_query(q, *unused):
@@ -83,9 +84,10 @@ def int8_attention(
     (taken from the same rounded U8 probabilities as P·V) and V dequantisation
     are FP32.  ``return_lse=True`` also returns natural-log normalisers.
     """
-    needs_packed_route = return_lse or kv_permutation is not None
-    if needs_packed_route:
-        # the LSE and the permuted order live in the packed container
+    # The permuted order lives in the packed container, and so do the log-normalisers of traced and
+    # wrapped tensors: the registered operators return the output alone.
+    plain = _plain_eager(q, k, v, attn_mask)
+    if kv_permutation is not None or (return_lse and not plain):
         packed = prequantize_int8_attention(
             q, k, v, scale=scale, attn_mask=attn_mask, v_quantization=v_quantization,
             is_causal=is_causal, return_lse=return_lse, kv_permutation=kv_permutation,
@@ -96,8 +98,8 @@ def int8_attention(
     # Plain eager tensors skip the operator dispatch (about 10 us per call, a third of a
     # short sequence's whole step); tracing, fake and wrapped tensors go through the
     # registered operators so that torch.compile sees them.
-    if _plain_eager(q, k, v, attn_mask):
-        return _run(q, k, v, attn_mask, scale, centered, is_causal)
+    if plain:
+        return _run(q, k, v, attn_mask, scale, centered, is_causal, return_lse)
     operators = getattr(torch.ops, OP_NAMESPACE)
     if attn_mask is None:
         return operators.int8_attention(q, k, v, scale, centered, is_causal)
