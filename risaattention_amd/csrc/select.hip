@@ -306,9 +306,11 @@ void launch_key_mask_kernel(const KeyMaskArgs& a, int dtype, hipStream_t stream)
 // regrouping of 32-bit scalar registers.  Lane s keeps word s, so the 32 words of a tile
 // leave in one 256-byte store.
 constexpr int kLaneTilesPerWave = 4;
-// A wave-uniform 32-bit value written into one lane of a vector register.
+// A wave-uniform 32-bit value written into one lane of a vector register.  The value comes from a vector
+// comparison, and a vector instruction may read such a scalar register two wait states later: the compiler
+// counts them for its own instructions only, so they stand in front of this one.
 __device__ __forceinline__ void write_lane(uint32_t& target, uint32_t uniform_value, int lane_index) {
-  asm("v_writelane_b32 %0, %1, %2" : "+v"(target) : "s"(uniform_value), "n"(lane_index));
+  asm("s_nop 1\n\tv_writelane_b32 %0, %1, %2" : "+v"(target) : "s"(uniform_value), "n"(lane_index));
 }
 template <bool ALIGNED>
 __global__ __launch_bounds__(256) void mask_lanes_kernel(const uint8_t* __restrict__ mask,
