@@ -246,14 +246,15 @@ def execute_dense_attention(
         sdpa_workspace_bytes(batch, q_heads, q_len, kv_heads, k_len, dim, cta_k, int(use_midpoint_affine),
                              mask_args[5], mask_args[3], mask_args[4], mask_args[6], mask_args[7]),
         dtype=torch.uint8, device=q.device)
+    call, lse_args = (lib.risa_sdpa_lse, (lse.data_ptr(),)) if return_lse else (lib.risa_sdpa_channels, ())
     native.check(
-        lib.risa_sdpa_lse(
+        call(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), output.data_ptr(), workspace.data_ptr(),
             workspace.numel(), batch, q_heads, q_len, kv_heads, k_len, dim, cta_k,
             q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
             v.stride(0), v.stride(1), v.stride(2), output.stride(0), output.stride(2), output.stride(1),
             attention_scale, DTYPE_CODES[input_dtype], DTYPE_CODES[output.dtype],
-            int(use_midpoint_affine), *mask_args, int(bool(is_causal)), *csr, q.shape[-1], native.pointer(lse),
+            int(use_midpoint_affine), *mask_args, int(bool(is_causal)), *csr, q.shape[-1], *lse_args,
             native.current_stream(q.device),
         )
     )

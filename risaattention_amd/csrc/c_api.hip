@@ -335,7 +335,7 @@ int risa_sdpa_quantize_channels(const void* q, void* q_int8, float* q_scale, con
                           v_stride_n, input_dtype, midpoint_affine, kv_permutation);
   if (status != 0) return status;
   hipStream_t hip_stream = static_cast<hipStream_t>(stream);
-  if (risa::can_prepare_fused(qk, value)) return risa::launch_prepare_fused(qk, value, hip_stream);
+  if (risa::can_prepare_fused(qk, value)) return risa::launch_prepare_fused(qk, value, {}, hip_stream);
   if (channels != head_dim)
     return risa::fail("risa_sdpa_quantize: rows of fewer channels than head_dim need the fused preparation");
   status = risa::launch_quantize_qk(qk, hip_stream);
@@ -505,8 +505,11 @@ int risa_prepare_mask_lanes(const void* mask, uint64_t* lanes, int mask_batch, i
   if (mask == nullptr || lanes == nullptr || mask_batch <= 0 || mask_heads <= 0 || q_len <= 0 || k_len <= 0)
     return risa::fail("risa_prepare_mask_lanes: bad extents");
   if (!aligned(lanes, 8)) return risa::fail("risa_prepare_mask_lanes: lane words must be 8-byte aligned");
-  return risa::launch_mask_lanes(mask, lanes, mask_batch, mask_heads, q_len, k_len,
-                                 mask_batch > 1 ? stride_b : 0, mask_heads > 1 ? stride_h : 0, stride_q,
+  if ((static_cast<int64_t>(q_len) + 127) / 128 * 4 > 65535 || static_cast<int64_t>(mask_batch) * mask_heads > 65535)
+    return risa::fail("risa_prepare_mask_lanes: more query blocks or mask planes than one launch covers");
+  return risa::launch_mask_lanes(risa::mask_lane_args(mask, lanes, mask_batch, mask_heads, q_len, k_len,
+                                                      mask_batch > 1 ? stride_b : 0, mask_heads > 1 ? stride_h : 0,
+                                                      stride_q),
                                  static_cast<hipStream_t>(stream));
 }
 
@@ -631,23 +634,12 @@ int risa_sdpa_lse(const void* q, const void* k, const void* v, void* out, void* 
                           midpoint_affine, nullptr);
   if (status != 0) return status;
   hipStream_t hip_stream = static_cast<hipStream_t>(stream);
-  if (risa::can_prepare_fused(qk, value)) {
-    status = risa::launch_prepare_fused(qk, value, hip_stream);
-  } else if (channels != head_dim) {
-    return fail("risa_sdpa: rows of fewer channels than head_dim need the fused preparation");
-  } else {
-    status = risa::launch_quantize_qk(qk, hip_stream);
-    if (status == 0) status = risa::launch_quantize_v(value, hip_stream);
-  }
-  if (status != 0) return status;
-  if (lse != nullptr) {
-    // what the anchor took off the logits goes where the attention kernel adds its own term to it
-    const risa::LseShiftArgs shift{q, k, reinterpret_cast<const int32_t*>(base + l.anchors), lse, batch, q_heads, kv_heads,
-                                   q_len, channels, input_dtype, q_stride_b, q_stride_h, q_stride_n, k_stride_b,
-                                   k_stride_h, k_stride_n, sm_scale};
-    status = risa::launch_lse_shift(shift, hip_stream);
-    if (status != 0) return status;
-  }
+  // The forms of the mask that the attention kernel reads, and what the anchor takes off the logits (it
+  // goes where the attention kernel adds its own term to it), ride in the launches of the preparation.
+  risa::PrepareRiders riders{};
+  risa::KeyMaskArgs key_mask{};
+  risa::MaskLaneArgs lanes{};
+  risa::LseShiftArgs shift{};
   const float* key_bias = nullptr;
   const int32_t* key_tiles = nullptr;
   int64_t bias_stride_b = 0, bias_stride_h = 0;
@@ -655,9 +647,9 @@ int risa_sdpa_lse(const void* q, const void* k, const void* v, void* out, void* 
   int64_t lanes_stride_b = 0, lanes_stride_h = 0;
   if (lanes_bytes != 0) {
     auto* words = reinterpret_cast<uint64_t*>(base + l.mask_lanes);
-    status = risa_prepare_mask_lanes(mask, words, mask_batch, mask_heads, q_len, k_len, mask_stride_b,
-                                     mask_stride_h, mask_stride_q, stream);
-    if (status != 0) return status;
+    lanes = risa::mask_lane_args(mask, words, mask_batch, mask_heads, q_len, k_len, mask_batch > 1 ? mask_stride_b : 0,
+                                 mask_heads > 1 ? mask_stride_h : 0, mask_stride_q);
+    riders.lanes = &lanes;
     mask_lanes = words;
     const int64_t plane = static_cast<int64_t>(risa::mask_lane_words(1, 1, q_len, k_len));
     lanes_stride_h = mask_heads > 1 ? plane : 0;
@@ -672,11 +664,20 @@ int risa_sdpa_lse(const void* q, const void* k, const void* v, void* out, void* 
     const bool lists = k_len > 1024 && q_len >= 256 && sm_scale > 0.0f && is_causal == 0 && sparse_row_offsets == nullptr;
     if (mask_dtype < 0 || mask_dtype > 3) return fail("risa_sdpa: attention mask must be bool, float16, bfloat16, or float32");
     auto* list = lists ? reinterpret_cast<int32_t*>(base + l.key_tiles) : nullptr;
-    status = risa::launch_key_mask(mask, list, bias, batch, q_heads, mask_batch, mask_heads, k_len, padded, cta_k,
-                                   mask_stride_b, mask_stride_h, mask_stride_k, mask_dtype, hip_stream);
-    if (status != 0) return status;
+    key_mask = risa::key_mask_args(mask, list, bias, batch, q_heads, mask_batch, mask_heads, k_len, padded, cta_k,
+                                   mask_stride_b, mask_stride_h, mask_stride_k);
+    riders.key_mask = &key_mask;
+    riders.key_mask_dtype = mask_dtype;
     key_tiles = list;
   }
+  if (lse != nullptr) {
+    shift = {q, k, reinterpret_cast<const int32_t*>(base + l.anchors), lse, batch, q_heads, kv_heads, q_len, channels,
+             input_dtype, q_stride_b, q_stride_h, q_stride_n, k_stride_b, k_stride_h, k_stride_n, sm_scale};
+    riders.shift = &shift;
+  }
+  if (!risa::can_prepare_fused(qk, value)) return fail("risa_sdpa: operands do not qualify for the fused preparation");
+  status = risa::launch_prepare_fused(qk, value, riders, hip_stream);
+  if (status != 0) return status;
   // (behind the K codes lie those of V, a whole key tile at least; behind the sections the partial results
   // of key ranges, where the workspace is as large as risa_sdpa_workspace_bytes says)
   return attend(base + l.q_codes, base + l.k_codes, base + l.v_codes, out, q_scale, k_scale,

@@ -127,10 +127,6 @@ int launch_key_mask_tiles(const void* mask, int32_t* tiles, int batch, int heads
                           int tile_size, int64_t stride_b, int64_t stride_h, int64_t stride_k,
                           int dtype, hipStream_t stream);
 
-// Q/K/V preparation in two launches (short sequences, no permutation).
-bool can_prepare_fused(const QkArgs& qk, const ValueArgs& v);
-int launch_prepare_fused(const QkArgs& qk, const ValueArgs& v, hipStream_t stream);
-
 // Lane words of a boolean mask with 64-key tiles: [batch, heads, ceil(q_len/128)*4,
 // ceil(k_len/64), 32] 64-bit words, batch and heads being the mask's own extents.
 // What the 32 lane words of one (block of 32 queries, 64-key tile) have in common: every bit
@@ -140,16 +136,51 @@ constexpr int kLaneTileMixed = 0, kLaneTileVisible = 1, kLaneTileHidden = 2;
 size_t mask_lane_words(int batch, int heads, int q_len, int k_len);
 size_t mask_lane_bytes(int batch, int heads, int q_len, int k_len);  // words, classes and tile lists
 size_t mask_tile_list_offset(int batch, int heads, int q_len, int k_len);  // of the lists, in bytes
-int launch_mask_lanes(const void* mask, uint64_t* lanes, int batch, int heads, int q_len, int k_len,
-                      int64_t stride_b, int64_t stride_h, int64_t stride_q, hipStream_t stream);
+struct MaskLaneArgs {
+  const uint8_t* mask;
+  uint64_t* lanes;
+  int32_t* classes;  // one per 32 lane words
+  int32_t* lists;    // [planes][query_waves / 4][key_tiles + 1]
+  int heads, planes, q_len, k_len, key_tiles, query_waves;
+  int64_t stride_b, stride_h, stride_q;
+  bool aligned;  // sixteen mask bytes a load
+};
+MaskLaneArgs mask_lane_args(const void* mask, uint64_t* lanes, int batch, int heads, int q_len, int k_len,
+                            int64_t stride_b, int64_t stride_h, int64_t stride_q);
+int launch_mask_lanes(const MaskLaneArgs& args, hipStream_t stream);
 
-// Both of one key-only mask in one launch; `tiles` may be null.
-int launch_key_mask(const void* mask, int32_t* tiles, float* bias, int batch, int heads, int mask_batch,
-                    int mask_heads, int length, int padded, int tile_size, int64_t stride_b,
-                    int64_t stride_h, int64_t stride_k, int dtype, hipStream_t stream);
+// Both derived forms of a key-only mask in one launch: the list of tiles with a visible key per
+// (batch, head), and the additive row in the exp2 domain per mask plane (bias * log2(e), the FP32
+// product the attention kernel would form per score; -inf for hidden and out-of-range keys).
+// Either output may be null.
+struct KeyMaskArgs {
+  const void* mask;
+  int32_t* tiles;  // [batch, heads, tiles + 1]
+  float* bias;     // [bias_planes, padded]
+  int batch, heads, bias_heads, bias_planes, length, tile_size, padded;
+  int64_t stride_b, stride_h, stride_k;            // of the mask as the lists see it (0: shared)
+  int64_t bias_stride_b, bias_stride_h;
+};
+KeyMaskArgs key_mask_args(const void* mask, int32_t* tiles, float* bias, int batch, int heads, int mask_batch,
+                          int mask_heads, int length, int padded, int tile_size, int64_t stride_b,
+                          int64_t stride_h, int64_t stride_k);
+int launch_key_mask(const KeyMaskArgs& args, int dtype, hipStream_t stream);
 
 int launch_key_bias(const void* mask, float* bias, int batch, int heads, int length, int padded,
                     int64_t stride_b, int64_t stride_h, int64_t stride_k, int dtype,
                     hipStream_t stream);
+
+// What rides in the launches of the fused preparation (null: nothing of the kind): the derived forms of
+// a mask and the LSE shift, neither of which needs a launch of its own there.
+struct PrepareRiders {
+  const KeyMaskArgs* key_mask;
+  int key_mask_dtype;
+  const MaskLaneArgs* lanes;
+  const LseShiftArgs* shift;
+};
+
+// Q/K/V preparation in one to three launches.
+bool can_prepare_fused(const QkArgs& qk, const ValueArgs& v);
+int launch_prepare_fused(const QkArgs& qk, const ValueArgs& v, const PrepareRiders& riders, hipStream_t stream);
 
 }  // namespace risa

@@ -9,12 +9,12 @@ bool can_prepare_fused(const QkArgs& qk, const ValueArgs& v) {
          qk.cta_k == v.cta_k && qk.dtype == v.dtype;
 }
 
-int launch_prepare_fused(const QkArgs& qk, const ValueArgs& v, hipStream_t stream) {
+int launch_prepare_fused(const QkArgs& qk, const ValueArgs& v, const PrepareRiders& riders, hipStream_t stream) {
   if (!can_prepare_fused(qk, v)) return fail("risa_sdpa: operands do not qualify for the fused preparation");
   if (v.workspace_bytes < value_workspace_bytes(v.batch, v.heads, v.length, v.head_dim, v.midpoint_affine))
     return fail("risa_quantize_v: workspace is too small");
   const Workspace w = carve(v.workspace, v.batch, v.heads, v.length, v.head_dim, v.midpoint_affine);
-  FusedArgs a{};
+  FusedRiders a{};
   a.qk = qk;
   a.v = v;
   a.part_max = w.part_max;
@@ -41,11 +41,42 @@ int launch_prepare_fused(const QkArgs& qk, const ValueArgs& v, hipStream_t strea
   a.code_blocks_x = (v.padded + kCodeBlockPositions - 1) / kCodeBlockPositions;
   a.q_wide = rows_are_16_byte_aligned(qk.q, qk.q_stride_b, qk.q_stride_h, qk.q_stride_n, qk.dtype);
   a.k_wide = rows_are_16_byte_aligned(qk.k, qk.k_stride_b, qk.k_stride_h, qk.k_stride_n, qk.dtype);
+  // Riders.  (The flags of a key list are LDS of every workgroup of the launch, so long rows get a
+  // launch of their own: 4 KB, 262144 keys, take no workgroup from a compute unit.)
+  const bool key_mask_rides = riders.key_mask != nullptr && key_mask_flag_bytes(*riders.key_mask) <= 4096;
+  if (key_mask_rides) {
+    a.key_mask = *riders.key_mask;
+    a.key_mask_dtype = riders.key_mask_dtype;
+    a.key_mask_blocks = key_mask_blocks(a.key_mask);
+    a.key_mask_flag_bytes = static_cast<int>(key_mask_flag_bytes(a.key_mask));
+  }
+  const bool second_launch = !one_launch(a);
+  // (lane words where the mask is read sixteen bytes at a time; the tile lists need the words first)
+  const bool lanes_ride = riders.lanes != nullptr && second_launch && riders.lanes->aligned;
+  if (lanes_ride) {
+    a.lanes = *riders.lanes;
+    a.lane_groups = mask_lane_groups(a.lanes);
+    a.lane_blocks = a.lane_groups * a.lanes.query_waves * a.lanes.planes;
+    a.list_blocks = (a.lanes.query_waves / 4 * a.lanes.planes + 3) / 4;
+  }
+  const bool masked = a.key_mask_blocks != 0 || a.lane_blocks != 0;
+  const bool shift_rides = riders.shift != nullptr && second_launch && masked;
+  if (shift_rides) {
+    a.shift = *riders.shift;
+    a.shift_rows = lse_shift_rows(a.shift);
+    a.shift_blocks_x = lse_shift_blocks(a.shift, a.shift_rows);
+    a.shift_blocks = a.shift_blocks_x * a.shift.q_heads * a.shift.batch;
+  }
   if (qk.channels != qk.head_dim)
-    launch_prepare_padded(a, stream);
+    (masked ? launch_prepare_padded_masked : launch_prepare_padded)(a, stream);
   else
-    launch_by_type<false>(a, stream);
-  return check_launch("risa_sdpa preparation");
+    (masked ? launch_prepare_masked : launch_by_type<false, false>)(a, stream);
+  int status = check_launch("risa_sdpa preparation");
+  if (status == 0 && riders.key_mask != nullptr && !key_mask_rides)
+    status = launch_key_mask(*riders.key_mask, riders.key_mask_dtype, stream);
+  if (status == 0 && riders.lanes != nullptr && !lanes_ride) status = launch_mask_lanes(*riders.lanes, stream);
+  if (status == 0 && riders.shift != nullptr && !shift_rides) status = launch_lse_shift(*riders.shift, stream);
+  return status;
 }
 
 }  // namespace risa

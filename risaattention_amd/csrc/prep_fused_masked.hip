@@ -1,0 +1,9 @@
+// Fused preparation with the derived forms of a mask in its first launch (a translation unit of its own,
+// compiled beside prep_fused.hip).
+#include "prep_fused_kernels.hpp"
+
+namespace risa {
+
+void launch_prepare_masked(const FusedRiders& a, hipStream_t stream) { launch_by_type<false, true>(a, stream); }
+
+}  // namespace risa

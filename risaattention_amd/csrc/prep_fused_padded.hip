@@ -6,6 +6,6 @@
 
 namespace risa {
 
-void launch_prepare_padded(const FusedArgs& a, hipStream_t stream) { launch_by_type<true>(a, stream); }
+void launch_prepare_padded(const FusedRiders& a, hipStream_t stream) { launch_by_type<true, false>(a, stream); }
 
 }  // namespace risa

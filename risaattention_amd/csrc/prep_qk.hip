@@ -75,70 +75,16 @@ int launch_quantize_qk(const QkArgs& a, hipStream_t stream) {
   return check_launch("risa_quantize_qk");
 }
 
-// ---------------------------------------------------------------------------
-// LSE anchor correction: out[b,h,i] = scale * <q[b,h,i], k[b,h/G,anchor]>,
-// products and sums kept separate, lanes stride 32 over channels, shuffle-down
-// tree (reference csrc/kernels/lse_correction.cu:4-28).
-// grid (ceil(Lq/8), Hq, B), 256 threads: one 32-lane half per query row.
-// ---------------------------------------------------------------------------
 namespace {
-// kShiftRows rows per half wavefront, loads of all of them in flight: eight (one took 17 us for 48
-// heads x 4096 x 64 in 16 bits, 2.9 TB/s; eight take 5.3), but one for launches of up to four
-// workgroups per compute unit, where eight rows are a longer chain than one and leave wavefronts out
-// (16 heads x 64 x 128 3.3 us with eight, 2.5 with one; x 512 3.3 and 3.2; x 768 3.3 and 3.7).
-template <int DT, int kShiftRows>
-__global__ __launch_bounds__(256) void lse_shift_kernel(const void* __restrict__ q,
-                                                        const void* __restrict__ k,
-                                                        const int* __restrict__ anchors,
-                                                        float* __restrict__ out, int q_heads,
-                                                        int kv_heads, int q_len, int dim,
-                                                        int64_t qb, int64_t qh, int64_t qn,
-                                                        int64_t kb, int64_t kh, int64_t kn,
-                                                        float scale) {
-  const int sub = threadIdx.x & 31;
-  const int first_row = (blockIdx.x * 8 + (threadIdx.x >> 5)) * kShiftRows;
-  const int head = blockIdx.y, batch = blockIdx.z;
-  if (first_row >= q_len) return;
-  const int kv_head = head / (q_heads / kv_heads);
-  const int anchor = anchors[batch * kv_heads + kv_head];
-  float sum[kShiftRows];
-#pragma unroll
-  for (int i = 0; i < kShiftRows; ++i) sum[i] = 0.0f;
-  if (anchor >= 0) {
-    const int64_t q_base = batch * qb + head * qh;
-    const int64_t k_base = batch * kb + kv_head * kh + static_cast<int64_t>(anchor) * kn;
-#pragma unroll 2
-    for (int d = sub; d < dim; d += 32) {
-      const float key = load1<DT>(k, k_base + d);
-      float query[kShiftRows];
-#pragma unroll
-      for (int i = 0; i < kShiftRows; ++i)  // (rows past the end read the last one)
-        query[i] = load1<DT>(q, q_base + static_cast<int64_t>(min(first_row + i, q_len - 1)) * qn + d);
-#pragma unroll
-      for (int i = 0; i < kShiftRows; ++i) {
-        const float product = query[i] * key;
-        sum[i] = sum[i] + product;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kShiftRows; ++i) sum[i] = segment_down_sum(sum[i]);
-  }
-  float mine = sum[0];
-#pragma unroll
-  for (int i = 1; i < kShiftRows; ++i) mine = sub == i ? sum[i] : mine;
-  if (sub < kShiftRows && first_row + sub < q_len)
-    out[(static_cast<int64_t>(batch) * q_heads + head) * q_len + first_row + sub] = mine * scale;
+template <int DT, int kShiftRows> __global__ __launch_bounds__(256) void lse_shift_kernel(const LseShiftArgs a) {
+  lse_shift_block<DT, kShiftRows>(a, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 }  // namespace
 
 int launch_lse_shift(const LseShiftArgs& a, hipStream_t stream) {
-  const int64_t small = static_cast<int64_t>((a.q_len + 7) / 8) * a.q_heads * a.batch;
-  const int rows = small <= 4 * static_cast<int64_t>(narrow_attention_limit()) ? 1 : 8;
-  dim3 grid((a.q_len + 8 * rows - 1) / (8 * rows), a.q_heads, a.batch);
-#define RISA_LSE(DTV)                                                                             \
-  (rows == 1 ? lse_shift_kernel<DTV, 1> : lse_shift_kernel<DTV, 8>)<<<grid, 256, 0, stream>>>(     \
-      a.q, a.k, a.anchors, a.out, a.q_heads, a.kv_heads, a.q_len, a.head_dim, a.q_stride_b,        \
-      a.q_stride_h, a.q_stride_n, a.k_stride_b, a.k_stride_h, a.k_stride_n, a.scale)
+  const int rows = lse_shift_rows(a);
+  dim3 grid(lse_shift_blocks(a, rows), a.q_heads, a.batch);
+#define RISA_LSE(DTV) (rows == 1 ? lse_shift_kernel<DTV, 1> : lse_shift_kernel<DTV, 8>)<<<grid, 256, 0, stream>>>(a)
   if (a.dtype == kF32)
     RISA_LSE(kF32);
   else if (a.dtype == kF16)

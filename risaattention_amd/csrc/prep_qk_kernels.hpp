@@ -591,5 +591,58 @@ inline int rows_are_16_byte_aligned(const void* base, int64_t stride_b, int64_t 
   return reinterpret_cast<uintptr_t>(base) % 16 == 0 && ((stride_b | stride_h | stride_n) & 7) == 0;
 }
 
+// ---------------------------------------------------------------------------
+// LSE anchor correction: out[b,h,i] = scale * <q[b,h,i], k[b,h/G,anchor]>,
+// products and sums kept separate, lanes stride 32 over channels, shuffle-down
+// tree (reference csrc/kernels/lse_correction.cu:4-28).
+// One workgroup per 8 (64) query rows of a head, 256 threads.
+// ---------------------------------------------------------------------------
+// kShiftRows rows per half wavefront, loads of all of them in flight: eight (one took 17 us for 48
+// heads x 4096 x 64 in 16 bits, 2.9 TB/s; eight take 5.3), but one for launches of up to four
+// workgroups per compute unit, where eight rows are a longer chain than one and leave wavefronts out
+// (16 heads x 64 x 128 3.3 us with eight, 2.5 with one; x 512 3.3 and 3.2; x 768 3.3 and 3.7).
+template <int DT, int kShiftRows>
+__device__ __forceinline__ void lse_shift_block(const LseShiftArgs& a, int block, int head, int batch) {
+  const int q_len = a.q_len, dim = a.head_dim;
+  const int sub = threadIdx.x & 31;
+  const int first_row = (block * 8 + (threadIdx.x >> 5)) * kShiftRows;
+  if (first_row >= q_len) return;
+  const int kv_head = head / (a.q_heads / a.kv_heads);
+  const int anchor = a.anchors[batch * a.kv_heads + kv_head];
+  float sum[kShiftRows];
+#pragma unroll
+  for (int i = 0; i < kShiftRows; ++i) sum[i] = 0.0f;
+  if (anchor >= 0) {
+    const int64_t q_base = batch * a.q_stride_b + head * a.q_stride_h;
+    const int64_t k_base = batch * a.k_stride_b + kv_head * a.k_stride_h + static_cast<int64_t>(anchor) * a.k_stride_n;
+#pragma unroll 2
+    for (int d = sub; d < dim; d += 32) {
+      const float key = load1<DT>(a.k, k_base + d);
+      float query[kShiftRows];
+#pragma unroll
+      for (int i = 0; i < kShiftRows; ++i)  // (rows past the end read the last one)
+        query[i] = load1<DT>(a.q, q_base + static_cast<int64_t>(min(first_row + i, q_len - 1)) * a.q_stride_n + d);
+#pragma unroll
+      for (int i = 0; i < kShiftRows; ++i) {
+        const float product = query[i] * key;
+        sum[i] = sum[i] + product;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kShiftRows; ++i) sum[i] = segment_down_sum(sum[i]);
+  }
+  float mine = sum[0];
+#pragma unroll
+  for (int i = 1; i < kShiftRows; ++i) mine = sub == i ? sum[i] : mine;
+  if (sub < kShiftRows && first_row + sub < q_len)
+    a.out[(static_cast<int64_t>(batch) * a.q_heads + head) * q_len + first_row + sub] = mine * a.scale;
+}
+// Rows per half wavefront (see above) and workgroups per head.
+inline int lse_shift_rows(const LseShiftArgs& a) {
+  const int64_t small = static_cast<int64_t>((a.q_len + 7) / 8) * a.q_heads * a.batch;
+  return small <= 4 * static_cast<int64_t>(narrow_attention_limit()) ? 1 : 8;
+}
+inline int lse_shift_blocks(const LseShiftArgs& a, int rows) { return (a.q_len + 8 * rows - 1) / (8 * rows); }
+
 }  // namespace
 }  // namespace risa

@@ -7,6 +7,7 @@
 
 #include "common.hpp"
 #include "launchers.hpp"
+#include "mask_kernels.hpp"
 
 namespace risa {
 namespace {
@@ -192,93 +193,14 @@ __global__ __launch_bounds__(256) void compact_rows_kernel(const uint8_t* __rest
   }
 }
 
-// Both derived forms of a key-only mask in one launch: the list of tiles with a visible key per
-// (batch, head), and the additive row in the exp2 domain per mask plane (bias * log2(e), the FP32
-// product the attention kernel would form per score; -inf for hidden and out-of-range keys).
-// Either output may be null.
-struct KeyMaskArgs {
-  const void* mask;
-  int32_t* tiles;  // [batch, heads, tiles + 1]
-  float* bias;     // [bias_planes, padded]
-  int batch, heads, bias_heads, bias_planes, length, tile_size, padded;
-  int64_t stride_b, stride_h, stride_k;            // of the mask as the lists see it (0: shared)
-  int64_t bias_stride_b, bias_stride_h;
-};
-
-template <int DT> __device__ __forceinline__ float key_term(const void* mask, int64_t index) {
-  if constexpr (DT == kBool) {
-    return static_cast<const uint8_t*>(mask)[index] != 0 ? 0.0f : -__builtin_inff();
-  } else {
-    return load1<DT>(mask, index);
-  }
-}
-
-// The first batch * heads workgroups (when lists are asked for): flags of 64-key runs, eight loads
-// in flight per thread (one load per tile and wavefront, each waited for, took 10 us for 72
-// tiles), then one wavefront compacts the active tile ids in ascending order and appends the
-// count.  The others: 256 keys of a bias plane each.
 template <int DT> __global__ __launch_bounds__(256) void key_mask_kernel(const KeyMaskArgs a) {
   extern __shared__ unsigned char run_flags[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int rows = a.tiles != nullptr ? a.batch * a.heads : 0;
-  if (static_cast<int>(blockIdx.x) >= rows) {
-    const int per_plane = (a.padded + 255) / 256;
-    const int block = blockIdx.x - rows;
-    const int plane = block / per_plane, key = block % per_plane * 256 + tid;
-    if (key >= a.padded) return;
-    float value = -__builtin_inff();
-    if (key < a.length) {
-      const float term = key_term<DT>(a.mask, plane / a.bias_heads * a.bias_stride_b + plane % a.bias_heads * a.bias_stride_h +
-                                                  key * a.stride_k);
-      if (__builtin_isfinite(term)) value = term * 1.44269504088896340736f;
-    }
-    a.bias[static_cast<int64_t>(plane) * a.padded + key] = value;
-    return;
-  }
-  const int64_t row = blockIdx.x;
-  const int64_t mask_row = row / a.heads * a.stride_b + row % a.heads * a.stride_h;
-  constexpr int IN_FLIGHT = 8;
-  for (int first = 0; first < a.length; first += 256 * IN_FLIGHT) {
-    float term[IN_FLIGHT];
-#pragma unroll
-    for (int j = 0; j < IN_FLIGHT; ++j)
-      term[j] = key_term<DT>(a.mask, mask_row + min(first + j * 256 + tid, a.length - 1) * a.stride_k);
-#pragma unroll
-    for (int j = 0; j < IN_FLIGHT; ++j) {
-      const int run = first + j * 256 + wave * 64;  // first key of the wavefront's run
-      const bool any = __ballot(run + lane < a.length && __builtin_isfinite(term[j])) != 0;
-      if (lane == 0 && run < a.length) run_flags[run / 64] = any;
-    }
-  }
-  __syncthreads();
-  if (wave != 0) return;
-  const int tiles = (a.length + a.tile_size - 1) / a.tile_size;
-  const int runs = (a.length + 63) / 64, runs_per_tile = a.tile_size / 64;
-  int32_t* out = a.tiles + row * (tiles + 1);
-  int count = 0;
-  for (int base = 0; base < tiles; base += 64) {
-    const int tile = base + lane;
-    bool active = false;
-    for (int r = 0; r < runs_per_tile; ++r) {
-      const int run = tile * runs_per_tile + r;
-      active |= run < runs && run_flags[run] != 0;
-    }
-    const uint64_t votes = __ballot(active);
-    if (active) {
-      const uint64_t lower = lane == 0 ? 0ull : (votes & ((1ull << lane) - 1ull));
-      out[count + __builtin_popcountll(lower)] = tile;
-    }
-    count += __builtin_popcountll(votes);
-  }
-  // Slots behind the active ids are never read by the attention kernel.
-  for (int slot = count + lane; slot < tiles; slot += 64) out[slot] = -1;
-  if (lane == 0) out[tiles] = count;
+  key_mask_block<DT>(a, blockIdx.x, run_flags);
 }
 
 void launch_key_mask_kernel(const KeyMaskArgs& a, int dtype, hipStream_t stream) {
-  const int rows = a.tiles != nullptr ? a.batch * a.heads : 0;
-  const int blocks = rows + (a.bias != nullptr ? a.bias_planes * ((a.padded + 255) / 256) : 0);
-  const size_t flags = rows != 0 ? (a.length + 63) / 64 : 0;
+  const int blocks = key_mask_blocks(a);
+  const size_t flags = key_mask_flag_bytes(a);
   if (dtype == kBool)
     key_mask_kernel<kBool><<<blocks, 256, flags, stream>>>(a);
   else if (dtype == kF32)
@@ -289,125 +211,16 @@ void launch_key_mask_kernel(const KeyMaskArgs& a, int dtype, hipStream_t stream)
     key_mask_kernel<kBF16><<<blocks, 256, flags, stream>>>(a);
 }
 
-// Lane words of a boolean mask (the form kMaskLanes of the attention kernel reads): for
-// every block of 32 queries and 64-key tile, 32 words; bit l of word 16*rb + i is the mask
-// element of query 32*block + l % 32 and key 64*tile + 32*rb + 8*(i / 4) + 4*(l / 32) + i % 4,
-// which is score (rb, i) of lane l in the attention kernel.  Rows past the last query and
-// keys past the last key have no bit set.
-//
-// grid (groups of 16 tiles, blocks of 32 queries, batch*heads of the mask), 256 threads: a
-// wavefront takes four consecutive key tiles of one query block (256 mask bytes per row, all
-// requested before the first is used).  Lane (row, half) reads, per tile and 32-key block,
-// the sixteen elements at keys 16*half .. 16*half+15 of the block (one 16-byte load when
-// ALIGNED): the eight-key groups b4 = 2*half and 2*half+1, both four-key halves of each.
-// A vote over element (b', h', r) of every lane therefore holds, in its low 32 bits, the
-// rows' decisions for group b' and, in its high 32 bits, those for group 2+b', four-key
-// half h' each; a lane word wants the two halves h' of one group side by side, which is a
-// regrouping of 32-bit scalar registers.  Lane s keeps word s, so the 32 words of a tile
-// leave in one 256-byte store.
-constexpr int kLaneTilesPerWave = 4;
-// A wave-uniform 32-bit value written into one lane of a vector register.  The value comes from a vector
-// comparison, and a vector instruction may read such a scalar register two wait states later: the compiler
-// counts them for its own instructions only, so they stand in front of this one.
-__device__ __forceinline__ void write_lane(uint32_t& target, uint32_t uniform_value, int lane_index) {
-  asm("s_nop 1\n\tv_writelane_b32 %0, %1, %2" : "+v"(target) : "s"(uniform_value), "n"(lane_index));
+template <bool ALIGNED> __global__ __launch_bounds__(256) void mask_lanes_kernel(const MaskLaneArgs a) {
+  mask_lanes_block<ALIGNED>(a, blockIdx.x, blockIdx.y, blockIdx.z);
 }
-template <bool ALIGNED>
-__global__ __launch_bounds__(256) void mask_lanes_kernel(const uint8_t* __restrict__ mask,
-                                                         uint64_t* __restrict__ lanes,
-                                                         int32_t* __restrict__ classes, int heads,
-                                                         int q_len, int k_len, int key_tiles,
-                                                         int query_waves, int64_t stride_b,
-                                                         int64_t stride_h, int64_t stride_q) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int query_wave = blockIdx.y, plane = blockIdx.z;
-  const int row = query_wave * 32 + (lane & 31), half = lane >> 5;
-  const bool row_ok = row < q_len;
-  const uint8_t* row_mask = mask + (plane / heads) * stride_b + (plane % heads) * stride_h +
-                            static_cast<int64_t>(row_ok ? row : q_len - 1) * stride_q;
-  uint64_t* out = lanes + (static_cast<int64_t>(plane) * query_waves + query_wave) * key_tiles * 32;
-  const int first_tile = (blockIdx.x * 4 + wave) * kLaneTilesPerWave;
-  typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-  v4u chunk[kLaneTilesPerWave][2];
-#pragma unroll
-  for (int t = 0; t < kLaneTilesPerWave; ++t) {
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      const int key = (first_tile + t) * 64 + rb * 32 + half * 16;
-      v4u words = {0u, 0u, 0u, 0u};
-      if (ALIGNED && key + 15 < k_len) {
-        words = *reinterpret_cast<const v4u*>(row_mask + key);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          if (key + j < k_len && row_mask[key + j] != 0) words[j >> 2] |= 1u << (8 * (j & 3));
-        }
-      }
-      if (!row_ok) words = v4u{0u, 0u, 0u, 0u};
-      chunk[t][rb] = words;
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < kLaneTilesPerWave; ++t) {
-    if (first_tile + t >= key_tiles) break;  // wave-uniform
-    // word s of the tile goes to lane s, 32 bits at a time, straight from the scalar registers
-    uint32_t mine_low = 0, mine_high = 0;
-    uint64_t every = ~uint64_t{0}, any = 0;  // what all words of the tile / at least one of them hold
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-#pragma unroll
-      for (int group = 0; group < 2; ++group) {  // b'
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint64_t first = __ballot(((chunk[t][rb][group * 2] >> (8 * r)) & 0xffu) != 0);
-          const uint64_t second = __ballot(((chunk[t][rb][group * 2 + 1] >> (8 * r)) & 0xffu) != 0);
-          every &= first & second;
-          any |= first | second;
-          const int low_slot = rb * 16 + group * 4 + r;        // b4 = b'
-          const int high_slot = rb * 16 + (2 + group) * 4 + r;  // b4 = 2 + b'
-          write_lane(mine_low, static_cast<uint32_t>(first), low_slot);
-          write_lane(mine_high, static_cast<uint32_t>(second), low_slot);
-          write_lane(mine_low, static_cast<uint32_t>(first >> 32), high_slot);
-          write_lane(mine_high, static_cast<uint32_t>(second >> 32), high_slot);
-        }
-      }
-    }
-    const uint64_t mine = mine_low | (static_cast<uint64_t>(mine_high) << 32);
-    if (lane < 32) out[static_cast<int64_t>(first_tile + t) * 32 + lane] = mine;
-    if (lane == 0) {
-      classes[(static_cast<int64_t>(plane) * query_waves + query_wave) * key_tiles + first_tile + t] =
-          every == ~uint64_t{0} ? kLaneTileVisible : any == 0 ? kLaneTileHidden : kLaneTileMixed;
-    }
-  }
+
+// grid (query blocks, planes)
+__global__ __launch_bounds__(64) void mask_tile_lists_kernel(const MaskLaneArgs a) {
+  mask_tile_list(a, blockIdx.x, blockIdx.y, threadIdx.x);
 }
 
 }  // namespace
-
-// Tile lists of the mask: grid (query blocks, planes), one wavefront.  A tile is listed for a
-// block of 128 queries unless all four of its 32-query classes say "no visible key"; entry
-// [tiles] of a list holds its length (the layout the attention kernel reads for key-mask
-// tiles).  A block that sees nothing keeps an empty list: its rows come out as zeros.
-__global__ __launch_bounds__(64) void mask_tile_lists_kernel(const int32_t* __restrict__ classes,
-                                                            int32_t* __restrict__ lists, int key_tiles,
-                                                            int query_blocks) {
-  const int lane = threadIdx.x;
-  const int block = blockIdx.x, plane = blockIdx.y;
-  const int32_t* wave_classes = classes + (static_cast<int64_t>(plane) * query_blocks + block) * 4 * key_tiles;
-  int32_t* list = lists + (static_cast<int64_t>(plane) * query_blocks + block) * (key_tiles + 1);
-  int count = 0;
-  for (int first = 0; first < key_tiles; first += 64) {
-    const int tile = first + lane;
-    bool listed = false;
-    if (tile < key_tiles) {
-#pragma unroll
-      for (int w = 0; w < 4; ++w) listed = listed || wave_classes[w * key_tiles + tile] != kLaneTileHidden;
-    }
-    const uint64_t ballot = __ballot(listed);
-    if (listed) list[count + __popcll(ballot & ((uint64_t{1} << lane) - 1))] = tile;
-    count += __popcll(ballot);
-  }
-  if (lane == 0) list[key_tiles] = count;
-}
 
 size_t mask_lane_words(int batch, int heads, int q_len, int k_len) {
   const size_t query_waves = (static_cast<size_t>(q_len) + 127) / 128 * 4;
@@ -431,22 +244,34 @@ size_t mask_lane_bytes(int batch, int heads, int q_len, int k_len) {
   return mask_tile_list_offset(batch, heads, q_len, k_len) + (lists * sizeof(int32_t) + 7) / 8 * 8;
 }
 
-int launch_mask_lanes(const void* mask, uint64_t* lanes, int batch, int heads, int q_len, int k_len,
-                      int64_t stride_b, int64_t stride_h, int64_t stride_q, hipStream_t stream) {
-  const int query_waves = (q_len + 127) / 128 * 4;
-  const int key_tiles = (k_len + 63) / 64;
-  if (query_waves > 65535 || static_cast<int64_t>(batch) * heads > 65535)
-    return fail("risa_prepare_mask_lanes: more query blocks or mask planes than one launch covers");
-  const dim3 grid((key_tiles + 4 * kLaneTilesPerWave - 1) / (4 * kLaneTilesPerWave), query_waves, batch * heads);
-  const bool aligned = reinterpret_cast<uintptr_t>(mask) % 16 == 0 && ((stride_b | stride_h | stride_q) & 15) == 0;
-  auto kernel = aligned ? mask_lanes_kernel<true> : mask_lanes_kernel<false>;
+MaskLaneArgs mask_lane_args(const void* mask, uint64_t* lanes, int batch, int heads, int q_len, int k_len,
+                            int64_t stride_b, int64_t stride_h, int64_t stride_q) {
   unsigned char* bytes = reinterpret_cast<unsigned char*>(lanes);
-  int32_t* classes = reinterpret_cast<int32_t*>(bytes + mask_lane_class_offset(batch, heads, q_len, k_len));
-  int32_t* lists = reinterpret_cast<int32_t*>(bytes + mask_tile_list_offset(batch, heads, q_len, k_len));
-  kernel<<<grid, 256, 0, stream>>>(static_cast<const uint8_t*>(mask), lanes, classes, heads, q_len, k_len,
-                                   key_tiles, query_waves, stride_b, stride_h, stride_q);
-  mask_tile_lists_kernel<<<dim3(query_waves / 4, batch * heads), 64, 0, stream>>>(classes, lists, key_tiles,
-                                                                              query_waves / 4);
+  MaskLaneArgs a{};
+  a.mask = static_cast<const uint8_t*>(mask);
+  a.lanes = lanes;
+  a.classes = reinterpret_cast<int32_t*>(bytes + mask_lane_class_offset(batch, heads, q_len, k_len));
+  a.lists = reinterpret_cast<int32_t*>(bytes + mask_tile_list_offset(batch, heads, q_len, k_len));
+  a.heads = heads;
+  a.planes = batch * heads;
+  a.q_len = q_len;
+  a.k_len = k_len;
+  a.key_tiles = (k_len + 63) / 64;
+  a.query_waves = (q_len + 127) / 128 * 4;
+  a.stride_b = stride_b;
+  a.stride_h = stride_h;
+  a.stride_q = stride_q;
+  a.aligned = reinterpret_cast<uintptr_t>(mask) % 16 == 0 && ((stride_b | stride_h | stride_q) & 15) == 0;
+  return a;
+}
+
+int launch_mask_lanes(const MaskLaneArgs& a, hipStream_t stream) {
+  const dim3 grid(mask_lane_groups(a), a.query_waves, a.planes);
+  if (a.aligned)
+    mask_lanes_kernel<true><<<grid, 256, 0, stream>>>(a);
+  else
+    mask_lanes_kernel<false><<<grid, 256, 0, stream>>>(a);
+  mask_tile_lists_kernel<<<dim3(a.query_waves / 4, a.planes), 64, 0, stream>>>(a);
   return check_launch("risa_prepare_mask_lanes");
 }
 
@@ -508,9 +333,9 @@ int launch_key_mask_tiles(const void* mask, int32_t* tiles, int batch, int heads
   return check_launch("risa_prepare_key_mask_tiles");
 }
 
-int launch_key_mask(const void* mask, int32_t* tiles, float* bias, int batch, int heads, int mask_batch,
-                    int mask_heads, int length, int padded, int tile_size, int64_t stride_b,
-                    int64_t stride_h, int64_t stride_k, int dtype, hipStream_t stream) {
+KeyMaskArgs key_mask_args(const void* mask, int32_t* tiles, float* bias, int batch, int heads, int mask_batch,
+                          int mask_heads, int length, int padded, int tile_size, int64_t stride_b,
+                          int64_t stride_h, int64_t stride_k) {
   KeyMaskArgs a{};
   a.mask = mask;
   a.tiles = tiles;
@@ -527,6 +352,10 @@ int launch_key_mask(const void* mask, int32_t* tiles, float* bias, int batch, in
   a.stride_k = stride_k;
   a.bias_stride_b = mask_batch > 1 ? stride_b : 0;
   a.bias_stride_h = mask_heads > 1 ? stride_h : 0;
+  return a;
+}
+
+int launch_key_mask(const KeyMaskArgs& a, int dtype, hipStream_t stream) {
   launch_key_mask_kernel(a, dtype, stream);
   return check_launch("risa_sdpa key mask");
 }

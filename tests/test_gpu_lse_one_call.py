@@ -3,7 +3,8 @@
 The packed route adds the anchor correction to the log-normalisers as tensors; the single call stores
 it first and lets the attention kernel add its term.  Both are one FP32 addition, so results are equal
 bit for bit in every form the call takes: kernels of few and of many workgroups, split key ranges, rows
-that the preparation pads, every mask form, types and layouts.
+that the preparation pads, every mask form, types and layouts.  (Keys of head dim 256 fill whole tiles or
+have more than 2048 tokens here: the packed route takes another kernel for the others.)
 """
 
 from __future__ import annotations
@@ -26,8 +27,17 @@ FORMS = [
     (2, 24, 8, 1000, 1300, 128, torch.float16, "midpoint_affine", False, "padding", True),
     (1, 40, 8, 1025, 900, 128, torch.float32, "absmax", False, "bias", False),
     (1, 40, 8, 1100, 1100, 200, torch.bfloat16, "absmax", True, None, False),
-    (1, 24, 8, 1500, 1280, 256, torch.bfloat16, "absmax", False, None, False),  # (ragged: another kernel there)
+    (1, 24, 8, 1500, 1280, 256, torch.bfloat16, "absmax", False, None, False),
     (1, 16, 16, 128, 4096, 128, torch.bfloat16, "absmax", False, "padding", False),  # split key ranges
+    # mask forms made by workgroups of the preparation: one launch and two, lane words of aligned rows
+    # (the packed route makes all of them in launches of their own)
+    (2, 24, 24, 1000, 1296, 64, torch.bfloat16, "absmax", False, "bool", False),
+    (3, 16, 16, 1153, 4160, 128, torch.bfloat16, "midpoint_affine", False, "bool", False),
+    (2, 24, 24, 512, 512, 64, torch.float16, "absmax", False, "bool", False),
+    (1, 40, 8, 1025, 6016, 80, torch.bfloat16, "absmax", False, "documents", False),
+    (2, 8, 8, 256, 512, 64, torch.bfloat16, "absmax", False, "padding", False),
+    (2, 24, 24, 260, 1025, 64, torch.float32, "absmax", False, "key_bias", False),
+    (1, 24, 8, 1000, 5000, 256, torch.bfloat16, "midpoint_affine", True, "key_bias", False),
 ]
 
 
@@ -50,6 +60,12 @@ def test_one_call_matches_packed_route(form):
         mask = torch.rand(batch, 1, q_len, k_len, generator=generator) < 0.7
         mask[:, :, :5] = False  # rows that see no key
         mask = mask.cuda()
+    elif mask_kind == "documents":
+        mask = (torch.arange(q_len)[:, None] * 8 // q_len == torch.arange(k_len) * 8 // k_len)[None, None].cuda()
+    elif mask_kind == "key_bias":
+        mask = torch.randn(batch, 1, 1, k_len, generator=generator)
+        mask[:, :, :, 128:400] = -torch.inf
+        mask = mask.half().cuda()
     elif mask_kind == "bias":
         mask = torch.randn(batch, 1, q_len, k_len, generator=generator).cuda()
     packed = risa.prequantize_int8_attention(q, k, v, attn_mask=mask, v_quantization=mode, is_causal=causal,
