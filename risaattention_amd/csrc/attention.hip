@@ -180,8 +180,8 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
   p.sm2 = a.sm_scale * kLog2e;
   p.out_dtype = a.out_dtype;
   p.workspace = a.block_mass;
-  p.lse = a.lse;
-  p.lse_shift = a.lse_shift;
+  if (reinterpret_cast<uintptr_t>(a.lse) % 4 != 0) return fail("risa_attention: LSE must be 4-byte aligned");
+  p.lse = a.lse_holds_shift ? reinterpret_cast<float*>(reinterpret_cast<char*>(a.lse) + 1) : a.lse;
   p.causal = a.is_causal ? 1 : 0;
   p.whole_key_tiles = a.whole_key_tiles ? 1 : 0;
   // Diagnostic switch, read at every launch: RISA_COMPILED_LOOP=1 sends every kernel that has a
@@ -216,8 +216,8 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
 
   // A launch that cannot give every compute unit more than one workgroup runs the
   // raw-score path with sixteen queries per wavefront (two wavefronts per SIMD).  So does
-  // every launch with head dim 256, masked, causal and capturing ones included: thirty-two
-  // queries of 256 channels per wavefront need some 380 registers, which leaves one
+  // every launch with head dim 256 that attention_d256.hip does not take (below): for the compiler
+  // thirty-two queries of 256 channels per wavefront need some 380 registers, which leaves one
   // wavefront per SIMD (1200 against 1630 dense-equivalent TOPS at N=16K).
   const int64_t workgroups = static_cast<int64_t>(p.n_qb) * a.q_heads * a.batch;
   const bool narrow = fast && p.index_mode != 2 && !capture &&

@@ -173,7 +173,7 @@ int checked_v_args(risa::ValueArgs& a, const void* v, void* out, float* scale, f
 
 namespace {
 
-// One attention launch from the C arguments; `lse_shift`: the kernel adds it to `lse`.
+// One attention launch from the C arguments; `lse_holds_shift`: the kernel adds to what `lse` holds.
 int attend(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
                    const float* q_scale, const float* k_scale, const float* v_scale,
                    const float* v_center, const int32_t* v_tile_sum, const void* mask,
@@ -182,7 +182,7 @@ int attend(const void* q_int8, const void* k_int8, const void* v_int8, void* out
                    int k_len, int q_heads, int kv_heads, int head_dim, int64_t out_stride_b,
                    int64_t out_stride_n, int64_t out_stride_h, float sm_scale, int out_dtype,
                    const int32_t* sparse_row_offsets, const int32_t* sparse_block_indices,
-                   float* block_mass, int is_causal, float* lse, const float* lse_shift, const int32_t* key_mask_tiles,
+                   float* block_mass, int is_causal, float* lse, bool lse_holds_shift, const int32_t* key_mask_tiles,
                    const float* key_bias, int64_t key_bias_stride_b, int64_t key_bias_stride_h,
                    const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
                    int64_t mask_lanes_stride_h, int64_t k_bytes, void* split_workspace,
@@ -228,7 +228,7 @@ int attend(const void* q_int8, const void* k_int8, const void* v_int8, void* out
   a.block_mass = block_mass;
   a.is_causal = is_causal != 0;
   a.lse = lse;
-  a.lse_shift = lse_shift;
+  a.lse_holds_shift = lse_holds_shift;
   a.key_mask_tiles = key_mask_tiles;
   if (key_bias != nullptr && (mask == nullptr || mask_stride_q != 0))
     return fail("risa_attention: a key bias row goes with a key-only mask (query stride 0)");
@@ -388,7 +388,7 @@ int risa_attention_split(const void* q_int8, const void* k_int8, const void* v_i
                    const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
                    int64_t mask_lanes_stride_h, int64_t k_bytes, void* split_workspace,
                    size_t split_workspace_bytes, void* stream) {
-  return attend(q_int8, k_int8, v_int8, out, q_scale, k_scale, v_scale, v_center, v_tile_sum, mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, cta_k, batch, q_len, k_len, q_heads, kv_heads, head_dim, out_stride_b, out_stride_n, out_stride_h, sm_scale, out_dtype, sparse_row_offsets, sparse_block_indices, block_mass, is_causal, lse, nullptr, key_mask_tiles, key_bias, key_bias_stride_b, key_bias_stride_h, mask_lanes, mask_lanes_stride_b, mask_lanes_stride_h, k_bytes, split_workspace, split_workspace_bytes, stream);
+  return attend(q_int8, k_int8, v_int8, out, q_scale, k_scale, v_scale, v_center, v_tile_sum, mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, cta_k, batch, q_len, k_len, q_heads, kv_heads, head_dim, out_stride_b, out_stride_n, out_stride_h, sm_scale, out_dtype, sparse_row_offsets, sparse_block_indices, block_mass, is_causal, lse, false, key_mask_tiles, key_bias, key_bias_stride_b, key_bias_stride_h, mask_lanes, mask_lanes_stride_b, mask_lanes_stride_h, k_bytes, split_workspace, split_workspace_bytes, stream);
 }
 
 int risa_attention_readable_keys(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
@@ -685,7 +685,7 @@ int risa_sdpa_lse(const void* q, const void* k, const void* v, void* out, void* 
                         mask_stride_q, mask_stride_k, mask_dtype, cta_k, batch, q_len, k_len,
                         q_heads, kv_heads, head_dim, out_stride_b, out_stride_n, out_stride_h,
                         sm_scale, output_dtype, sparse_row_offsets, sparse_block_indices, nullptr,
-                        is_causal, lse, lse, key_tiles, key_bias, bias_stride_b, bias_stride_h,
+                        is_causal, lse, lse != nullptr, key_tiles, key_bias, bias_stride_b, bias_stride_h,
                         mask_lanes, lanes_stride_b, lanes_stride_h, static_cast<int64_t>(l.bytes - l.k_codes),
                         base + l.bytes, workspace_bytes - l.bytes, stream);
 }

@@ -80,7 +80,7 @@ struct AttentionArgs {
   bool is_causal;
   bool whole_key_tiles;  // cta_k rows behind the last key can be read (their contents do not matter)
   float* lse;
-  const float* lse_shift;  // added to lse as it is stored (may be the same memory), or null
+  bool lse_holds_shift;  // the log-normalisers are added to what lse holds
   const int32_t* key_mask_tiles;
   const float* key_bias;  // [Bm,Hm,padded] from launch_key_bias, or null
   int64_t key_bias_stride_b, key_bias_stride_h;

@@ -418,3 +418,21 @@ def test_short_tile_lists_match_oracle(risa, dim, heads, output_dtype):
                                                pattern.block_indices[: int(offsets[rows])].clone(), 1, 2, q_len, k_len,
                                                128, packed.cta_k, packed.attention_scale, 0.5, 0.5))
         assert relative_l2(to_numpy(twin), to_numpy(out[:, :2])) < 1e-4
+
+
+@pytest.mark.parametrize("rows,tiles", [(2049, 127), (255, 128), (300, 129), (4100, 63), (257, 65), (2, 3)])
+def test_selection_at_the_edges_of_counting_and_of_loads_in_flight(risa, rows, tiles):
+    """Up to 128 tiles a row is sorted by counting, beyond by the network; the offsets take eight rows per
+    thread at a time.  Every place is taken once with repeated, negative-zero and zero masses."""
+    from risaattention_amd.patterns import select_retained_mass_csr
+
+    g = torch.Generator().manual_seed(rows + tiles)
+    masses = (torch.rand(rows, tiles, generator=g) * 8).floor() / 8  # many ties
+    masses[rows // 2] = 0
+    masses[rows // 3, ::2] *= -0.0
+    masses = masses.cuda()
+    row_offsets, block_indices, measured = select_retained_mass_csr(masses, 0.9)
+    ro, bi, expected_measured, _ = oracle_selection.select_retained_mass(masses.cpu().numpy(), 0.9)
+    np.testing.assert_array_equal(row_offsets.cpu().numpy(), ro)
+    np.testing.assert_array_equal(block_indices.cpu().numpy(), bi)
+    assert measured == pytest.approx(expected_measured, rel=1e-12)
