@@ -300,10 +300,22 @@ def tile_body(e, p, last, prio, label):
         e.valu(f"v_lshlrev_b32_e32 v{past}, 2, v{past}", [past])
         e.valu(f"v_sub_u32_e32 v{rem}, v{rem}, v{past}", [rem])
         e.valu(f"v_mov_b32_e32 v{past}, {bits}", [past])
+        # A select reads its comparison two wait states behind it (nothing in hardware holds it back), so
+        # three scalar pairs take turns.  (Keys below 64 are inline constants, which is what a comparison
+        # into such a pair takes.)
+        masks = ["vcc", pair(p.kat), pair(p.at)]
+        selects = []
         for rb in range(RB):
+            if rb == 2:
+                e.valu(f"v_add_u32_e32 v{rem}, 0xffffffc0, v{rem}", [rem])  # - 64
             for i in range(16):
-                e.valu(f"v_cmp_lt_i32_e32 vcc, {rb * 32 + (i >> 2) * 8 + (i & 3)}, v{rem}")
-                e.valu(f"v_cndmask_b32_e32 v{S[rb] + i}, v{past}, v{S[rb] + i}, vcc", [S[rb] + i])
+                mask = masks[(rb * 16 + i) % 3]
+                e.valu(f"v_cmp_lt_i32_e64 {mask}, {rb % 2 * 32 + (i >> 2) * 8 + (i & 3)}, v{rem}")
+                selects.append(lambda r=S[rb] + i, m=mask: e.valu(f"v_cndmask_b32_e64 v{r}, v{past}, v{r}, {m}", [r]))
+                if len(selects) > 2:
+                    selects.pop(0)()
+        for select in selects:
+            select()
         e.raw(f"{label}_whole:")
 
     for rb in (2, 3):

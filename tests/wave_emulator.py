@@ -3,8 +3,9 @@ one workgroup with their registers, LDS and the global memory they may touch, va
 
 What it refuses: an access outside the given memory, an LDS read of bytes a copy is still to fill or
 that nothing has filled, a register touched while an LDS read or scalar load is to fill it, a barrier
-reached with loads in flight or not by every wavefront, and vector instructions on a matrix result
-before it is there."""
+reached with loads in flight or not by every wavefront, vector instructions on a matrix result before it
+is there, and vector instructions that read a comparison's scalar result less than two wait states behind
+it (what the compiler leaves between its own: nothing in hardware holds the reader back)."""
 
 import re
 
@@ -12,6 +13,7 @@ import numpy as np
 
 LANES = np.arange(64)
 MATRIX_RESULT_STATES = 12  # wait states between an 8-pass matrix instruction and a vector one on its result
+COMPARISON_STATES = 2  # wait states between a vector comparison and a vector instruction that reads its result
 
 
 class Memory:
@@ -45,6 +47,7 @@ class Wave:
             self.v[register] = np.broadcast_to(np.asarray(values).astype(np.uint32), 64)
         self.s, self.vcc, self.scc, self.exec, self.m0 = {}, np.zeros(64, bool), 0, np.ones(64, bool), 0
         self.pending_lds, self.pending_scalar, self.pending_copies, self.written, self.clock = [], [], [], {}, 0
+        self.compared = {}  # scalar registers ("vcc" by name) -> when a vector comparison wrote them
 
     # ---- operands ------------------------------------------------------------------------------------
     @staticmethod
@@ -185,9 +188,16 @@ class Wave:
                 elif op.startswith("v_cmp"):
                     self.check(touched, line)
                     a, b = self.vector(args[1]), self.vector(args[2])
-                    self.vcc = {"v_cmp_gt_f32_e32": f(a) > f(b), "v_cmp_lt_i32_e32": i(a) < i(b), "v_cmp_ne_u32_e32": a != b}[op]
+                    result = {"gt_f32": f(a) > f(b), "lt_i32": i(a) < i(b), "ne_u32": a != b}[re.sub(r"v_cmp_|_e\d\d", "", op)]
+                    if args[0] == "vcc":
+                        self.vcc = result
+                    else:
+                        self.assign(args[0], int(sum(int(bit) << lane for lane, bit in enumerate(result))))
+                    self.compared.update({n: self.clock for n in self.registers(args[0])[1] or ["vcc"]})
                 elif op.startswith("v_"):
                     self.check(touched, line)
+                    for n in {n for k, n in touched if k == "s"} | {"vcc"} & set(args):
+                        assert self.clock - self.compared.get(n, -100) > COMPARISON_STATES, f"comparison's result too early: {line}"
                     x = [self.vector(t) for t in args[1:] if not re.fullmatch(r"s\[\d+:\d+\]|vcc", t)]
                     if op.startswith("v_cndmask"):
                         result = np.where(self.lanes_of(args[3]), x[1], x[0])
