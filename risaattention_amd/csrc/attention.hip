@@ -16,6 +16,8 @@ template <> int launch_attention_variant<64>(const KernelParams&, int, bool, boo
 template <> int launch_attention_variant<128>(const KernelParams&, int, bool, bool, bool, int, hipStream_t);
 int launch_attention_narrow(const KernelParams& p, int head_dim, int cta_k, hipStream_t stream);
 int launch_attention_d256(const KernelParams& p, bool fast, hipStream_t stream);
+int launch_attention_key_ranges(const KernelParams& p, int head_dim, int cta_k, bool fast, int mask_mode,
+                                hipStream_t stream);
 int launch_attention_narrow_general(const KernelParams& p, int head_dim, int cta_k, bool fast, bool indexed,
                                     bool capture, int mask_mode, hipStream_t stream);
 
@@ -181,7 +183,7 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
   p.out_dtype = a.out_dtype;
   p.workspace = a.block_mass;
   if (reinterpret_cast<uintptr_t>(a.lse) % 4 != 0) return fail("risa_attention: LSE must be 4-byte aligned");
-  p.lse = a.lse_holds_shift ? reinterpret_cast<float*>(reinterpret_cast<char*>(a.lse) + 1) : a.lse;
+  p.lse = reinterpret_cast<uintptr_t>(a.lse) | (a.lse_holds_shift ? 1 : 0);
   p.causal = a.is_causal ? 1 : 0;
   p.whole_key_tiles = a.whole_key_tiles ? 1 : 0;
   // Diagnostic switch, read at every launch: RISA_COMPILED_LOOP=1 sends every kernel that has a
@@ -229,8 +231,9 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
   const bool narrow_general = !narrow && mask_mode != kMaskLanes &&
                               (a.head_dim > 128 || workgroups <= narrow_attention_limit());
   // Few query blocks: ranges of the key tiles go to workgroups of their own.  (A sparse pattern's lists
-  // can be much shorter than the key range, which nothing here knows.)
-  if ((narrow || narrow_general) && !capture && !sparse && a.split_workspace != nullptr) {
+  // can be much shorter than the key range, which nothing here knows; tile lists come with the additive row.)
+  if ((narrow || narrow_general) && !capture && !sparse && a.split_workspace != nullptr &&
+      (p.index_mode == 0 || a.key_bias != nullptr)) {
     const AttentionExtents extents{a.batch, a.q_heads, a.q_len, a.k_len, a.head_dim, a.cta_k};
     const SplitKind kind = fast ? SplitKind::kPlain
                            : a.mask != nullptr && a.key_bias == nullptr ? SplitKind::kMaskTensor : SplitKind::kScaled;
@@ -258,6 +261,8 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
                           workgroups > (a.is_causal ? 2 : 1) * narrow_attention_limit();
   if (wide_heads)
     status = launch_attention_d256(p, fast, stream);
+  else if (p.key_parts > 1)
+    status = launch_attention_key_ranges(p, a.head_dim, a.cta_k, fast, mask_mode, stream);
   else if (narrow)
     status = launch_attention_narrow(p, a.head_dim, a.cta_k, stream);
   else if (narrow_general)

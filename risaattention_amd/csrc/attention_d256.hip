@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256, 2) void attention_d256_kernel(const KernelPara
       *reinterpret_cast<v4i*>(out_block + 2 * static_cast<int64_t>(row) * p.out_stride_n + chunk * 16) = piece;
     }
   }
-  if (p.lse != nullptr && half == 0 && query < p.q_len) {
+  if (p.lse != 0 && half == 0 && query < p.q_len) {
     store_lse(p, bhq * p.q_len + query,
               row_valid ? (__builtin_amdgcn_logf(d_total) + m_run) / kLog2e : -__builtin_inff());
   }

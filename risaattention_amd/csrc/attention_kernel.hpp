@@ -84,11 +84,11 @@ struct KernelParams {
   int index_mode;
   int64_t tile_list_stride_b, tile_list_stride_h;  // mode 3: elements between the lists of mask planes (0: shared)
   float* workspace;  // capture
-  float* lse;  // (an odd address: see store_lse)
+  uintptr_t lse;  // address of the log-normalisers, or 0; its lowest bit: see store_lse
   int causal;
   int whole_key_tiles;  // the last key tile can be copied whole although fewer keys are left
   int compiled_loop;  // non-zero: every tile through the loop the compiler schedules (see RISA_COMPILED_LOOP)
-  int key_parts;   // ranges of the key tiles that workgroups of their own walk (sixteen-query kernel; 0, 1: one)
+  int key_parts;   // ranges of the key tiles that workgroups of their own walk (attention_key_ranges.hip; 0: one)
   float* partial;  // their results, before merge_key_parts_kernel
 };
 
@@ -96,9 +96,9 @@ struct KernelParams {
 // K anchor took off, to be added: a parameter of its own is a scalar register more from the first
 // instruction on, which the compiled tile loop of 16/4 heads x 2048 showed (0.8 us of 48.4).
 __device__ __forceinline__ void store_lse(const KernelParams& p, int64_t row, float value) {
-  const bool holds_shift = (reinterpret_cast<uintptr_t>(p.lse) & 1) != 0;
-  float* target = reinterpret_cast<float*>(reinterpret_cast<char*>(p.lse) - (holds_shift ? 1 : 0)) + row;
-  *target = holds_shift ? value + *target : value;
+  typedef __attribute__((address_space(1))) float* GlobalFloats;
+  const GlobalFloats target = (GlobalFloats)(p.lse & ~uintptr_t{1}) + row;
+  *target = (p.lse & 1) != 0 ? value + *target : value;
 }
 
 // Byte offset of 16-byte chunk `chunk` of row `row` in a swizzled LDS tile.
@@ -1423,7 +1423,7 @@ __global__ __launch_bounds__(256, attention_workgroups(D, CTA_K, FAST, INDEXED, 
       *reinterpret_cast<v4i*>(out_block + 2 * static_cast<int64_t>(row) * p.out_stride_n + chunk * 16) = piece;
     }
   }
-  if (p.lse != nullptr && half == 0 && query_ok) {
+  if (p.lse != 0 && half == 0 && query_ok) {
     store_lse(p, bhq * p.q_len + query,
               row_valid ? (__builtin_amdgcn_logf(d_total) + m_run) / kLog2e : -__builtin_inff());
   }

@@ -115,7 +115,7 @@ __device__ __forceinline__ void store_narrow_lse(const KernelParams& p, int64_t 
 }
 
 template <int D, int CTA_K, int WAVES, int KSPLIT = 1, bool INDEXED = false, bool GENERAL = false,
-          bool CAPTURE = false, int MASK_DT = -1, bool MASK_VEC = false>
+          bool CAPTURE = false, int MASK_DT = -1, bool MASK_VEC = false, bool RANGES = false>
 __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(const KernelParams p) {
   static_assert(WAVES == 8 || WAVES == 4 || WAVES == 2, "seeds and scales are copied by two different wavefronts");
   static_assert(KSPLIT == 1 || (KSPLIT == 2 && WAVES <= 4), "at most eight wavefronts per workgroup");
@@ -123,6 +123,7 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
   static_assert(!(GENERAL || CAPTURE) || (WAVES == 8 && KSPLIT == 1), "masks and capture: 128-query workgroups");
   static_assert(GENERAL || MASK_DT < 0, "the raw-score path takes no mask");
   static_assert(!(CAPTURE && INDEXED), "statistics are captured on dense runs");
+  static_assert(!RANGES || (WAVES == 8 && KSPLIT == 1 && !CAPTURE), "ranges of the key tiles: 128-query workgroups");
   constexpr bool TENSOR_MASK = MASK_DT >= 0 && MASK_DT != kKeyBias;
   constexpr int QUERIES = 16 * WAVES;
   using Shape = NarrowTileShape<D, CTA_K, MASK_DT>;
@@ -143,8 +144,7 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
   unsigned char* lds = lds_all + part * Shape::kLdsBytes;
 
   const int query_blocks = (p.q_len + QUERIES - 1) / QUERIES;
-  constexpr bool RANGES = WAVES == 8 && KSPLIT == 1 && !CAPTURE;  // of the key tiles: blockIdx.y, p.key_parts of them
-  const int block = blockIdx.x, key_part = blockIdx.y;
+  const int block = blockIdx.x;
   int bx, head, batch;
   if (GENERAL && p.causal) {
     // longest query blocks first, across all heads (as in the wide kernel)
@@ -192,23 +192,22 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
       listed = (limit + CTA_K - 1) / CTA_K;
     }
   }
-  // This workgroup's range of them: all, or one of p.key_parts ranges whose results
-  // merge_key_parts_kernel puts together.  KSPLIT == 2: its second part takes the last floor(n/2) tiles
-  // of the range, the first part the rest.
+  // This workgroup's share of them: all; RANGES: one of p.key_parts ranges (blockIdx.y), whose results
+  // merge_key_parts_kernel puts together.  KSPLIT == 2: its second part takes the last floor(n/2) tiles, the
+  // first part the rest.
   int first_tile = 0, n_it = listed;
-  if (RANGES && p.key_parts > 1) {
-    first_tile = listed * key_part / p.key_parts;
-    n_it = listed * (key_part + 1) / p.key_parts - first_tile;
-  }
-  const int in_range = n_it;
-  if constexpr (KSPLIT == 2) {
-    n_it = part == 0 ? in_range - in_range / 2 : in_range / 2;
-    if (part == 1) first_tile += in_range - n_it;
-  }
   // Only the last listed tile of the query block takes the last-tile formulas: its maxima start from
   // this floor, and only it can hold keys past the end.
-  const bool holds_last = first_tile + n_it == listed;
-  const float last_floor = holds_last ? kRowFloor : -__builtin_inff();
+  float last_floor = kRowFloor;
+  if constexpr (RANGES) {
+    first_tile = listed * static_cast<int>(blockIdx.y) / p.key_parts;
+    n_it = listed * (static_cast<int>(blockIdx.y) + 1) / p.key_parts - first_tile;
+  } else if constexpr (KSPLIT == 2) {
+    const int second_half = listed / 2;
+    n_it = part == 0 ? listed - second_half : second_half;
+    first_tile = part == 0 ? 0 : listed - second_half;
+  }
+  if ((RANGES || KSPLIT == 2) && first_tile + n_it != listed) last_floor = -__builtin_inff();
   // listed tiles come through the scalar cache (uniform address; as vector loads their wait
   // would include every vector load requested before them)
   auto tile_at = [&](int step) -> int {
@@ -758,7 +757,7 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
   if constexpr (KSPLIT == 2) {
     // Both parts share the workgroup's barrier: with an odd tile count the second part has
     // walked one tile less and takes the barrier of the tile it does not have.
-    if (part == 1 && (in_range & 1)) __syncthreads();
+    if (part == 1 && (listed & 1)) __syncthreads();
   }
 
   // ---- merge of the two key halves ----------------------------------------------------------
@@ -794,9 +793,9 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
 
   // ---- partial result of a range of the key tiles ---------------------------------------------
   // Value-major, so that the lanes of a wavefront store neighbouring words.
-  if (RANGES && p.key_parts > 1) {
+  if constexpr (RANGES) {
     constexpr int VALUES = CB * 4 + 2;
-    float* at = p.partial + ((static_cast<int64_t>(key_part) * gridDim.x + block) * WAVES + wave) * (VALUES * 64) + lane;
+    float* at = p.partial + ((static_cast<int64_t>(blockIdx.y) * gridDim.x + block) * WAVES + wave) * (VALUES * 64) + lane;
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
@@ -820,93 +819,18 @@ __global__ __launch_bounds__(64 * WAVES * KSPLIT) void attention_narrow_kernel(c
   if (query_ok) {
     store_narrow_rows<D, CB>(p, bhk, batch, head, query, grp, 0, o_acc, d_total,
                              GENERAL && (MASK_DT >= 0 || p.causal));
-    if (p.lse != nullptr && grp == 0) store_narrow_lse(p, bhq, query, m_run, d_total);
+    if (p.lse != 0 && grp == 0) store_narrow_lse(p, bhq, query, m_run, d_total);
   }
 }
 
-// Puts the ranges of the key tiles together (p.key_parts partial results per query): the online-softmax
-// update once more, so only the order of FP32 additions differs from a walk over all tiles.  A wavefront
-// takes sixteen queries of an attention_narrow_kernel<D, CTA_K, 8> workgroup and 64 channels, so that
-// few query blocks still fill the machine.
-template <int D> __global__ __launch_bounds__(256) void merge_key_parts_kernel(const KernelParams p) {
-  constexpr int CB = D / 16, VALUES = CB * 4 + 2, WAVES = 8, QUERIES = 16 * WAVES;
-  const int lane = threadIdx.x & 63, ql = lane & 15, grp = lane >> 4;
-  const int query_blocks = (p.q_len + QUERIES - 1) / QUERIES;
-  const int blocks = query_blocks * p.q_heads * p.batch;
-  const int index = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-  const int first_cb = index % (D / 64) * 4, walked = index / (D / 64);  // wavefront of the walking launch
-  if (walked >= blocks * WAVES) return;
-  const int wave = walked % WAVES, block = walked / WAVES;
-  int bx, head, batch;
-  if (p.causal) {
-    const int heads = p.q_heads * p.batch;
-    const int rest = block % heads;
-    bx = query_blocks - 1 - block / heads;
-    head = rest % p.q_heads;
-    batch = rest / p.q_heads;
-  } else {
-    bx = block % query_blocks;
-    const int rest = block / query_blocks;
-    head = rest % p.q_heads;
-    batch = rest / p.q_heads;
-  }
-  const int64_t bhk = static_cast<int64_t>(batch) * p.kv_heads + head / (p.q_heads / p.kv_heads);
-  const int64_t bhq = static_cast<int64_t>(batch) * p.q_heads + head;
-  const int query = bx * QUERIES + wave * 16 + ql;
-  const int64_t part_stride = static_cast<int64_t>(blocks) * WAVES * (VALUES * 64);
-  const float* at = p.partial + static_cast<int64_t>(walked) * (VALUES * 64) + lane;
-  // Four ranges at a time, their loads in flight together (one by one, a range costs its round trip:
-  // 16 of them 23 us for 16 query blocks of 128 channels).  Past the last range the last one is read again
-  // and counts nothing.
-  constexpr int BATCH = 4;
-  float m = kRowFloor, d = 0.0f, o_acc[4][4] = {};
-  for (int first = 0; first < p.key_parts; first += BATCH) {
-    float value[BATCH][4][4], its_m[BATCH], its_d[BATCH];
-#pragma unroll
-    for (int j = 0; j < BATCH; ++j) {
-      const float* source = at + min(first + j, p.key_parts - 1) * part_stride;
-      its_m[j] = source[CB * 4 * 64];
-      its_d[j] = source[(CB * 4 + 1) * 64];
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) value[j][cb][i] = source[((first_cb + cb) * 4 + i) * 64];
-    }
-    float top = m;
-#pragma unroll
-    for (int j = 0; j < BATCH; ++j) top = __builtin_fmaxf(top, its_m[j]);
-    const float scale = __builtin_amdgcn_exp2f(m - top);
-    m = top;
-    d *= scale;
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o_acc[cb][i] *= scale;
-#pragma unroll
-    for (int j = 0; j < BATCH; ++j) {
-      const float weight = first + j < p.key_parts ? __builtin_amdgcn_exp2f(its_m[j] - m) : 0.0f;
-      d = __builtin_fmaf(its_d[j], weight, d);
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o_acc[cb][i] = __builtin_fmaf(value[j][cb][i], weight, o_acc[cb][i]);
-    }
-  }
-  float d_total = d + __shfl_xor(d, 16);
-  d_total += __shfl_xor(d_total, 32);
-  if (query < p.q_len) {
-    store_narrow_rows<D, 4>(p, bhk, batch, head, query, grp, first_cb, o_acc, d_total, p.mask_dtype >= 0 || p.causal);
-    if (p.lse != nullptr && grp == 0 && first_cb == 0) store_narrow_lse(p, bhq, query, m, d_total);
-  }
-}
-
-// Launch of one variant: grid of ceil(q_len / (16 * WAVES)) * heads * batch workgroups.
+// Launch of one variant: grid of ceil(q_len / (16 * WAVES)) * heads * batch workgroups, p.key_parts times as
+// many with RANGES.
 template <int D, int CTA_K, int WAVES, int KSPLIT, bool INDEXED = false, bool GENERAL = false,
-          bool CAPTURE = false, int MASK_DT = -1, bool MASK_VEC = false>
+          bool CAPTURE = false, int MASK_DT = -1, bool MASK_VEC = false, bool RANGES = false>
 int launch_narrow_block(const KernelParams& p, hipStream_t stream) {
   using Shape = NarrowTileShape<D, CTA_K, MASK_DT>;
   constexpr int kLdsBytes = Shape::kLdsBytes * KSPLIT;
-  auto kernel = attention_narrow_kernel<D, CTA_K, WAVES, KSPLIT, INDEXED, GENERAL, CAPTURE, MASK_DT, MASK_VEC>;
+  auto kernel = attention_narrow_kernel<D, CTA_K, WAVES, KSPLIT, INDEXED, GENERAL, CAPTURE, MASK_DT, MASK_VEC, RANGES>;
   static thread_local int configured_device = -1;
   int device = -1;
   if (hipGetDevice(&device) != hipSuccess) return fail("risa_attention: hipGetDevice failed");
@@ -918,14 +842,9 @@ int launch_narrow_block(const KernelParams& p, hipStream_t stream) {
     configured_device = device;
   }
   constexpr int QUERIES = 16 * WAVES;
-  const unsigned blocks = static_cast<unsigned>((p.q_len + QUERIES - 1) / QUERIES) * p.q_heads * p.batch;
-  constexpr bool RANGES = WAVES == 8 && KSPLIT == 1 && !CAPTURE;
-  const unsigned parts = RANGES && p.key_parts > 1 ? p.key_parts : 1;
-  kernel<<<dim3(blocks, parts), 64 * WAVES * KSPLIT, kLdsBytes, stream>>>(p);
-  if constexpr (RANGES) {
-    const unsigned wavefronts = blocks * WAVES * (D / 64);
-    if (parts > 1) merge_key_parts_kernel<D><<<dim3((wavefronts + 3) / 4), 256, 0, stream>>>(p);
-  }
+  const unsigned query_blocks = static_cast<unsigned>((p.q_len + QUERIES - 1) / QUERIES);
+  const dim3 grid(query_blocks * p.q_heads * p.batch, RANGES ? p.key_parts : 1);
+  kernel<<<grid, 64 * WAVES * KSPLIT, kLdsBytes, stream>>>(p);
   return 0;
 }
 

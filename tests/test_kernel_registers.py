@@ -34,15 +34,21 @@ def kernels(elf):
     return msgpack.unpackb(elf[note.end():note.end() + size])["amdhsa.kernels"]
 
 
-@pytest.fixture(scope="module")
-def attention_kernels():
-    """(D, CTA_K, FAST, INDEXED, CAPTURE, MASK_DT, MASK_MODE) -> metadata."""
+def variants(template):
+    """Template arguments -> metadata."""
     found = {}
     for elf in code_objects(native.library_path().read_bytes()):
         for kernel in kernels(elf):
-            name = re.search(r"16attention_kernelI((?:L[ib]n?\d+E)+)E", kernel[".name"])
+            name = re.search(template + r"I((?:L[ib]n?\d+E)+)E", kernel[".name"])
             if name:
                 found[tuple(int(x.replace("n", "-")) for x in re.findall(r"L[ib](n?\d+)E", name.group(1)))] = kernel
+    return found
+
+
+@pytest.fixture(scope="module")
+def attention_kernels():
+    """(D, CTA_K, FAST, INDEXED, CAPTURE, MASK_DT, MASK_MODE) -> metadata."""
+    found = variants("16attention_kernel")
     assert len(found) > 50
     return found
 
@@ -77,3 +83,10 @@ def test_key_only_masks_spill_no_scalar_register(attention_kernels):
     for shape in ((64, 64), (128, 128)):
         for indexed in (0, 1):
             assert attention_kernels[(*shape, 0, indexed, 0, KEY_BIAS, SCALAR)][".sgpr_spill_count"] == 0, (shape, indexed)
+
+
+def test_ranges_of_the_keys_are_kernels_of_their_own():
+    """Their run-time tests would take scalar registers and instructions from every walk over all tiles."""
+    narrow = variants("23attention_narrow_kernel")  # (..., RANGES)
+    ranges = {arguments[:-1] for arguments in narrow if len(arguments) == 10 and arguments[-1]}
+    assert len(ranges) == 60 and all((*arguments, 0) in narrow for arguments in ranges)
