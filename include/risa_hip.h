@@ -228,6 +228,10 @@ int risa_attention_split(const void* q_int8, const void* k_int8, const void* v_i
                    size_t split_workspace_bytes, void* stream);
 size_t risa_attention_split_bytes(int batch, int q_heads, int q_len, int k_len, int head_dim, int cta_k,
                                   int mask_dtype, int64_t mask_stride_q);
+/* The bytes that one call takes, 0 where it is not split: its scale and causal flag decide too (a key-only
+ * mask: with its additive row).  Both sizes belong to the current device's number of compute units. */
+size_t risa_attention_split_bytes_for(int batch, int q_heads, int q_len, int k_len, int head_dim, int cta_k,
+                                      int mask_dtype, int64_t mask_stride_q, float sm_scale, int is_causal);
 
 /*
  * Quantise and attend in one call.  Replaces risa_sdpa (reference
@@ -249,6 +253,12 @@ size_t risa_sdpa_workspace_bytes(int batch, int q_heads, int q_len, int kv_heads
                                  int head_dim, int cta_k, int midpoint_affine, int mask_dtype,
                                  int64_t mask_stride_q, int64_t mask_stride_k, int mask_batch,
                                  int mask_heads);
+/* The size covers the partial results of key ranges (risa_attention_split) for any scale and flags; this is
+ * what a call with the given ones takes.  With less, down to the sections alone, the keys are not split. */
+size_t risa_sdpa_workspace_bytes_for(int batch, int q_heads, int q_len, int kv_heads, int k_len,
+                                     int head_dim, int cta_k, int midpoint_affine, int mask_dtype,
+                                     int64_t mask_stride_q, int64_t mask_stride_k, int mask_batch,
+                                     int mask_heads, float sm_scale, int is_causal, int sparse);
 int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* workspace,
               size_t workspace_bytes, int batch, int q_heads, int q_len, int kv_heads, int k_len,
               int head_dim, int cta_k, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,

@@ -158,18 +158,21 @@ int attention_key_parts(const AttentionExtents& e, SplitKind kind, bool causal) 
   return best_parts;
 }
 
+size_t attention_split_bytes(const AttentionExtents& e, SplitKind kind, bool causal) {
+  const size_t parts = attention_key_parts(e, kind, causal);
+  const size_t blocks = static_cast<size_t>(e.batch) * e.q_heads * ((e.q_len + kQueryBlock - 1) / kQueryBlock);
+  return parts > 1 ? parts * blocks * key_part_bytes(e.head_dim) : 0;
+}
+
 size_t attention_split_bytes(const AttentionExtents& e, int mask_dtype, int64_t mask_stride_q) {
   const bool tensor = mask_dtype >= 0 && mask_stride_q != 0;
-  int parts = 1;
+  size_t bytes = 0;
   for (const bool causal : {false, true}) {
-    parts = std::max(parts, attention_key_parts(e, tensor ? SplitKind::kMaskTensor : SplitKind::kScaled, causal));
-    if (mask_dtype < 0) parts = std::max(parts, attention_key_parts(e, SplitKind::kPlain, causal));
+    bytes = std::max(bytes, attention_split_bytes(e, tensor ? SplitKind::kMaskTensor : SplitKind::kScaled, causal));
     // (a key-only mask without its additive row is read like a mask tensor)
-    if (mask_dtype >= 0) parts = std::max(parts, attention_key_parts(e, SplitKind::kMaskTensor, causal));
+    bytes = std::max(bytes, attention_split_bytes(e, mask_dtype < 0 ? SplitKind::kPlain : SplitKind::kMaskTensor, causal));
   }
-  if (parts <= 1) return 0;
-  const size_t blocks = static_cast<size_t>(e.batch) * e.q_heads * ((e.q_len + kQueryBlock - 1) / kQueryBlock);
-  return parts * blocks * key_part_bytes(e.head_dim);
+  return bytes;
 }
 
 int launch_attention_key_ranges(const KernelParams& p, int head_dim, int cta_k, bool fast, int mask_mode,

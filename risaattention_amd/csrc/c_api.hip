@@ -375,6 +375,15 @@ size_t risa_attention_split_bytes(int batch, int q_heads, int q_len, int k_len, 
   return risa::attention_split_bytes({batch, q_heads, q_len, k_len, head_dim, cta_k}, mask_dtype, mask_stride_q);
 }
 
+size_t risa_attention_split_bytes_for(int batch, int q_heads, int q_len, int k_len, int head_dim, int cta_k,
+                                      int mask_dtype, int64_t mask_stride_q, float sm_scale, int is_causal) {
+  if (batch <= 0 || q_heads <= 0 || q_len <= 0 || k_len <= 0 || (cta_k != 64 && cta_k != 128) ||
+      (head_dim != 64 && head_dim != 128 && head_dim != 256))
+    return 0;
+  const risa::SplitKind kind = risa::split_kind(mask_dtype >= 0, mask_stride_q == 0, is_causal != 0, sm_scale);
+  return risa::attention_split_bytes({batch, q_heads, q_len, k_len, head_dim, cta_k}, kind, is_causal != 0);
+}
+
 int risa_attention_split(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
                    const float* q_scale, const float* k_scale, const float* v_scale,
                    const float* v_center, const int32_t* v_tile_sum, const void* mask,
@@ -565,14 +574,10 @@ SdpaLayout sdpa_layout(int batch, int q_heads, int q_len, int kv_heads, int k_le
   return l;
 }
 
-}  // namespace
-
-extern "C" {
-
-size_t risa_sdpa_workspace_bytes(int batch, int q_heads, int q_len, int kv_heads, int k_len,
-                                 int head_dim, int cta_k, int midpoint_affine, int mask_dtype,
-                                 int64_t mask_stride_q, int64_t mask_stride_k, int mask_batch,
-                                 int mask_heads) {
+// Bytes of the sections, without the partial results of key ranges behind them.
+size_t sdpa_section_bytes(int batch, int q_heads, int q_len, int kv_heads, int k_len, int head_dim, int cta_k,
+                          int midpoint_affine, int mask_dtype, int64_t mask_stride_q, int64_t mask_stride_k,
+                          int mask_batch, int mask_heads) {
   if (batch <= 0 || q_heads <= 0 || q_len <= 0 || kv_heads <= 0 || k_len <= 0 || head_dim <= 0 ||
       (cta_k != 64 && cta_k != 128))
     return 0;
@@ -581,8 +586,31 @@ size_t risa_sdpa_workspace_bytes(int batch, int q_heads, int q_len, int kv_heads
                                              batch, q_heads, mask_batch, mask_heads, q_len, k_len);
   return sdpa_layout(batch, q_heads, q_len, kv_heads, k_len, head_dim, cta_k, midpoint_affine != 0,
                      key_only, lanes)
-             .bytes +
-         risa_attention_split_bytes(batch, q_heads, q_len, k_len, head_dim, cta_k, mask_dtype, mask_stride_q);
+      .bytes;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t risa_sdpa_workspace_bytes(int batch, int q_heads, int q_len, int kv_heads, int k_len,
+                                 int head_dim, int cta_k, int midpoint_affine, int mask_dtype,
+                                 int64_t mask_stride_q, int64_t mask_stride_k, int mask_batch,
+                                 int mask_heads) {
+  const size_t sections = sdpa_section_bytes(batch, q_heads, q_len, kv_heads, k_len, head_dim, cta_k, midpoint_affine,
+                                             mask_dtype, mask_stride_q, mask_stride_k, mask_batch, mask_heads);
+  return sections + risa_attention_split_bytes(batch, q_heads, q_len, k_len, head_dim, cta_k, mask_dtype, mask_stride_q);
+}
+
+size_t risa_sdpa_workspace_bytes_for(int batch, int q_heads, int q_len, int kv_heads, int k_len,
+                                     int head_dim, int cta_k, int midpoint_affine, int mask_dtype,
+                                     int64_t mask_stride_q, int64_t mask_stride_k, int mask_batch,
+                                     int mask_heads, float sm_scale, int is_causal, int sparse) {
+  const size_t sections = sdpa_section_bytes(batch, q_heads, q_len, kv_heads, k_len, head_dim, cta_k, midpoint_affine,
+                                             mask_dtype, mask_stride_q, mask_stride_k, mask_batch, mask_heads);
+  if (sparse != 0) return sections;
+  return sections + risa_attention_split_bytes_for(batch, q_heads, q_len, k_len, head_dim, cta_k, mask_dtype,
+                                                   mask_stride_q, sm_scale, is_causal);
 }
 
 int risa_sdpa_lse(const void* q, const void* k, const void* v, void* out, void* workspace,

@@ -94,13 +94,17 @@ int launch_attention(const AttentionArgs& args, hipStream_t stream);
 // compute units of the current device (the MI355X's 256 when no device can be queried).
 int narrow_attention_limit();
 // Ranges that workgroups of their own walk where a launch has few query blocks (1: no split), and the
-// bytes their results take before they are put together (0 where nothing is split, whatever the scale
-// and the causal flag are).
+// bytes their results take before they are put together (0 where nothing is split): of one call, and
+// enough for any scale and causal flag.
 struct AttentionExtents {
   int batch, q_heads, q_len, k_len, head_dim, cta_k;
 };
 enum class SplitKind { kPlain, kScaled, kMaskTensor };  // raw scores; pre-scaled ones, additive rows too; masks read per score
+inline SplitKind split_kind(bool mask, bool key_row, bool causal, float sm_scale) {
+  return !mask && !causal && sm_scale > 0.0f ? SplitKind::kPlain : mask && !key_row ? SplitKind::kMaskTensor : SplitKind::kScaled;
+}
 int attention_key_parts(const AttentionExtents& e, SplitKind kind, bool causal);
+size_t attention_split_bytes(const AttentionExtents& e, SplitKind kind, bool causal);
 size_t attention_split_bytes(const AttentionExtents& e, int mask_dtype, int64_t mask_stride_q);
 // of one range of one query block: eight wavefronts, head_dim / 4 outputs, maximum and denominator a lane
 constexpr size_t key_part_bytes(int head_dim) { return size_t{512} * (head_dim / 4 + 2) * sizeof(float); }

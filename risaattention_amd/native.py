@@ -81,6 +81,7 @@ SIGNATURES = {
         + [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_ptr, _c_size, _c_ptr],
     ),
     "risa_attention_split_bytes": (_c_size, [_c_int] * 7 + [_c_i64]),
+    "risa_attention_split_bytes_for": (_c_size, [_c_int] * 7 + [_c_i64, _c_f32, _c_int]),
     "risa_mask_lanes_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_i64, _c_i64] + [_c_int] * 6),
     "risa_prepare_mask_lanes": (
         _c_int,
@@ -91,6 +92,8 @@ SIGNATURES = {
         [_c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_i64, _c_i64, _c_i64, _c_int, _c_ptr],
     ),
     "risa_sdpa_workspace_bytes": (_c_size, [_c_int] * 9 + [_c_i64, _c_i64, _c_int, _c_int]),
+    "risa_sdpa_workspace_bytes_for": (
+        _c_size, [_c_int] * 9 + [_c_i64, _c_i64, _c_int, _c_int, _c_f32, _c_int, _c_int]),
     "risa_sdpa": (
         _c_int,
         [_c_ptr] * 5 + [_c_size] + [_c_int] * 7 + [_c_i64] * 12 + [_c_f32, _c_int, _c_int, _c_int]

@@ -538,3 +538,30 @@ def test_partial_results_of_key_ranges_are_sized_by_the_extents():
     assert plain > 0 and plain % part == 0 and plain // part <= 16
     assert size(1, 16, 128, 8192, 128, 64, 3, 8192) >= plain
     assert size(1, 0, 128, 8192, 128, 128, -1, 0) == size(1, 16, 128, 8192, 96, 128, -1, 0) == 0
+
+
+def test_partial_results_are_sized_by_the_call():
+    """What a call takes, not what another scale, flag or a sparse pattern would; enough for all of them
+    is the most that any takes."""
+    library = native.library()
+    split, enough = library.risa_attention_split_bytes_for, library.risa_attention_split_bytes
+    causal_only = (1, 8, 2048, 2048, 128, 128, -1, 0)
+    assert split(*causal_only, 0.1, 0) == 0 < split(*causal_only, 0.1, 1)
+    for call in (causal_only, (1, 16, 128, 8192, 128, 128, -1, 0), (2, 4, 1300, 2600, 256, 128, -1, 0), (1, 2, 33, 1024, 64, 64, -1, 0)):
+        assert enough(*call) == max(split(*call, scale, causal) for scale in (0.1, 0.0, -0.1) for causal in (0, 1))
+    for mask in ((3, 0), (3, 500), (0, 0), (0, 500)):  # key-only and query-dependent masks
+        call = (1, 16, 128, 8192, 128, 64, *mask)
+        assert 0 < split(*call, 0.1, 0) <= enough(*call)
+    workspace, call = library.risa_sdpa_workspace_bytes_for, (1, 8, 2048, 8, 2048, 128, 128, 0, -1, 0, 1, 1, 1)
+    sections = workspace(*call, 0.1, 0, 0)
+    assert workspace(*call, 0.1, 1, 0) == sections + split(*causal_only, 0.1, 1) == library.risa_sdpa_workspace_bytes(*call)
+    assert workspace(*call, 0.1, 1, 1) == sections  # lists of a pattern are not split
+
+
+def test_remembered_sizes_belong_to_a_device():
+    attend.forget_cached_sizes()
+    for device in (0, 1):
+        attend.attention_split_bytes(device, 1, 16, 128, 8192, 128, 128, -1, 0, 0.1, 0)
+        attend.call_workspace_bytes(device, 1, 2, 64, 2, 64, 128, 64, 0, -1, 0, 1, 1, 1, 0.1, 0, 0)
+    assert attend.attention_split_bytes.cache_info().misses == attend.call_workspace_bytes.cache_info().misses == 2
+    attend.forget_cached_sizes()
