@@ -235,7 +235,7 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
   if ((narrow || narrow_general) && !capture && !sparse && a.split_workspace != nullptr &&
       (p.index_mode == 0 || a.key_bias != nullptr)) {
     const AttentionExtents extents{a.batch, a.q_heads, a.q_len, a.k_len, a.head_dim, a.cta_k};
-    const SplitKind kind = split_kind(a.mask != nullptr, a.key_bias != nullptr, a.is_causal, a.sm_scale);
+    const SplitKind kind = split_kind(a.mask != nullptr ? a.mask_dtype : -1, a.key_bias != nullptr, a.is_causal, a.sm_scale);
     const int parts = attention_key_parts(extents, kind, a.is_causal);
     const size_t blocks = static_cast<size_t>(workgroups);
     if (parts > 1 && a.split_workspace_bytes >= parts * blocks * key_part_bytes(a.head_dim)) {

@@ -120,39 +120,57 @@ template <int D, int CTA_K> int launch_tile(const KernelParams& p, bool fast, in
 
 // How many ranges of the key tiles the workgroups of a launch of few query blocks walk.
 //
-// A workgroup takes its key tiles one after the other, 1 to 2.5 us per 64 keys however few workgroups
+// A workgroup takes its key tiles one after the other, 0.8 to 2.5 us per 64 keys however few workgroups
 // there are, so a launch that leaves compute units idle is split until they have work: the fewest
 // microseconds of a model of both sides.  Walking takes the longest chain of tiles (under the causal
 // rule, where workgroups of all lengths follow each other, the work of all of them where that is
-// more); a split adds 6 us and a write and read of the partial results.  Whole call, one range -> the best of
-// 2 to 24 (which one in brackets), 128 channels unless said otherwise, heads x queries x keys:
-//   plain       16 x 128 x 2048 35.0 -> 28.6 us (8), x 8192 91.4 -> 54.6 (16), 16 x 512 x 4096 55.1 -> 47.4 (4),
-//               256 channels 16 x 128 x 2048 62.9 -> 39.5 (8), 16 x 1024 x 4096 118 -> 99.6 (2)
-//   causal      1 x 8192 117 -> 50.9 us (4), 4 x 8192 133 -> 104 (2), 2 x 4096 66.2 -> 39.5 (4)
-//   padding     16 x 128 x 2048 49.5 -> 31.3 us (8), 16 x 512 x 4096 80.7 -> 52.6 (4), 64 channels 80.7 -> 44.0 (8)
-//   boolean     16 x 128 x 8192 269 -> 64.6 us (16), 16 x 512 x 1024 48.9 -> 34.1 (4), 16 x 1024 x 4096 141 -> 95.3 (2)
-// and where the model does not split: plain 16 x 512 x 1024 29.1 -> 30.4 us (4), 16 x 1024 x 4096 59.0 -> 61.4 (2),
-// 8 x 128 x 512 16.0 -> 16.9 (4); padding, 64 channels 16 x 1024 x 1024 32.7 -> 30.7 (4).
+// more, 0.75 tiles per workgroup of a range included); a split adds a launch, its ranges' epilogues and a
+// write and read of the partial results.
+//
+// The constants are those of 1647 launches of 1 to 256 workgroups and 300 to 16384 keys, attention from packed
+// operands with one range and with up to nine numbers of them each.  Over 737 others, what the model picks
+// takes 1.015 times the best number on the average (one range everywhere about 1.8), and 3 launches more than
+// 1 % longer than with one range, up to 1.16 times.  (With one row for causal launches and those with pre-scaled
+// scores, and none for plain launches that split in two inside their workgroups: 1.024, 18 launches, up to
+// 1.20 times.)  One range -> the number picked (in brackets), us, heads x queries x keys x channels:
+//   plain    16 x 96 x 11630 x 64 67.3 -> 25.7 (14), 2 x 1316 x 3494 x 256 64.8 -> 25.3 (10), 48 x 128 x 3072 x 128
+//            27.8 -> 22.3 (5); not split: 2 x 1024 x 1792 x 64 13.8 (14.4 with 4)
+//   causal   4 x 2688 x 64 43.2 -> 27.8 (4); not split: 16 x 1664 x 64 29.0 (31.4 with 2), 12 x 1664 x 128 28.0 (29.1 with 2)
+//   boolean  2 x 1152 x 893 x 64 51.4 -> 19.6 (7); not split: 64 x 99 x 464 x 128 17.9 (19.3 with 2)
+//   float    16 x 144 x 393 x 128 29.8 -> 18.9 (4)
+struct RangeCosts {
+  float per_64_keys[3];  // of head dims 64, 128 and 256
+  float fixed, per_range, per_megabyte;
+};
+
 int attention_key_parts(const AttentionExtents& e, SplitKind kind, bool causal) {
   const int64_t blocks = (e.q_len + kQueryBlock - 1) / kQueryBlock;
   const int64_t workgroups = blocks * e.batch * e.q_heads;
   if (e.k_len <= 2 * e.cta_k) return 1;
   const int units = narrow_attention_limit();
   if (workgroups > units) return 1;
-  const int wide = e.head_dim == 64 ? 0 : e.head_dim == 128 ? 1 : 2;
-  constexpr float kPer64Keys[3][3] = {{0.85f, 1.05f, 1.5f}, {1.1f, 1.1f, 1.6f}, {1.7f, 2.0f, 2.5f}};
-  const float per_tile = kPer64Keys[static_cast<int>(kind)][wide] * (e.cta_k / 64);
   const int tiles = ((causal ? std::min(e.k_len, e.q_len) : e.k_len) + e.cta_k - 1) / e.cta_k;
   // (without a split, plain launches of at most half a workgroup per unit split four or more tiles in two
   // inside their workgroups)
   const bool halves = kind == SplitKind::kPlain && !causal && workgroups * 2 <= units && tiles >= 4 &&
                       !(e.head_dim == 256 && e.cta_k == 128);
+  const bool short_halves = halves && e.head_dim != 256;
+  const bool causal_row = causal && kind == SplitKind::kScaled;
+  constexpr RangeCosts kHalves{{0.75f, 1.05f, 1.5f}, 5.0f, 0.2f, 1.0f / 3.0f};
+  constexpr RangeCosts kCausal{{0.8f, 1.1f, 2.1f}, 3.0f, 0.3f, 0.45f};
+  constexpr RangeCosts kKinds[] = {{{0.85f, 1.05f, 1.5f}, 6.0f, 0.0f, 1.0f / 3.0f},   // plain
+                                   {{1.1f, 1.1f, 1.6f}, 6.0f, 0.0f, 1.0f / 3.0f},     // scaled
+                                   {{1.4f, 1.7f, 2.3f}, 5.0f, 0.0f, 1.0f / 3.0f},     // boolean masks
+                                   {{1.7f, 2.0f, 2.5f}, 6.0f, 0.0f, 1.0f / 3.0f}};    // float masks
+  const RangeCosts& costs = short_halves ? kHalves : causal_row ? kCausal : kKinds[static_cast<int>(kind)];
+  const float per_tile = costs.per_64_keys[e.head_dim == 64 ? 0 : e.head_dim == 128 ? 1 : 2] * (e.cta_k / 64);
   const float all = causal ? 0.5f * workgroups * (tiles + 1) / units : 0.0f;  // tiles per unit
-  float best = per_tile * std::max<float>(halves ? (tiles + 1) / 2 : tiles, all);
+  float best = per_tile * std::max<float>(halves ? (tiles + 1) / 2 : tiles, all) * (short_halves ? 0.95f : 1.0f);
   int best_parts = 1;
   for (int parts = 2; parts <= 16 && parts <= tiles && workgroups * parts <= (causal ? 2 : 1) * units; ++parts) {
     const float megabytes = workgroups * parts * key_part_bytes(e.head_dim) * 1e-6f;
-    const float time = per_tile * std::max<float>((tiles + parts - 1) / parts, all) + 6.0f + megabytes / 3.0f;
+    const float walk = std::max<float>((tiles + parts - 1) / parts, causal_row ? all + 0.75f * workgroups * parts / units : all);
+    const float time = per_tile * walk + costs.fixed + costs.per_range * parts + costs.per_megabyte * megabytes;
     if (time < best) best = time, best_parts = parts;
   }
   return best_parts;
@@ -165,12 +183,12 @@ size_t attention_split_bytes(const AttentionExtents& e, SplitKind kind, bool cau
 }
 
 size_t attention_split_bytes(const AttentionExtents& e, int mask_dtype, int64_t mask_stride_q) {
-  const bool tensor = mask_dtype >= 0 && mask_stride_q != 0;
   size_t bytes = 0;
   for (const bool causal : {false, true}) {
-    bytes = std::max(bytes, attention_split_bytes(e, tensor ? SplitKind::kMaskTensor : SplitKind::kScaled, causal));
-    // (a key-only mask without its additive row is read like a mask tensor)
-    bytes = std::max(bytes, attention_split_bytes(e, mask_dtype < 0 ? SplitKind::kPlain : SplitKind::kMaskTensor, causal));
+    // (a key-only mask without its additive row is read like a mask tensor; -1 is a scale that hides the plain path)
+    for (const float sm_scale : {1.0f, -1.0f})
+      bytes = std::max(bytes, attention_split_bytes(e, split_kind(mask_dtype, mask_stride_q == 0, causal, sm_scale), causal));
+    if (mask_dtype >= 0) bytes = std::max(bytes, attention_split_bytes(e, split_kind(mask_dtype, false, causal, 1.0f), causal));
   }
   return bytes;
 }

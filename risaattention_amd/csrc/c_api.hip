@@ -380,7 +380,7 @@ size_t risa_attention_split_bytes_for(int batch, int q_heads, int q_len, int k_l
   if (batch <= 0 || q_heads <= 0 || q_len <= 0 || k_len <= 0 || (cta_k != 64 && cta_k != 128) ||
       (head_dim != 64 && head_dim != 128 && head_dim != 256))
     return 0;
-  const risa::SplitKind kind = risa::split_kind(mask_dtype >= 0, mask_stride_q == 0, is_causal != 0, sm_scale);
+  const risa::SplitKind kind = risa::split_kind(mask_dtype, mask_stride_q == 0, is_causal != 0, sm_scale);
   return risa::attention_split_bytes({batch, q_heads, q_len, k_len, head_dim, cta_k}, kind, is_causal != 0);
 }
 

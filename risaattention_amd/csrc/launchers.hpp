@@ -99,9 +99,10 @@ int narrow_attention_limit();
 struct AttentionExtents {
   int batch, q_heads, q_len, k_len, head_dim, cta_k;
 };
-enum class SplitKind { kPlain, kScaled, kMaskTensor };  // raw scores; pre-scaled ones, additive rows too; masks read per score
-inline SplitKind split_kind(bool mask, bool key_row, bool causal, float sm_scale) {
-  return !mask && !causal && sm_scale > 0.0f ? SplitKind::kPlain : mask && !key_row ? SplitKind::kMaskTensor : SplitKind::kScaled;
+enum class SplitKind { kPlain, kScaled, kBoolMask, kFloatMask };  // raw scores; pre-scaled ones, additive rows too; masks read per score
+inline SplitKind split_kind(int mask_dtype, bool key_row, bool causal, float sm_scale) {  // (mask_dtype -1: no mask)
+  if (mask_dtype < 0) return !causal && sm_scale > 0.0f ? SplitKind::kPlain : SplitKind::kScaled;
+  return key_row ? SplitKind::kScaled : mask_dtype == kBool ? SplitKind::kBoolMask : SplitKind::kFloatMask;
 }
 int attention_key_parts(const AttentionExtents& e, SplitKind kind, bool causal);
 size_t attention_split_bytes(const AttentionExtents& e, SplitKind kind, bool causal);

@@ -565,3 +565,21 @@ def test_remembered_sizes_belong_to_a_device():
         attend.call_workspace_bytes(device, 1, 2, 64, 2, 64, 128, 64, 0, -1, 0, 1, 1, 1, 0.1, 0, 0)
     assert attend.attention_split_bytes.cache_info().misses == attend.call_workspace_bytes.cache_info().misses == 2
     attend.forget_cached_sizes()
+
+
+# heads, queries, keys, head dim, mask dtype (-1: none), causal; key-tile size: measured with one range and with two to
+# sixteen (256 compute units)
+SPLIT_IS_SLOWER = [(16, 1664, 1664, 64, -1, 1, 64), (12, 1664, 1664, 128, -1, 1, 128), (4, 547, 547, 64, -1, 1, 64),
+                   (2, 1024, 1792, 64, -1, 0, 64), (24, 256, 2432, 64, -1, 0, 64), (2, 520, 1152, 128, -1, 0, 128),
+                   (64, 99, 464, 128, 3, 0, 64)]
+SPLIT_IS_FASTER = [(4, 2688, 2688, 64, -1, 1, 64), (8, 1839, 1839, 64, -1, 1, 64), (48, 128, 3072, 128, -1, 0, 128),
+                   (2, 1316, 3494, 256, -1, 0, 128), (16, 144, 393, 128, 0, 0, 64), (2, 1152, 893, 64, 3, 0, 64)]
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the rule asks the device for its compute units")
+@pytest.mark.parametrize("call", SPLIT_IS_SLOWER + SPLIT_IS_FASTER)
+def test_keys_are_split_where_that_was_measured_faster(call):
+    heads, q_len, k_len, dim, mask_dtype, causal, key_tile = call
+    size = native.library().risa_attention_split_bytes_for(1, heads, q_len, k_len, dim, key_tile, mask_dtype,
+                                                           k_len if mask_dtype >= 0 else 0, 0.1, causal)
+    assert (size > 0) == (call in SPLIT_IS_FASTER)
