@@ -25,7 +25,7 @@ from .policy import (
     select_key_block_size,
     validate_inputs,
 )
-from .prepare import KEYS_WITH_ROOM, pad_head_dim, resolve_scale, rows_hold_whole_runs
+from .prepare import keys_have_room, pad_head_dim, resolve_scale, rows_hold_whole_runs
 from .types import PrequantizedInt8Attention, RetainedMassPattern
 
 
@@ -150,8 +150,9 @@ def launch_attention(*, q_codes, k_codes, v_codes, output, q_scale, k_scale, v_s
     mask_lanes = prepare_mask_lanes(attn_mask, cta_k, dim)
     lane_args = (None, 0, 0) if mask_lanes is None else (mask_lanes[0].data_ptr(), mask_lanes[1], mask_lanes[2])
     # (a last tile of fewer keys is copied whole where the storage goes on behind the keys)
-    whole = padded == k_len or k_len < KEYS_WITH_ROOM
-    readable_keys = 0 if whole else k_codes.untyped_storage().nbytes() - k_codes.storage_offset()
+    readable_keys = 0
+    if keys_have_room(k_len, cta_k, dim):
+        readable_keys = k_codes.untyped_storage().nbytes() - k_codes.storage_offset()
     # (launches of few query blocks split the keys over workgroups and keep their results here)
     split_bytes = 0
     if block_mass is None and row_offsets is None:

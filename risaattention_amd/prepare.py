@@ -27,8 +27,15 @@ from .types import PrequantizedInt8Attention
 # Packed keys whose last tile is not full get a key tile of room behind them from this length on, so
 # that the attention kernel copies that tile whole: 0.3 to 0.8 us less on the GPU, 1 us more on the
 # host, which is what a call of the split path waits for below (44 us of host work against 42 on the
-# GPU, 32 heads x 1045 keys).
+# GPU, 32 heads x 1045 keys).  Head dim 256 over 128-key tiles has it at every length: the kernel of its larger
+# launches copies whole tiles only (150 -> 125 us for 544 workgroups x 2048 keys), and the call that prepares
+# and attends in one has room always, so both take the same kernel.
 KEYS_WITH_ROOM = 2048
+
+
+def keys_have_room(k_len: int, cta_k: int, dim: int) -> bool:
+    """Whether packed keys are followed by a key tile of room."""
+    return k_len % cta_k != 0 and (k_len >= KEYS_WITH_ROOM or (dim == 256 and cta_k == 128))
 
 
 @dataclass
@@ -112,11 +119,11 @@ def quantize_inputs(q, k, v, attn_mask, scale, use_midpoint_affine: bool,
         return torch.empty(shape, dtype=dtype, device=device)
 
     q_codes = empty(batch, q_heads, q_len, dim, dtype=torch.int8)
-    if k_len == padded or k_len < KEYS_WITH_ROOM:
-        k_codes = empty(batch, kv_heads, k_len, dim, dtype=torch.int8)
-    else:
+    if keys_have_room(k_len, cta_k, dim):
         k_codes = empty(batch * kv_heads * k_len * dim + cta_k * dim, dtype=torch.int8).as_strided(
             (batch, kv_heads, k_len, dim), (kv_heads * k_len * dim, k_len * dim, dim, 1))
+    else:
+        k_codes = empty(batch, kv_heads, k_len, dim, dtype=torch.int8)
     q_scale = empty(batch, q_heads, -(-q_len // 128) * (64 if dim == 256 else 32), dtype=torch.float32)
     k_scale = empty(batch, kv_heads, -(-k_len // cta_k) * 4, dtype=torch.float32)
     v_codes = empty(rows, padded, dtype=torch.int8)

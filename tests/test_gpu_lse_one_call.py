@@ -3,8 +3,7 @@
 The packed route adds the anchor correction to the log-normalisers as tensors; the single call stores
 it first and lets the attention kernel add its term.  Both are one FP32 addition, so results are equal
 bit for bit in every form the call takes: kernels of few and of many workgroups, split key ranges, rows
-that the preparation pads, every mask form, types and layouts.  (Keys of head dim 256 fill whole tiles or
-have more than 2048 tokens here: the packed route takes another kernel for the others.)
+that the preparation pads, every mask form, types and layouts.
 """
 
 from __future__ import annotations
@@ -28,6 +27,11 @@ FORMS = [
     (1, 40, 8, 1025, 900, 128, torch.float32, "absmax", False, "bias", False),
     (1, 40, 8, 1100, 1100, 200, torch.bfloat16, "absmax", True, None, False),
     (1, 24, 8, 1500, 1280, 256, torch.bfloat16, "absmax", False, None, False),
+    # head dim 256 with a ragged last key tile and more workgroups than compute units (two under the causal rule)
+    (2, 24, 8, 1500, 1025, 256, torch.bfloat16, "absmax", False, None, False),
+    (1, 24, 8, 1500, 1999, 200, torch.float16, "midpoint_affine", False, "key_bias", True),
+    (2, 24, 8, 1500, 1333, 256, torch.bfloat16, "absmax", False, "padding", False),
+    (2, 24, 8, 1500, 1500, 256, torch.bfloat16, "absmax", True, None, False),
     (1, 16, 16, 128, 4096, 128, torch.bfloat16, "absmax", False, "padding", False),  # split key ranges
     # mask forms made by workgroups of the preparation: one launch and two, lane words of aligned rows
     # (the packed route makes all of them in launches of their own)
