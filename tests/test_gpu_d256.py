@@ -62,3 +62,39 @@ def test_rows_that_see_no_key(risa, masked):
         mask[..., 700:] = True  # rows below see nothing under the causal rule
     out, lse = risa.int8_attention(q, k, v, attn_mask=mask, is_causal=masked, return_lse=True)
     assert not out.any() and torch.isneginf(lse).all()
+
+
+@pytest.mark.parametrize("dim,token_major", [(256, False), (200, True)])
+@pytest.mark.parametrize("mode", ["raw", "causal", "padding", "padding_causal", "rows", "rows_causal", "head_rows"])
+def test_every_batch_head_and_mask_plane(risa, mode, dim, token_major):
+    """Grouped heads over several batches: masks of another length per batch, additive rows per (batch, head) and
+    per head, tile lists of their own, both layouts, rows that the preparation pads."""
+    batch, heads, kv_heads, causal = 2, 36, 12, mode.endswith("causal")
+    q_len, k_len = (1100, 1181) if causal else (650, 1281)
+
+    def tensor(count, length, seed, **options):
+        if token_major:
+            return seeded((batch, length, count, dim), torch.bfloat16, seed, **options).transpose(1, 2)
+        return seeded((batch, count, length, dim), torch.bfloat16, seed, **options)
+
+    q, k = tensor(heads, q_len, 1, scale=1.5), tensor(kv_heads, k_len, 2, scale=1.5)
+    v = tensor(kv_heads, k_len, 3, offset=0.25)
+    mask = None
+    if mode.startswith("padding"):
+        mask = torch.arange(k_len, device="cuda") < torch.tensor([k_len, 700], device="cuda")[:, None, None, None]
+    elif "rows" in mode:
+        mask = seeded((1 if mode == "head_rows" else batch, heads, 1, k_len), torch.float32, 4)
+        mask[..., ::97] = -math.inf
+        mask[:, ::2, :, 256:512] = -math.inf  # tiles hidden from every other head
+    options = {"attn_mask": mask, "is_causal": causal}
+    out = both(risa, q, k, v, **options)
+    packed = risa.prequantize_int8_attention(q, k, v, **options)
+    rows = risa.int8_attention_from_prequantized(packed, output_layout="nhd")
+    assert rows.stride(1) < rows.stride(2) and torch.equal(rows, out)
+
+    from oracle import pipeline
+
+    of_last = None if mask is None else mask[-1:, -1:]
+    prepared = oracle_prequantize(q[-1:, -1:], k[-1:, -1:], v[-1:, -1:], attn_mask=of_last, is_causal=causal, return_lse=True)
+    expected, _, _ = pipeline.attend(prepared, return_lse=True)
+    assert relative_l2(to_numpy(out[-1:, -1:]), expected) < 1e-3
