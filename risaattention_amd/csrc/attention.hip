@@ -188,7 +188,8 @@ int launch_attention(const AttentionArgs& a, hipStream_t stream) {
   p.whole_key_tiles = a.whole_key_tiles ? 1 : 0;
   // Diagnostic switch, read at every launch: RISA_COMPILED_LOOP=1 sends every kernel that has a
   // hand-scheduled tile loop through the loop the compiler schedules instead (same results bit for
-  // bit; the tests compare the two).
+  // bit; the tests compare the two), and what attention_d256.hip takes through the sixteen-query kernel (which
+  // adds a denominator up in another order).
   const char* compiled_loop = std::getenv("RISA_COMPILED_LOOP");
   p.compiled_loop = compiled_loop != nullptr && compiled_loop[0] != '\0' && compiled_loop[0] != '0';
 

@@ -93,8 +93,8 @@ struct KernelParams {
 };
 
 // The log-normaliser of one row.  The lowest bit of p.lse says that the buffer holds the logits which the
-// K anchor took off, to be added: a parameter of its own is a scalar register more from the first
-// instruction on, which the compiled tile loop of 16/4 heads x 2048 showed (0.8 us of 48.4).
+// K anchor took off, to be added: as a parameter of its own the flag costs the sixteen-query kernel's launches
+// (16/4 heads x 2048 midpoint_affine, whole call, two pairs of runs: 48.4 and 49.0 us).
 __device__ __forceinline__ void store_lse(const KernelParams& p, int64_t row, float value) {
   typedef __attribute__((address_space(1))) float* GlobalFloats;
   const GlobalFloats target = (GlobalFloats)(p.lse & ~uintptr_t{1}) + row;

@@ -1,7 +1,8 @@
 // The sixteen-queries-per-wavefront kernel beyond the plain dense and reuse launches: tile
 // lists of key-only masks, capture, and the pre-scaled path (masks, causal, scale <= 0), all
-// with 128-query workgroups.  Every such launch with head dim 256 comes here, and those of
-// the other head dims that leave compute units with at most one workgroup.
+// with 128-query workgroups.  Those that leave compute units with at most one workgroup come
+// here, and with head dim 256 those that attention_d256.hip does not take (mask tensors, capture, 64-key
+// tiles, ragged keys without room behind them, two rounds of workgroups under the causal rule).
 #include "attention_narrow_kernel.hpp"
 
 namespace risa {

@@ -1,5 +1,6 @@
-// Attention kernel with sixteen queries per wavefront: launches with fewer workgroups
-// than compute units, and every launch with head dim 256.
+// Attention kernel with sixteen queries per wavefront: launches of at most one workgroup per compute
+// unit, ranges of their key tiles (attention_key_ranges.hip), and the launches with head dim 256 that
+// attention_d256.hip does not take.
 //
 // Same arithmetic as risa::attention_kernel (reference csrc/kernels/attention_int8.cuh:
 // 145-1026; the raw-score path, and for head dim 256 also the pre-scaled path with masks,

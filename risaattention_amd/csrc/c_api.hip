@@ -351,7 +351,12 @@ int risa_sdpa_quantize(const void* q, void* q_int8, float* q_scale, const void* 
                        int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b, int64_t v_stride_h,
                        int64_t v_stride_n, int input_dtype, int midpoint_affine,
                        int32_t* anchor_indices, const int32_t* kv_permutation, void* stream) {
-  return risa_sdpa_quantize_channels(q, q_int8, q_scale, k, k_int8, k_scale, v, v_int8, v_scale, v_center, v_tile_sum, v_workspace, v_workspace_bytes, batch, q_heads, q_len, kv_heads, k_len, head_dim, cta_k, q_stride_b, q_stride_h, q_stride_n, k_stride_b, k_stride_h, k_stride_n, v_stride_b, v_stride_h, v_stride_n, input_dtype, midpoint_affine, anchor_indices, kv_permutation, head_dim, stream);
+  return risa_sdpa_quantize_channels(q, q_int8, q_scale, k, k_int8, k_scale, v, v_int8, v_scale, v_center,
+                                     v_tile_sum, v_workspace, v_workspace_bytes, batch, q_heads, q_len,
+                                     kv_heads, k_len, head_dim, cta_k, q_stride_b, q_stride_h, q_stride_n,
+                                     k_stride_b, k_stride_h, k_stride_n, v_stride_b, v_stride_h, v_stride_n,
+                                     input_dtype, midpoint_affine, anchor_indices, kv_permutation, head_dim,
+                                     stream);
 }
 
 int risa_value_tile_sums(const void* v_int8, int32_t* tile_sum, int batch_heads, int head_dim,
@@ -397,7 +402,12 @@ int risa_attention_split(const void* q_int8, const void* k_int8, const void* v_i
                    const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
                    int64_t mask_lanes_stride_h, int64_t k_bytes, void* split_workspace,
                    size_t split_workspace_bytes, void* stream) {
-  return attend(q_int8, k_int8, v_int8, out, q_scale, k_scale, v_scale, v_center, v_tile_sum, mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, cta_k, batch, q_len, k_len, q_heads, kv_heads, head_dim, out_stride_b, out_stride_n, out_stride_h, sm_scale, out_dtype, sparse_row_offsets, sparse_block_indices, block_mass, is_causal, lse, false, key_mask_tiles, key_bias, key_bias_stride_b, key_bias_stride_h, mask_lanes, mask_lanes_stride_b, mask_lanes_stride_h, k_bytes, split_workspace, split_workspace_bytes, stream);
+  return attend(q_int8, k_int8, v_int8, out, q_scale, k_scale, v_scale, v_center, v_tile_sum, mask,
+                mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, cta_k, batch, q_len,
+                k_len, q_heads, kv_heads, head_dim, out_stride_b, out_stride_n, out_stride_h, sm_scale,
+                out_dtype, sparse_row_offsets, sparse_block_indices, block_mass, is_causal, lse, false,
+                key_mask_tiles, key_bias, key_bias_stride_b, key_bias_stride_h, mask_lanes, mask_lanes_stride_b,
+                mask_lanes_stride_h, k_bytes, split_workspace, split_workspace_bytes, stream);
 }
 
 int risa_attention_readable_keys(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
@@ -412,7 +422,13 @@ int risa_attention_readable_keys(const void* q_int8, const void* k_int8, const v
                    const float* key_bias, int64_t key_bias_stride_b, int64_t key_bias_stride_h,
                    const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
                    int64_t mask_lanes_stride_h, int64_t k_bytes, void* stream) {
-  return risa_attention_split(q_int8, k_int8, v_int8, out, q_scale, k_scale, v_scale, v_center, v_tile_sum, mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, cta_k, batch, q_len, k_len, q_heads, kv_heads, head_dim, out_stride_b, out_stride_n, out_stride_h, sm_scale, out_dtype, sparse_row_offsets, sparse_block_indices, block_mass, is_causal, lse, key_mask_tiles, key_bias, key_bias_stride_b, key_bias_stride_h, mask_lanes, mask_lanes_stride_b, mask_lanes_stride_h, k_bytes, nullptr, 0, stream);
+  return risa_attention_split(q_int8, k_int8, v_int8, out, q_scale, k_scale, v_scale, v_center, v_tile_sum,
+                              mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype,
+                              cta_k, batch, q_len, k_len, q_heads, kv_heads, head_dim, out_stride_b,
+                              out_stride_n, out_stride_h, sm_scale, out_dtype, sparse_row_offsets,
+                              sparse_block_indices, block_mass, is_causal, lse, key_mask_tiles, key_bias,
+                              key_bias_stride_b, key_bias_stride_h, mask_lanes, mask_lanes_stride_b,
+                              mask_lanes_stride_h, k_bytes, nullptr, 0, stream);
 }
 
 int risa_attention(const void* q_int8, const void* k_int8, const void* v_int8, void* out,
@@ -427,7 +443,13 @@ int risa_attention(const void* q_int8, const void* k_int8, const void* v_int8, v
                    const float* key_bias, int64_t key_bias_stride_b, int64_t key_bias_stride_h,
                    const uint64_t* mask_lanes, int64_t mask_lanes_stride_b,
                    int64_t mask_lanes_stride_h, void* stream) {
-  return risa_attention_readable_keys(q_int8, k_int8, v_int8, out, q_scale, k_scale, v_scale, v_center, v_tile_sum, mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, cta_k, batch, q_len, k_len, q_heads, kv_heads, head_dim, out_stride_b, out_stride_n, out_stride_h, sm_scale, out_dtype, sparse_row_offsets, sparse_block_indices, block_mass, is_causal, lse, key_mask_tiles, key_bias, key_bias_stride_b, key_bias_stride_h, mask_lanes, mask_lanes_stride_b, mask_lanes_stride_h, 0, stream);
+  return risa_attention_readable_keys(q_int8, k_int8, v_int8, out, q_scale, k_scale, v_scale, v_center,
+                                      v_tile_sum, mask, mask_stride_b, mask_stride_h, mask_stride_q,
+                                      mask_stride_k, mask_dtype, cta_k, batch, q_len, k_len, q_heads, kv_heads,
+                                      head_dim, out_stride_b, out_stride_n, out_stride_h, sm_scale, out_dtype,
+                                      sparse_row_offsets, sparse_block_indices, block_mass, is_causal, lse,
+                                      key_mask_tiles, key_bias, key_bias_stride_b, key_bias_stride_h,
+                                      mask_lanes, mask_lanes_stride_b, mask_lanes_stride_h, 0, stream);
 }
 
 size_t risa_selector_workspace_size(int) { return 0; }
@@ -703,7 +725,6 @@ int risa_sdpa_lse(const void* q, const void* k, const void* v, void* out, void* 
              input_dtype, q_stride_b, q_stride_h, q_stride_n, k_stride_b, k_stride_h, k_stride_n, sm_scale};
     riders.shift = &shift;
   }
-  if (!risa::can_prepare_fused(qk, value)) return fail("risa_sdpa: operands do not qualify for the fused preparation");
   status = risa::launch_prepare_fused(qk, value, riders, hip_stream);
   if (status != 0) return status;
   // (behind the K codes lie those of V, a whole key tile at least; behind the sections the partial results
@@ -728,7 +749,12 @@ int risa_sdpa_channels(const void* q, const void* k, const void* v, void* out, v
               int64_t mask_stride_q, int64_t mask_stride_k, int mask_dtype, int mask_batch,
               int mask_heads, int is_causal, const int32_t* sparse_row_offsets,
               const int32_t* sparse_block_indices, int channels, void* stream) {
-  return risa_sdpa_lse(q, k, v, out, workspace, workspace_bytes, batch, q_heads, q_len, kv_heads, k_len, head_dim, cta_k, q_stride_b, q_stride_h, q_stride_n, k_stride_b, k_stride_h, k_stride_n, v_stride_b, v_stride_h, v_stride_n, out_stride_b, out_stride_n, out_stride_h, sm_scale, input_dtype, output_dtype, midpoint_affine, mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, mask_batch, mask_heads, is_causal, sparse_row_offsets, sparse_block_indices, channels, nullptr, stream);
+  return risa_sdpa_lse(q, k, v, out, workspace, workspace_bytes, batch, q_heads, q_len, kv_heads, k_len,
+                       head_dim, cta_k, q_stride_b, q_stride_h, q_stride_n, k_stride_b, k_stride_h, k_stride_n,
+                       v_stride_b, v_stride_h, v_stride_n, out_stride_b, out_stride_n, out_stride_h, sm_scale,
+                       input_dtype, output_dtype, midpoint_affine, mask, mask_stride_b, mask_stride_h,
+                       mask_stride_q, mask_stride_k, mask_dtype, mask_batch, mask_heads, is_causal,
+                       sparse_row_offsets, sparse_block_indices, channels, nullptr, stream);
 }
 
 int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* workspace,
@@ -741,7 +767,12 @@ int risa_sdpa(const void* q, const void* k, const void* v, void* out, void* work
               int64_t mask_stride_q, int64_t mask_stride_k, int mask_dtype, int mask_batch,
               int mask_heads, int is_causal, const int32_t* sparse_row_offsets,
               const int32_t* sparse_block_indices, void* stream) {
-  return risa_sdpa_channels(q, k, v, out, workspace, workspace_bytes, batch, q_heads, q_len, kv_heads, k_len, head_dim, cta_k, q_stride_b, q_stride_h, q_stride_n, k_stride_b, k_stride_h, k_stride_n, v_stride_b, v_stride_h, v_stride_n, out_stride_b, out_stride_n, out_stride_h, sm_scale, input_dtype, output_dtype, midpoint_affine, mask, mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, mask_batch, mask_heads, is_causal, sparse_row_offsets, sparse_block_indices, head_dim, stream);
+  return risa_sdpa_channels(q, k, v, out, workspace, workspace_bytes, batch, q_heads, q_len, kv_heads, k_len,
+                            head_dim, cta_k, q_stride_b, q_stride_h, q_stride_n, k_stride_b, k_stride_h,
+                            k_stride_n, v_stride_b, v_stride_h, v_stride_n, out_stride_b, out_stride_n,
+                            out_stride_h, sm_scale, input_dtype, output_dtype, midpoint_affine, mask,
+                            mask_stride_b, mask_stride_h, mask_stride_q, mask_stride_k, mask_dtype, mask_batch,
+                            mask_heads, is_causal, sparse_row_offsets, sparse_block_indices, head_dim, stream);
 }
 
 }  // extern "C"
