@@ -156,7 +156,7 @@ def launch_attention(*, q_codes, k_codes, v_codes, output, q_scale, k_scale, v_s
     # (launches of few query blocks split the keys over workgroups and keep their results here)
     split_bytes = 0
     if block_mass is None and row_offsets is None:
-        split_bytes = attention_split_bytes(torch.cuda.current_device(), batch, q_heads, q_len, k_len, dim, cta_k,
+        split_bytes = attention_split_bytes(q_codes.device.index, batch, q_heads, q_len, k_len, dim, cta_k,
                                             mask_args[5], mask_args[3], float(sm_scale), int(bool(is_causal)))
     split = torch.empty(split_bytes, dtype=torch.uint8, device=q_codes.device) if split_bytes else None
     out_b = output.stride(0) if batch > 1 else q_heads * q_len * dim
@@ -185,8 +185,8 @@ def attention_split_bytes(device, *call) -> int:
 @functools.lru_cache(maxsize=256)
 def call_workspace_bytes(device, *call) -> int:
     """``risa_sdpa_workspace_bytes_for`` of the library, remembered per argument tuple: serving loops
-    ask for the same few shapes.  ``device`` is the current one, whose compute units decide whether
-    the keys of a call are split over workgroups."""
+    ask for the same few shapes.  ``device`` is the index of the call's device, whose compute units
+    decide whether the keys of a call are split over workgroups."""
     return native.library().risa_sdpa_workspace_bytes_for(*call)
 
 
@@ -253,7 +253,7 @@ def execute_dense_attention(
                      batch if attn_mask.stride(0) != 0 else 1, q_heads if attn_mask.stride(1) != 0 else 1)
     # the size query takes the mask's dtype, query and key strides and own extents
     workspace = torch.empty(
-        call_workspace_bytes(torch.cuda.current_device(), batch, q_heads, q_len, kv_heads, k_len, dim, cta_k,
+        call_workspace_bytes(q.device.index, batch, q_heads, q_len, kv_heads, k_len, dim, cta_k,
                              int(use_midpoint_affine), mask_args[5], mask_args[3], mask_args[4], mask_args[6],
                              mask_args[7], attention_scale, int(bool(is_causal)), int(csr[0] is not None)),
         dtype=torch.uint8, device=q.device)
