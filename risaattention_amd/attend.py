@@ -228,7 +228,8 @@ def execute_dense_attention(
     if dim != original_dim and not rows_hold_whole_runs(q, k, v):
         q, k, v, dim = pad_head_dim(q, k, v)
     attention_scale = resolve_scale(scale, original_dim)
-    batch, q_heads, q_len, _ = q.shape
+    batch, q_heads, q_len, channels = q.shape
+    device, causal = q.device, int(bool(is_causal))
     kv_heads, k_len = k.shape[1], k.shape[2]
     query_mask = attn_mask is not None and attn_mask.stride(-2) != 0
     cta_k = select_key_block_size(dim, k_len, has_mask=query_mask)
@@ -237,36 +238,35 @@ def execute_dense_attention(
     if sparse_pattern is not None:
         check_pattern_for(sparse_pattern, batch=batch, q_heads=q_heads, q_len=q_len, k_len=k_len, cta_k=cta_k,
                           attention_scale=attention_scale, is_causal=bool(is_causal), attn_mask=attn_mask,
-                          device=q.device)
+                          device=device)
         if sparse_pattern.sparsity >= MIN_PATTERN_SPARSITY:
             csr = (sparse_pattern.row_offsets.data_ptr(), sparse_pattern.block_indices.data_ptr())
     out_dtype = output_dtype_for(input_dtype)
     if output_layout == "nhd":
-        output = torch.empty(batch, q_len, q_heads, dim, dtype=out_dtype, device=q.device).permute(0, 2, 1, 3)
+        output = torch.empty(batch, q_len, q_heads, dim, dtype=out_dtype, device=device).permute(0, 2, 1, 3)
     else:
-        output = torch.empty(batch, q_heads, q_len, dim, dtype=out_dtype, device=q.device)
-    lse = torch.empty((batch, q_heads, q_len), dtype=torch.float32, device=q.device) if return_lse else None
+        output = torch.empty(batch, q_heads, q_len, dim, dtype=out_dtype, device=device)
+    lse = torch.empty((batch, q_heads, q_len), dtype=torch.float32, device=device) if return_lse else None
     if attn_mask is None:
         mask_args = (None, 0, 0, 0, 0, -1, 1, 1)
     else:
         mask_args = (attn_mask.data_ptr(), *attn_mask.stride(), MASK_DTYPE_CODES[attn_mask.dtype],
                      batch if attn_mask.stride(0) != 0 else 1, q_heads if attn_mask.stride(1) != 0 else 1)
     # the size query takes the mask's dtype, query and key strides and own extents
-    workspace = torch.empty(
-        call_workspace_bytes(q.device.index, batch, q_heads, q_len, kv_heads, k_len, dim, cta_k,
-                             int(use_midpoint_affine), mask_args[5], mask_args[3], mask_args[4], mask_args[6],
-                             mask_args[7], attention_scale, int(bool(is_causal)), int(csr[0] is not None)),
-        dtype=torch.uint8, device=q.device)
+    size = call_workspace_bytes(device.index, batch, q_heads, q_len, kv_heads, k_len, dim, cta_k,
+                                int(use_midpoint_affine), mask_args[5], mask_args[3], mask_args[4], mask_args[6],
+                                mask_args[7], attention_scale, causal, int(csr[0] is not None))
+    workspace = torch.empty(size, dtype=torch.uint8, device=device)
+    out_strides = output.stride()
     call, lse_args = (lib.risa_sdpa_lse, (lse.data_ptr(),)) if return_lse else (lib.risa_sdpa_channels, ())
     native.check(
         call(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), output.data_ptr(), workspace.data_ptr(),
-            workspace.numel(), batch, q_heads, q_len, kv_heads, k_len, dim, cta_k,
-            q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
-            v.stride(0), v.stride(1), v.stride(2), output.stride(0), output.stride(2), output.stride(1),
-            attention_scale, DTYPE_CODES[input_dtype], DTYPE_CODES[output.dtype],
-            int(use_midpoint_affine), *mask_args, int(bool(is_causal)), *csr, q.shape[-1], *lse_args,
-            native.current_stream(q.device),
+            size, batch, q_heads, q_len, kv_heads, k_len, dim, cta_k,
+            *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], out_strides[0], out_strides[2], out_strides[1],
+            attention_scale, DTYPE_CODES[input_dtype], DTYPE_CODES[out_dtype],
+            int(use_midpoint_affine), *mask_args, causal, *csr, channels, *lse_args,
+            native.current_stream(device),
         )
     )
     if original_dim != dim:
