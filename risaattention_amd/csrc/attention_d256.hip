@@ -3,12 +3,12 @@
 // are staged and why the compiler cannot schedule it).
 //
 // The sixteen-query kernel reads every K and V fragment twice as often from LDS and leaves its vector
-// and matrix cycles (59 and 32 % of its time) one behind the other: one barrier holds all eight
+// and matrix cycles (59 and 33 % of its time) one behind the other: one barrier holds all eight
 // wavefronts of a compute unit in the same phase.  Here the two wavefronts of a SIMD belong to different
-// workgroups and drift apart.  16/4 heads x 8192: 1.62 -> 1.12 million cycles, at 1.77 instead of 2.02 GHz
-// (the power the part is allowed bounds it: on all-zero operands 662 -> 462 us), whole call 740 -> 617 us
-// = 1.78e15 operations a second.  Without the copies of K and V it takes 8 % less.  Arithmetic per score
-// as in attention_kernel.hpp.
+// workgroups and drift apart (77 and 50 %).  16/4 heads x 8192: 1.61 -> 1.04 million cycles, at 1.71 instead
+// of 1.99 GHz (the power the part is allowed bounds it: on all-zero operands 2.11 GHz and 480 us), 810 -> 611 us
+// with counters, whole call 740 -> 617 us = 1.78e15 operations a second.  Arithmetic per score as in
+// attention_kernel.hpp.
 #include "attention_kernel.hpp"
 
 namespace risa {
