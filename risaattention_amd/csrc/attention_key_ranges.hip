@@ -185,7 +185,7 @@ size_t attention_split_bytes(const AttentionExtents& e, SplitKind kind, bool cau
 size_t attention_split_bytes(const AttentionExtents& e, int mask_dtype, int64_t mask_stride_q) {
   size_t bytes = 0;
   for (const bool causal : {false, true}) {
-    // (a key-only mask without its additive row is read like a mask tensor; -1 is a scale that hides the plain path)
+    // (unmasked calls: raw and pre-scaled scores; a key-only mask without its additive row is read like a mask tensor)
     for (const float sm_scale : {1.0f, -1.0f})
       bytes = std::max(bytes, attention_split_bytes(e, split_kind(mask_dtype, mask_stride_q == 0, causal, sm_scale), causal));
     if (mask_dtype >= 0) bytes = std::max(bytes, attention_split_bytes(e, split_kind(mask_dtype, false, causal, 1.0f), causal));
